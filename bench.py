@@ -54,16 +54,16 @@ sys.path.insert(0, ROOT)
 METRIC = "flux-advection Mcell-steps/s at 256^3; step ms NN-warm-PCG vs PCG at 1e-6 res"
 PEAK_FP32_TFLOPS = 157.3          # published FP32 vector rate (packed FP32 instructions)
 PEAK_FP32_NONPACKED_TFLOPS = 78.6  # one FP32 FMA per lane and cycle: this build emits no packed FP32
-# Work the quadrature kernel executes: its 1D WENO6 evaluations, counted on the device, at 73 flop
-# each (an FMA counts 2, the reciprocal 1): the arithmetic of one evaluation in the compiled kernel
-# (five sample differences, second and third differences, three candidates, the common squared
-# first difference and three indicator forms over 7 products, weights, blend).
-FLOP_PER_WENO6_EXECUTED = 73
+# Work the quadrature kernel executes per 1D WENO6 evaluation (an FMA counts 2, a reciprocal 1): 65
+# flop from the samples (first and second differences, three weighted candidates, three indicator
+# forms, weights, blend), 16 for a z stencil read from the pass's tables (a cubic over a quadratic).
+FLOP_PER_WENO6_EXECUTED = 65
+FLOP_PER_WENO6_TABLE = 16
 # The reference rule's count: every psi point and density point is one 3D WENO6 interpolation,
 # 43 1D evaluations of 200 flop as written in the reference's weno.h:34-68 (8,600 flop per point).
 FLOP_PER_WENO3D_POINT = 43 * 200
 PEAK_HBM_GBS = 8000.0
-# HBM bytes per launch of piece_kernel<1> at the default workload (256^3, CFL 4), from two
+# HBM bytes per launch of piece_brick_kernel at the default workload (256^3, CFL 4), from two
 # rocprofv3 counter passes (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, factors from a 1 GiB device copy);
 # recorded in profiles/density_step_256_cfl4_hbm_counters.md
 TRAFFIC_BYTES_256_CFL4 = 12.124e9
@@ -118,16 +118,19 @@ def cpu_baseline(scenes, n, cfl, threads):
 
 
 def quad_roofline(st, steps, n, cfl, density, optimized=False):
-    """Roofline entry of the WENO6 integral quadrature kernel (piece_kernel<1>) from the
+    """Roofline entry of the WENO6 integral quadrature kernel (piece_brick_kernel) from the
     library's HIP-event spans and device work counters of the timed steps.  achieved counts the
-    flops the kernel executes (its 1D WENO6 evaluations x 73); the reference rule's count
+    flops the kernel executes; the reference rule's count
     (8,600 flop per 3D point) is reported beside it: the kernel shares the z pass between the
     points of a piece and needs no y pass for psi on a face level, so that count over the
     kernel's time is a throughput of the reference's work, not a fraction of the hardware."""
     points = st["psi_points"] + st["density_points"]
     quad_s = st["quad_ms"] / 1e3
     qlaunches = max(st["quad_launches"], 1)
-    executed = st["weno_evals"] * FLOP_PER_WENO6_EXECUTED / quad_s / 1e12 if quad_s > 0 else 0.0
+    # z stencils of a piece: 6 of psi and 36 of q, 42 with points in both halves of its cell
+    z_evals = 42 * st["psi_points"] + 6 * (st["density_points"] - st["psi_points"])
+    flop = z_evals * FLOP_PER_WENO6_TABLE + (st["weno_evals"] - z_evals) * FLOP_PER_WENO6_EXECUTED
+    executed = flop / quad_s / 1e12 if quad_s > 0 else 0.0
     rule = points * FLOP_PER_WENO3D_POINT / quad_s / 1e12 if quad_s > 0 else 0.0
     traffic = TRAFFIC_BYTES_256_CFL4 if (density and not optimized and n == 256 and cfl == 4.0) else None
     avg_quad_s = quad_s / qlaunches
@@ -135,9 +138,9 @@ def quad_roofline(st, steps, n, cfl, density, optimized=False):
             "frac": round(executed / PEAK_FP32_TFLOPS, 4), "traffic": traffic,
             "peak_nonpacked": PEAK_FP32_NONPACKED_TFLOPS,
             "frac_nonpacked": round(executed / PEAK_FP32_NONPACKED_TFLOPS, 4),
-            "kernel": ("piece_kernel<1, true> (WENO6-optimized integral quadrature; flops priced as the WENO6 "
+            "kernel": ("piece_brick_kernel<true> (WENO6-optimized integral quadrature; flops priced as the WENO6 "
                        "form's, without its two extra reciprocals)" if optimized else
-                       "piece_kernel<1> (WENO6 integral quadrature)"), "compute": "FP32 VALU, no MFMA",
+                       "piece_brick_kernel (WENO6 integral quadrature)"), "compute": "FP32 VALU, no MFMA",
             "avg_launch_ms": round(st["quad_ms"] / qlaunches, 3),
             "weno6_evals_per_launch": st["weno_evals"] / qlaunches, "flop_per_weno6": FLOP_PER_WENO6_EXECUTED,
             "reference_rule": {"TFLOPs": round(rule, 3), "weno3d_points_per_launch": points / qlaunches,

@@ -9,6 +9,7 @@
 
 #include "../../include/fia.h"
 #include "fia_internal.hpp"
+#include "fia_math.hpp"
 #include "fia_unet.hpp"
 
 using namespace fia;
@@ -99,6 +100,7 @@ struct fia_ctx {
     int *host_flags = nullptr;                   // pinned: twisted count, kernel error
     double *host_scal = nullptr;                 // pinned: PCG scalars of two solves read back while iterating
     DevBuf<double> piece_c[3], piece_ay, piece_val;
+    DevBuf<WenoHalf> weno_tab[2];          // z stencils of q and psi (WENO6 integral quadrature)
     DevBuf<unsigned> gen_n;                 // twisted faces: pieces per face and orientation
     DevBuf<unsigned long long> gen_start;   // their exclusive scan and total
     DevBuf<double> gen_c[3], gen_ay, gen_val;   // the twisted faces' piece records and values
@@ -207,7 +209,7 @@ size_t ctx_bytes(const fia_ctx *c) {
     size_t b = c->psi.bytes() + c->twisted.bytes() + c->degen.bytes() + c->counters.bytes() + c->scal.bytes() + c->bits.bytes() +
                c->solid.bytes() + c->genI.bytes();
     b += c->fsa.bytes() + c->fsb.bytes() + c->face_n.bytes() + c->face_start.bytes() + c->scan_tmp.bytes() + c->bounds.bytes() +
-         c->piece_ay.bytes() + c->piece_val.bytes();
+         c->piece_ay.bytes() + c->piece_val.bytes() + c->weno_tab[0].bytes() + c->weno_tab[1].bytes();
     for (int a = 0; a < 3; ++a) b += c->piece_c[a].bytes() + c->gen_c[a].bytes();
     b += c->gen_n.bytes() + c->gen_start.bytes() + c->gen_ay.bytes() + c->gen_val.bytes();
     for (int a = 0; a < 3; ++a) b += c->disp[a].bytes() + c->work[a].bytes() + c->gen[a].bytes();
@@ -425,6 +427,15 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     const bool weno_quad = piece_quadrature_mode(p) != 0;
     int sq = -1;
     if (weno_quad) HIP_TRY(span_begin(c, SK_QUAD, sq));
+    size_t psi_halves = 0;
+    const size_t q_halves = weno_table_halves(p, psi_halves);
+    if (q_halves > 0) {
+        HIP_TRY(c->weno_tab[0].ensure(q_halves));
+        HIP_TRY(c->weno_tab[1].ensure(psi_halves));
+        HIP_TRY(launch_weno_tables(p, c->weno_tab[0].p, c->weno_tab[1].p, c->stream));
+        p.q_tab = c->weno_tab[0].p;
+        p.psi_tab = c->weno_tab[1].p;
+    }
     if (!p.fuse_value) HIP_TRY(launch_pieces(p, nslots, c->stream));   // fused: the cutters stored the values
     if (weno_quad) HIP_TRY(span_end(c, sq));
     HIP_TRY(launch_face_sum(p, c->stream));
@@ -1046,7 +1057,7 @@ fia_status fia_ctx_destroy(fia_ctx *c) {
     c->psi.release(); c->twisted.release(); c->degen.release(); c->counters.release(); c->scal.release(); c->bits.release();
     c->solid.release(); c->genI.release();
     c->fsa.release(); c->fsb.release(); c->face_n.release(); c->face_start.release(); c->scan_tmp.release();
-    c->piece_ay.release(); c->piece_val.release();
+    c->piece_ay.release(); c->piece_val.release(); c->weno_tab[0].release(); c->weno_tab[1].release();
     for (int a = 0; a < 3; ++a) { c->piece_c[a].release(); c->gen_c[a].release(); }
     c->gen_n.release(); c->gen_start.release(); c->gen_ay.release(); c->gen_val.release();
     for (int a = 0; a < 3; ++a) { c->disp[a].release(); c->work[a].release(); c->gen[a].release(); }

@@ -11,6 +11,8 @@
 
 namespace fia {
 
+struct WenoHalf;   // fia_math.hpp
+
 // Device buffer that grows on demand (contents are not kept when it grows).
 template <class T> struct DevBuf {
     T *p = nullptr;
@@ -141,6 +143,9 @@ struct FaceParams {
     // quadrature kernel: 64, 128 or 256, anything else 256.  Each face and piece is one thread's
     // work, so the results do not depend on them.
     int face_block, piece_block;
+    // z stencils of q and psi (launch_weno_tables), or null: the WENO6 integral quadrature then
+    // evaluates every stencil from its samples
+    const WenoHalf *q_tab, *psi_tab;
 };
 // the general cutter's piece budget of one flux pass (records of 40 bytes): more pieces than this
 // report FIA_ERR_CAPACITY instead of running
@@ -162,6 +167,9 @@ hipError_t launch_seg_faces(const FaceParams &p, hipStream_t s);
 // 0: the general quadrature (piece_kernel<0>)
 int piece_quadrature_mode(const FaceParams &p);
 hipError_t launch_pieces(const FaceParams &p, unsigned long long nslots, hipStream_t s);
+// sizes of the z stencil tables of q and psi of p (0: this pass takes none), and their launch
+size_t weno_table_halves(const FaceParams &p, size_t &psi_halves);
+hipError_t launch_weno_tables(const FaceParams &p, WenoHalf *q_tab, WenoHalf *psi_tab, hipStream_t s);
 hipError_t launch_face_sum(const FaceParams &p, hipStream_t s);
 // exclusive scan of the slot counts in (n faces) into out; bounds[1], bounds[2] = first slots of
 // families 1 and 2 (at p.fam_base), bounds[3] = total; tile_tmp holds scan_temp_words(n) words

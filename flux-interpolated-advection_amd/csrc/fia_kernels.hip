@@ -11,7 +11,9 @@
 //   degenerate_kernel clipping pipeline for faces with a corner colour on an interior integer
 //   zero_velocity_face_kernel  the zero-velocity correction pass: the undeformed y faces' pieces
 //                     in closed form (at most 2 x 2 axis-aligned rectangles per face)
-//   piece_kernel      quadrature of every piece slot (WENO6 integral rule: piece_kernel<1>)
+//   weno_table_kernel, piece_brick_kernel  quadrature of every piece slot under the WENO6 integral
+//                     rule: the z stencils' interpolants in tables, read from LDS by bricks of faces
+//   piece_kernel      quadrature of every piece slot, any rule (small grids: piece_kernel<1>)
 //   face_sum_kernel   face flux = ordered sum of its slots
 //   general_*         the exact recursive cutter for the few twisted faces: pieces counted and
 //                     stored per face, integrated one thread per piece, summed per face; their
@@ -557,6 +559,149 @@ FIA_HD double piece_flux_weno_integral(const FaceParams &P, const double c[3], d
     return ay * (psi + (double)dens);
 }
 
+// ---------------------------------------------------------------------------------------------
+// z stencil tables of a pass (WENO6 integral rule): the interpolant of every z stencil of q and
+// psi as a WenoEntry.  A pass evaluates each stencil at some 300 fractions (8 pieces a cell, 36-42
+// rows of q each), and all but the fraction is the stencil's own.  Row (x, y) holds the first
+// halves of its mz + kWenoPad entries, then the second halves: neighbouring lanes read neighbouring
+// entries, so each of the two 16-byte loads of an entry covers half the cache lines that it would
+// with whole entries side by side.  Bound by the 32 bytes stored per entry.
+// ---------------------------------------------------------------------------------------------
+template <class V, bool OPT>
+FIA_HD void weno_table_body(const V *f, long rows, int mz, double kappa, WenoHalf *tab, long id) {
+    const int len = mz + kWenoPad;
+    const long row = id / len;
+    if (row >= rows) return;
+    const int e = (int)(id - row * len), base = e - 3;
+    const V *r = f + row * mz;
+    double v[6], g[5];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) v[i] = (double)r[clampi(base - 2 + i, 0, mz - 1)];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) g[i] = v[i + 1] - v[i];
+    const WenoEntry w = weno6_entry<OPT>(g, v[2], kappa);
+    WenoHalf *out = tab + row * 2 * len + e;
+    out[0] = w.a;
+    out[len] = w.b;
+}
+template <class V, bool OPT>
+__global__ void __launch_bounds__(kBlock) weno_table_kernel(const V *f, long rows, int mz, double kappa, WenoHalf *tab) {
+    weno_table_body<V, OPT>(f, rows, mz, kappa, tab, (long)blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// entry ze of row `row` of a table whose rows are len entries long
+FIA_HD WenoEntry table_entry(const WenoHalf *tab, int len, long row, int ze) {
+    const WenoHalf *e = tab + (row * 2 * len + ze);
+    return WenoEntry{e[0], e[len]};
+}
+
+// piece_flux_weno_integral<1, OPT> with the z passes read from the tables: the same rule, points,
+// y and x passes.  Every row index is clamped to the field and the z base to its row's entries,
+// which gives the clamped samples' stencils, so no stencil needs a test.  HALVES = 1: no lane of
+// the wave has a second point (f < 1/2), so the seventh row and its passes are left out.
+// q_entry(ix, r): q's entry of column ix and row r of the piece's stencil.
+template <bool OPT, int HALVES, class QEntry>
+FIA_HD double piece_flux_table(const FaceParams &P, double ay, int bx, int bz, float tx, float tz, double jf, double f,
+                               int J, const QEntry &q_entry) {
+    const int mx = P.g.m[0], my = P.g.m[1], mz = P.g.m[2];
+    const int len = mz + kWenoPad, ze = weno_entry_index(bz, mz);
+    const float sz = tz - 0.5f, pz = tz * (tz - 1.0f);
+    const double ey = 0.5 * P.g.e[1];
+    // psi on level J: the z pass of six columns and the x pass
+    const int lev = clampi(J, 0, my), zc = clampi(bz, 0, mz - 1);
+    double xr[6];
+#pragma unroll
+    for (int ix = 0; ix < 6; ++ix) {
+        const long row = (long)clampi(bx - 2 + ix, 0, mx - 1) * (my + 1) + lev;
+        xr[ix] = P.psi[row * mz + zc] + (double)weno_entry_delta(table_entry(P.psi_tab, len, row, ze), tz, sz, pz);
+    }
+    const double psi = weno6<double, OPT>(xr, WenoCoef(tx, P.kappa_psi));
+    // the density points: sample row B + h is the stencil base of half h
+    const int nh = f < 0.5 ? 1 : 2;
+    const int B = J - 1;
+    const double level = jf - ey, oqy = 0.5 - ey;
+    float ty[HALVES], wt[HALVES];
+    int edge[HALVES];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+        double a, part;
+        if (h == 0) { a = level; part = nh == 1 ? f : 0.5; }
+        else { a = level + 0.5; part = nh == 1 ? 0.0 : f - 0.5; }
+        const double s = (0.5 * part) * P.gauss.x[0] + 0.5 * part + a - oqy;
+        ty[h] = (float)(s - (double)(B + h));
+        wt[h] = (float)(part * P.gauss.w[0]);
+        edge[h] = -1;
+        if constexpr (OPT) {
+            if (s < 0.0 || s > (double)(my - 1)) edge[h] = clampi((s < 0.0 ? 0 : my - 1) - (B - 2), 0, 6);
+        }
+    }
+    const WenoCoef wx(tx, P.kappa_q);
+    const WenoCoef wy[2] = {WenoCoef(ty[0], P.kappa_q), WenoCoef(ty[HALVES - 1], P.kappa_q)};
+    float yv[HALVES][6];
+#pragma unroll
+    for (int ix = 0; ix < 6; ++ix) {
+        float zr[5 + HALVES];
+#pragma unroll
+        for (int r = 0; r < 5 + HALVES; ++r) {
+            const WenoEntry e = q_entry(ix, r);
+            zr[r] = e.a.x + weno_entry_delta(e, tz, sz, pz);
+        }
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) {
+            if (OPT && edge[h] >= 0) {
+                float v = zr[0];
+#pragma unroll
+                for (int r = 1; r < 5 + HALVES; ++r) v = edge[h] == r ? zr[r] : v;
+                yv[h][ix] = v;
+            } else {
+                yv[h][ix] = weno6<float, OPT>(&zr[h], wy[h]);
+            }
+        }
+    }
+    float dens = 0.0f;
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+        if (h < nh) dens += weno6<float, OPT>(yv[h], wx) * wt[h];
+    return ay * (psi + (double)dens);
+}
+// A piece's sample bases and fractions: x and z of its centre, the G face level J below it and the
+// height f above that level.
+struct PiecePoint {
+    int bx, bz, J;
+    float tx, tz;
+    double jf, f;
+};
+template <bool OPT> FIA_HD PiecePoint piece_point(const FaceParams &P, const double c[3]) {
+    PiecePoint t;
+    if constexpr (OPT) {
+        split_coord_clamped(c[0] - (0.5 - 0.5 * P.g.e[0]), P.g.m[0], t.bx, t.tx);
+        split_coord_clamped(c[2] - (0.5 - 0.5 * P.g.e[2]), P.g.m[2], t.bz, t.tz);
+    } else {
+        split_coord(c[0] - (0.5 - 0.5 * P.g.e[0]), t.bx, t.tx);
+        split_coord(c[2] - (0.5 - 0.5 * P.g.e[2]), t.bz, t.tz);
+    }
+    const double gy = c[1] + 0.5 * P.g.e[1];
+    t.jf = floor(gy);
+    t.f = gy - t.jf;
+    t.J = floor_index(t.jf);
+    return t;
+}
+template <bool OPT, class QEntry>
+FIA_HD double piece_flux_at(const FaceParams &P, const PiecePoint &t, double ay, const QEntry &q_entry) {
+    if (wave_all(t.f < 0.5)) return piece_flux_table<OPT, 1>(P, ay, t.bx, t.bz, t.tx, t.tz, t.jf, t.f, t.J, q_entry);
+    return piece_flux_table<OPT, 2>(P, ay, t.bx, t.bz, t.tx, t.tz, t.jf, t.f, t.J, q_entry);
+}
+// the same with q's entries read from the table in memory
+template <bool OPT> FIA_HD double piece_flux_memory(const FaceParams &P, const PiecePoint &t, double ay) {
+    const int mx = P.g.m[0], my = P.g.m[1];
+    const int len = P.g.m[2] + kWenoPad, ze = weno_entry_index(t.bz, P.g.m[2]);
+    return piece_flux_at<OPT>(P, t, ay, [&](int ix, int r) {
+        return table_entry(P.q_tab, len, (long)clampi(t.bx - 2 + ix, 0, mx - 1) * my + clampi(t.J - 3 + r, 0, my - 1), ze);
+    });
+}
+FIA_HD int piece_evals(double f) { return f < 0.5 ? 7 + 36 + 7 : 7 + 42 + 14; }
+FIA_HD int piece_points(double f) { return f < 0.5 ? 1 : 2; }
+
 // face id (< 2^30, checked on the host) -> (i, j, k), id = (i fy + j) fz + k
 FIA_HD void decode_face(const CompGrid &g, int fam, long id, int &i, int &j, int &k) {
     const FastDiv &dz = g.fz[fam], &dy = g.fy[fam];
@@ -904,16 +1049,187 @@ FIA_HD void piece_body(const FaceParams &P, unsigned long long q, int &npieces, 
     }
     P.piece_val[q] = val;
 }
-// The one-point WENO6 integral rule (QM = 1) is held to 128 VGPRs, four waves per SIMD, which its
-// VALU-bound quadrature needs to hide the row loads.  OPT: the "WENO6-optimized" interpolation
-// (its three reciprocals per evaluation do not fit 128 VGPRs; it is left to the compiler).
+// QM = 1 serves the grids that take no tables (weno_table_halves), held to three waves per SIMD (no
+// spill).  OPT: the "WENO6-optimized" interpolation (left to the compiler).
 template <int QM, bool OPT>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(QM == 1 && !OPT ? 4 : 1)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(QM == 1 && !OPT ? 3 : 1)))
 piece_kernel(FaceParams P, unsigned long long nslots) {
     const unsigned long long q = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
     int npieces = 0, npts = 0, nevals = 0;
     if (q < nslots) piece_body<QM, OPT>(P, q, npieces, npts, nevals);
     if (QM != 0 && P.stats) add_stats(P.stats, npieces, npts, nevals);   // counted for the WENO6 rule only
+}
+
+// The table quadrature, one block per brick of faces.  Read from memory, a piece's 42 rows of 32
+// bytes keep the vector caches' return path busy (a wave's lanes touch 2-4 rows a load): 16 ms at
+// 256^3, no faster than evaluating the stencils.  The faces of a brick of cells share their rows:
+// the block stages a box of q entries once in LDS and reads all rows from there, at constant offsets
+// from the piece's corner of the box.
+//   1. the rows of the brick's faces (each a contiguous range of slots) and their prefix; the least
+//      and greatest sample bases of the brick's moved vertices, between which its pieces lie;
+//   2. the box of entries into LDS, rows past the field's edge repeated as the clamped stencils do;
+//      where the flow deforms the brick by more than the box's spare rows, its middle;
+//   3. the pieces, 64 at a time per wave; one whose rows are not all in the box (also a sliver's
+//      far centroid) reads the table in memory.
+// Bound by VALU issue (83% of the cycles at 256^3, CFL 4): 1,566 VALU a wave of pieces, of which the
+// 42 z stencils take 10 and a reciprocal each, where evaluating the stencils from their samples took
+// 3,960; 15.8 -> 8.1 ms per launch (density step 26.1 -> 19.6 ms, with 0.25 ms for the two tables).
+// 768 threads: three waves per SIMD at 168 VGPRs; 512 leave latency (density step 21.1 ms), 1,024
+// spill (20.9).
+constexpr int kBrickX = 4, kBrickY = 8, kBrickZ = 16, kBrickThreads = 768;
+constexpr int kWinX = 12, kWinY = 18, kWinZ = 22;   // 149 KB of the CU's 160
+constexpr int kBrickRows = 3 * (kBrickX + 1) * (kBrickY + 1);
+static_assert(kBrickRows <= 192 && kBrickRows <= kBrickThreads, "a wave finds a row with three ballots");
+struct Bricks {
+    int n[3];
+    explicit Bricks(const CompGrid &g) {
+        const int b[3] = {kBrickX, kBrickY, kBrickZ};
+        for (int a = 0; a < 3; ++a) n[a] = (g.m[a] + b[a] - 1) / b[a];
+    }
+    size_t count() const { return (size_t)n[0] * n[1] * n[2]; }
+};
+template <bool OPT>
+__global__ void __launch_bounds__(kBrickThreads) piece_brick_kernel(FaceParams P, Bricks br) {
+    __shared__ WenoHalf win[kWinX * kWinY * 2 * kWinZ];
+    __shared__ unsigned long long row_start[kBrickRows];
+    __shared__ unsigned row_end[kBrickRows];   // lengths, then the inclusive prefix of them
+    __shared__ int box[6];                     // least bx, J, bz and greatest
+    // workgroups go to the 8 XCDs in turn: each XCD takes one contiguous eighth of the bricks
+    const int per = (int)(gridDim.x / 8), count = br.n[0] * br.n[1] * br.n[2];
+    const int brick = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (brick >= count) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    // the brick's cells [lo, hi) on each axis; the last brick also takes the faces past the last cell
+    const int bi[3] = {brick / (br.n[2] * br.n[1]), brick / br.n[2] % br.n[1], brick % br.n[2]};
+    constexpr int size[3] = {kBrickX, kBrickY, kBrickZ};
+    int lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        lo[a] = bi[a] * size[a];
+        hi[a] = min(lo[a] + size[a], P.g.m[a]);
+    }
+    int rows = 0;
+#pragma unroll
+    for (int fam = 0; fam < 3; ++fam) {
+        int end[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) end[a] = hi[a] + (fam == a && bi[a] == br.n[a] - 1 ? 1 : 0);
+        const int ny = end[1] - lo[1], n = (end[0] - lo[0]) * ny, t = tid - rows;
+        if (t >= 0 && t < n) {
+            const int i = lo[0] + t / ny, j = lo[1] + t % ny;
+            const size_t first = P.fam_base[fam] + ((size_t)i * P.g.fy[fam].d + j) * P.g.fz[fam].d + lo[2];
+            const size_t last = first + (size_t)(end[2] - lo[2]) - 1;
+            const unsigned long long s0 = P.face_start[first];
+            row_start[tid] = s0;
+            row_end[tid] = (unsigned)(P.face_start[last] + P.face_n[last] - s0);
+        }
+        rows += n;
+    }
+    if (tid < 6) box[tid] = tid < 3 ? INT32_MAX : INT32_MIN;
+    // the moved vertices' bases (x, z: floor(p - (0.5 - e/2)); y: the level floor(p + e/2))
+    int least[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, most[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
+    const int vy = hi[1] - lo[1] + 1, vz = hi[2] - lo[2] + 1;
+    for (int t = tid; t < (hi[0] - lo[0] + 1) * vy * vz; t += kBrickThreads) {
+        const int k = t % vz, j = t / vz % vy, i = t / (vz * vy);
+        const int lat[3] = {lo[0] + i, lo[1] + j, lo[2] + k};
+        const size_t v = idx3(lat[0], lat[1], lat[2], P.g.m[1] + 1, P.g.m[2] + 1);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float p = (float)lat[a] + (P.disp[a] ? P.disp[a][v] : 0.0f) - (a == 1 ? 0.0f : 0.5f);
+            const int c = floor_index((double)p);
+            least[a] = min(least[a], c);
+            most[a] = max(most[a], c);
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        for (int off = 32; off > 0; off >>= 1) {
+            least[a] = min(least[a], __shfl_down(least[a], off, 64));
+            most[a] = max(most[a], __shfl_down(most[a], off, 64));
+        }
+    }
+    __syncthreads();
+    if (lane == 0) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            atomicMin(&box[a], least[a]);
+            atomicMax(&box[3 + a], most[a]);
+        }
+    }
+    if (tid < 64) {   // one wave scans the rows' lengths
+        unsigned run = 0;
+        for (int r0 = 0; r0 < rows; r0 += 64) {
+            const int r = r0 + tid;
+            unsigned v = r < rows ? row_end[r] : 0u;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const unsigned o = __shfl_up(v, off, 64);
+                if (tid >= off) v += o;
+            }
+            v += run;
+            if (r < rows) row_end[r] = v;
+            run = __shfl(v, 63, 64);
+        }
+    }
+    __syncthreads();
+    const int mx = P.g.m[0], my = P.g.m[1], mz = P.g.m[2], len = mz + kWenoPad;
+    // the box: columns bx - 2 .. bx + 3, rows J - 3 .. J + 3, z entries of the bases
+    const auto middle = [](int from, int to, int cap, int &n) {
+        n = min(to - from + 1, cap);
+        return from + (to - from + 1 - n) / 2;
+    };
+    int nx, ny, nz;
+    const int wx = middle(box[0] - 2, box[3] + 3, kWinX, nx), wy = middle(box[1] - 3, box[4] + 3, kWinY, ny);
+    const int wz = middle(weno_entry_index(box[2], mz), weno_entry_index(box[5], mz), kWinZ, nz);
+    for (int t = tid; t < nx * ny * 2 * kWinZ; t += kBrickThreads) {
+        const int e = t % kWinZ, hr = t / kWinZ, half = hr & 1, row = hr >> 1;
+        const int x = row / ny, y = row - x * ny;
+        if (e >= nz) continue;
+        const size_t src = ((size_t)clampi(wx + x, 0, mx - 1) * my + clampi(wy + y, 0, my - 1)) * 2 + half;
+        win[((x * kWinY + y) * 2 + half) * kWinZ + e] = P.q_tab[src * len + wz + e];
+    }
+    __syncthreads();
+    const unsigned total = row_end[rows - 1];
+    int npieces = 0, npts = 0, nevals = 0;
+    for (unsigned p0 = tid & ~63; p0 < total; p0 += kBrickThreads) {
+        // the row of the wave's first piece (rows ending at or before it), then a lane's own
+        int r = 0;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int c = t * 64 + lane;
+            r += __popcll(__ballot(c < rows && row_end[min(c, kBrickRows - 1)] <= p0));
+        }
+        const unsigned p = p0 + lane;
+        if (p >= total) continue;
+        while (row_end[r] <= p) ++r;
+        const unsigned long long q = row_start[r] + (p - (r > 0 ? row_end[r - 1] : 0u));
+        const double ay = P.piece_ay[q];
+        double val = 0.0;
+        if (ay != 0.0) {
+            const double c3[3] = {P.piece_c[0][q], P.piece_c[1][q], P.piece_c[2][q]};
+            const PiecePoint t = piece_point<OPT>(P, c3);
+            const int dx = t.bx - 2 - wx, dy = t.J - 3 - wy, dz = weno_entry_index(t.bz, mz) - wz;
+            if (dx >= 0 && dx + 5 < nx && dy >= 0 && dy + 6 < ny && dz >= 0 && dz < nz) {
+                const WenoHalf *at = win + (dx * kWinY + dy) * 2 * kWinZ + dz;
+                val = piece_flux_at<OPT>(P, t, ay, [&](int ix, int iy) {
+                    const WenoHalf *e = at + (ix * kWinY + iy) * 2 * kWinZ;
+                    return WenoEntry{e[0], e[kWinZ]};
+                });
+            } else {
+                val = piece_flux_memory<OPT>(P, t, ay);
+            }
+            npieces += 1; npts += piece_points(t.f); nevals += piece_evals(t.f);
+        }
+        P.piece_val[q] = val;
+    }
+    if (P.stats) {   // one atomic per counter and wave
+        int x[kStatWords] = {npieces, npts, nevals};
+#pragma unroll
+        for (int w = 0; w < kStatWords; ++w) {
+            for (int off = 32; off > 0; off >>= 1) x[w] += __shfl_down(x[w], off, 64);
+            if (lane == 0) atomicAdd(P.stats + kStatWords * (blockIdx.x % kStatSlots) + w, (unsigned long long)x[w]);
+        }
+    }
 }
 
 // Phase 4: face flux = ordered sum of its slots (deterministic).
@@ -1368,12 +1684,47 @@ int piece_quadrature_mode(const FaceParams &p) {
     return 0;
 }
 
+// The tables serve the one-point WENO6 integral rule on grids of at least kBrickLeast bricks: below
+// that half the device is idle, and one thread per piece on every CU is faster (density step at
+// CFL 2, stencils against tables: 24^3 926 and 975 us, 32^3 (64 bricks) 707 and 722, 48^3 (216) 871
+// and 820).
+constexpr size_t kBrickLeast = 128;
+size_t weno_table_halves(const FaceParams &p, size_t &psi_halves) {
+    psi_halves = 0;
+    if (piece_quadrature_mode(p) != 1 || Bricks(p.g).count() < kBrickLeast) return 0;
+    const size_t len = (size_t)p.g.m[2] + kWenoPad;
+    const size_t q = (size_t)p.g.m[0] * p.g.m[1] * len, psi = (size_t)p.g.m[0] * (p.g.m[1] + 1) * len;
+    psi_halves = 2 * psi;
+    return 2 * q;
+}
+hipError_t launch_weno_tables(const FaceParams &p, WenoHalf *q_tab, WenoHalf *psi_tab, hipStream_t s) {
+    size_t np = 0;
+    const size_t nq = weno_table_halves(p, np);
+    if (nq == 0) return hipErrorInvalidValue;
+    const long rq = (long)p.g.m[0] * p.g.m[1], rp = (long)p.g.m[0] * (p.g.m[1] + 1);
+    const int mz = p.g.m[2];
+    const dim3 gq(grid_for(nq / 2, kBlock)), gp(grid_for(np / 2, kBlock)), b(kBlock);
+    if (p.weno_opt) {
+        hipLaunchKernelGGL((weno_table_kernel<float, true>), gq, b, 0, s, p.q, rq, mz, (double)p.kappa_q, q_tab);
+        hipLaunchKernelGGL((weno_table_kernel<double, true>), gp, b, 0, s, p.psi, rp, mz, (double)p.kappa_psi, psi_tab);
+    } else {
+        hipLaunchKernelGGL((weno_table_kernel<float, false>), gq, b, 0, s, p.q, rq, mz, (double)p.kappa_q, q_tab);
+        hipLaunchKernelGGL((weno_table_kernel<double, false>), gp, b, 0, s, p.psi, rp, mz, (double)p.kappa_psi, psi_tab);
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_pieces(const FaceParams &p, unsigned long long nslots, hipStream_t s) {
     if (nslots == 0) return hipSuccess;
     const int b = block_or_default(p.piece_block);
     const dim3 grid(grid_for(nslots, b));
     const int qm = piece_quadrature_mode(p);
-    if (p.weno_opt) {
+    if (p.q_tab) {
+        const Bricks br(p.g);
+        const dim3 bricks((br.count() + 7) / 8 * 8);
+        if (p.weno_opt) hipLaunchKernelGGL(piece_brick_kernel<true>, bricks, dim3(kBrickThreads), 0, s, p, br);
+        else hipLaunchKernelGGL(piece_brick_kernel<false>, bricks, dim3(kBrickThreads), 0, s, p, br);
+    } else if (p.weno_opt) {
         if (qm == 1) hipLaunchKernelGGL((piece_kernel<1, true>), grid, dim3(b), 0, s, p, nslots);
         else if (qm == 2) hipLaunchKernelGGL((piece_kernel<2, true>), grid, dim3(b), 0, s, p, nslots);
         else hipLaunchKernelGGL((piece_kernel<0, true>), grid, dim3(b), 0, s, p, nslots);

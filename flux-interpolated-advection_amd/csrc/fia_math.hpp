@@ -50,22 +50,24 @@ FIA_HD bool wave_all(bool p) {
 // C1 = -d5 d0 / 10, C2 = d0 d1 / 20 (all positive on [0,1]).  Candidate r (the Newton-form cubic
 // on samples r..r+3) equals f_2 + t g_2 + A h_r + B_r D_r with the second and third differences
 // h_k = g_{k+1} - g_k, D_k = h_{k+1} - h_k, A = t (t-1) / 2 and B_0 = t (t-1) (t+4) / 6,
-// B_1 = t (t-1) (t+1) / 6, B_2 = t (t-1) (t-2) / 6.  eps is the reference's 1e-6 in the units of
+// B_1 = t (t-1) (t+1) / 6, B_2 = t (t-1) (t-2) / 6; with D_r = h_{r+1} - h_r and its ideal weight
+// it enters as C_r (A h_r + B_r D_r) = l_r h_r + m_r h_{r+1}.  eps is the reference's 1e-6 in the units of
 // the indicators below (S_phys = kappa S / 180); kappa in (0, 1e3] keeps eps^4 a normal float.
 // eps2 is the 1e-30 that the "WENO6-optimized" variant adds to S_phys^2 (reference
 // src/weno.ispc:10-51), in the squared units of the same indicators.
 struct WenoCoef {
-    float t, A, B0, B1, B2, c0, c1, c2, eps, eps2;
+    float t, c0, c1, c2, eps, eps2;
+    float l0, m0, l1, m1, l2, m2;
     FIA_HD explicit WenoCoef(float tt, float kappa) {
-        const float p = tt * (tt - 1.0f);
+        const float p = tt * (tt - 1.0f) * (1.0f / 6.0f);
         t = tt;
-        A = 0.5f * p;
-        B0 = p * (tt + 4.0f) * (1.0f / 6.0f);
-        B1 = p * (tt + 1.0f) * (1.0f / 6.0f);
-        B2 = p * (tt - 2.0f) * (1.0f / 6.0f);
         c0 = (tt - 2.0f) * (tt - 3.0f) * (1.0f / 20.0f);
         c1 = (3.0f - tt) * (tt + 2.0f) * (1.0f / 10.0f);
         c2 = (tt + 2.0f) * (tt + 1.0f) * (1.0f / 20.0f);
+        const float p0 = p * c0, p1 = p * c1, p2 = p * c2;
+        l0 = p0 * (-1.0f - tt); m0 = p0 * (tt + 4.0f);
+        l1 = p1 * (2.0f - tt); m1 = p1 * (tt + 1.0f);
+        l2 = p2 * (5.0f - tt); m2 = p2 * (tt - 2.0f);
         eps = 1.8e-4f * fast_rcp(kappa);
         const float s = 180.0f * fast_rcp(kappa);
         eps2 = 1e-30f * (s * s);
@@ -86,29 +88,26 @@ struct WenoCoef {
 template <bool OPT = false>
 FIA_HD float weno6_delta(float g0, float g1, float g2, float g3, float g4, const WenoCoef &w) {
     const float h0 = g1 - g0, h1 = g2 - g1, h2 = g3 - g2, h3 = g4 - g3;
-    const float D0 = h1 - h0, D1 = h2 - h1, D2 = h3 - h2;
-    const float u0 = w.A * h0 + w.B0 * D0, u1 = w.A * h1 + w.B1 * D1, u2 = w.A * h2 + w.B2 * D2;
-    const float p00 = h0 * h0, p11 = h1 * h1, p22 = h2 * h2, p33 = h3 * h3;
-    const float p01 = h0 * h1, p12 = h1 * h2, p23 = h2 * h3;
+    const float u0 = w.l0 * h0 + w.m0 * h1, u1 = w.l1 * h1 + w.m1 * h2, u2 = w.l2 * h2 + w.m2 * h3;
+    const float p11 = h1 * h1, p22 = h2 * h2;
     const float base = 180.0f * (g2 * g2) + (OPT ? 0.0f : w.eps);
-    const float e0 = base + 244.0f * p00 - 683.0f * p01 + 634.0f * p11;
-    const float e1 = base + 244.0f * p11 - 293.0f * p12 + 244.0f * p22;
-    const float e2 = base + 634.0f * p22 - 683.0f * p23 + 244.0f * p33;
-    const float lin = w.t * g2;
+    const float e0 = h0 * (244.0f * h0 - 683.0f * h1) + (634.0f * p11 + base);
+    const float e1 = h1 * (244.0f * h1 - 293.0f * h2) + (244.0f * p22 + base);
+    const float e2 = h3 * (244.0f * h3 - 683.0f * h2) + (634.0f * p22 + base);
     if constexpr (OPT) {
-        const float a0 = w.c0 * fast_rcp(e0 * e0 + w.eps2), a1 = w.c1 * fast_rcp(e1 * e1 + w.eps2),
-                    a2 = w.c2 * fast_rcp(e2 * e2 + w.eps2);
-        return lin + (a0 * u0 + a1 * u1 + a2 * u2) * fast_rcp(a0 + a1 + a2);
+        const float b0 = fast_rcp(e0 * e0 + w.eps2), b1 = fast_rcp(e1 * e1 + w.eps2),
+                    b2 = fast_rcp(e2 * e2 + w.eps2);
+        return w.t * g2 + (b0 * u0 + b1 * u1 + b2 * u2) * fast_rcp(b0 * w.c0 + b1 * w.c1 + b2 * w.c2);
     }
     const float E0 = e0 * e0, E1 = e1 * e1, E2 = e2 * e2;
     if (fmaxf(e0, fmaxf(e1, e2)) < 1e9f) {
         // weights C_r / e_r^2 scaled by E0 E1 E2 (one reciprocal): for eps <= e < 1e9 every
         // product stays between eps^4 and 1e36
-        const float a0 = w.c0 * (E1 * E2), a1 = w.c1 * (E0 * E2), a2 = w.c2 * (E0 * E1);
-        return lin + (a0 * u0 + a1 * u1 + a2 * u2) * fast_rcp(a0 + a1 + a2);
+        const float b0 = E1 * E2, b1 = E0 * E2, b2 = E0 * E1;
+        return w.t * g2 + (b0 * u0 + b1 * u1 + b2 * u2) * fast_rcp(b0 * w.c0 + b1 * w.c1 + b2 * w.c2);
     }
-    const float a0 = w.c0 * fast_rcp(E0), a1 = w.c1 * fast_rcp(E1), a2 = w.c2 * fast_rcp(E2);
-    return lin + (a0 * u0 + a1 * u1 + a2 * u2) * fast_rcp(a0 + a1 + a2);
+    const float b0 = fast_rcp(E0), b1 = fast_rcp(E1), b2 = fast_rcp(E2);
+    return w.t * g2 + (b0 * u0 + b1 * u1 + b2 * u2) * fast_rcp(b0 * w.c0 + b1 * w.c1 + b2 * w.c2);
 }
 
 // WENO6 of six samples of type V (float, or double for the y-prefix psi).
@@ -157,6 +156,70 @@ template <class V> FIA_HD void load_row6(const V *__restrict__ base, unsigned of
 #pragma unroll
     for (int i = 0; i < 6; ++i) f[i] = r.v[i];
 }
+
+// ---- WENO6 of one stencil as a rational function of the fraction -------------------------------
+//
+// The smoothness indicators and candidates of a stencil depend on its samples alone, so over its
+// interval the interpolant is one rational function of t.  With s = t - 1/2, the ideal weights are
+// C_0 = (3.75 - 4 s + s^2) / 20, C_1 = (6.25 - s^2) / 10, C_2 = (3.75 + 4 s + s^2) / 20, the
+// candidates f_2 + t g_2 + t (t - 1) / 6 (3 h_r + (s + k_r) D_r), k = 4.5, 1.5, -1.5, and
+//   delta = t g_2 + t (t - 1) Q(s) / (1 + d_1 s + d_2 s^2),   Q a cubic:
+// the sum of C_r b_r (candidate r) over the sum of C_r b_r, b_r = 1 / e_r^2, both divided by the
+// latter's value at s = 0.  WenoEntry holds the nine numbers (the 1 left out): evaluating it takes
+// 12 instructions where weno6_delta takes 57.  It is worth building where a stencil is evaluated
+// at many fractions: the pieces of a flux pass evaluate each z stencil some 300 times.
+// weno6_entry works in FP64 and rounds the result, so an entry is as close to the exact
+// interpolant as weno6_delta's FP32 weights are.
+struct alignas(16) WenoHalf {
+    float x, y, z, w;
+};
+struct WenoEntry {
+    WenoHalf a, b;   // {f_2, g_2, q_0, q_1}, {q_2, q_3, d_1, d_2}
+};
+
+// g: the five first differences; kappa as in WenoCoef.  The weights' w_r = e_r^2 (OPT: e_r^2 +
+// eps2) are scaled by the largest, so their products stay in range for any FP32 samples.
+template <bool OPT> FIA_HD WenoEntry weno6_entry(const double g[5], double f2, double kappa) {
+    const double g2 = g[2];
+    const double h0 = g[1] - g[0], h1 = g2 - g[1], h2 = g[3] - g2, h3 = g[4] - g[3];
+    const double D0 = h1 - h0, D1 = h2 - h1, D2 = h3 - h2;
+    const double unit = 180.0 / kappa;
+    const double base = 180.0 * (g2 * g2) + (OPT ? 0.0 : 1e-6 * unit);
+    const double e0 = base + 244.0 * (h0 * h0) - 683.0 * (h0 * h1) + 634.0 * (h1 * h1);
+    const double e1 = base + 244.0 * (h1 * h1) - 293.0 * (h1 * h2) + 244.0 * (h2 * h2);
+    const double e2 = base + 634.0 * (h2 * h2) - 683.0 * (h2 * h3) + 244.0 * (h3 * h3);
+    const double add = OPT ? 1e-30 * (unit * unit) : 0.0;
+    double w0 = e0 * e0 + add, w1 = e1 * e1 + add, w2 = e2 * e2 + add;
+    const double inv = 1.0 / fmax(w0, fmax(w1, w2));
+    w0 *= inv; w1 *= inv; w2 *= inv;
+    const double b0 = w1 * w2, b1 = w0 * w2, b2 = w0 * w1;
+    const double n = 1.0 / (3.75 * (b0 + b2) + 12.5 * b1);
+    // C_r b_r n = c_r0 + c_r1 s + c_r2 s^2 (times 20 over 20), the candidates' 1/6 folded in
+    const double m0 = b0 * n * (1.0 / 6.0), m1 = b1 * n * (1.0 / 6.0), m2 = b2 * n * (1.0 / 6.0);
+    const double a0 = 3.0 * h0 + 4.5 * D0, a1 = 3.0 * h1 + 1.5 * D1, a2 = 3.0 * h2 - 1.5 * D2;
+    WenoEntry r;
+    r.a.x = (float)f2;
+    r.a.y = (float)g2;
+    r.a.z = (float)(3.75 * (m0 * a0 + m2 * a2) + 12.5 * (m1 * a1));
+    r.a.w = (float)(4.0 * (m2 * a2 - m0 * a0) + 3.75 * (m0 * D0 + m2 * D2) + 12.5 * (m1 * D1));
+    r.b.x = (float)(m0 * a0 - 2.0 * (m1 * a1) + m2 * a2 + 4.0 * (m2 * D2 - m0 * D0));
+    r.b.y = (float)(m0 * D0 - 2.0 * (m1 * D1) + m2 * D2);
+    r.b.z = (float)(4.0 * (b2 - b0) * n);
+    r.b.w = (float)((b0 - 2.0 * b1 + b2) * n);
+    return r;
+}
+
+// The interpolant's distance from f_2 at fraction t, with s = t - 1/2 and p = t (t - 1).
+FIA_HD float weno_entry_delta(const WenoEntry &e, float t, float s, float p) {
+    const float q = e.a.z + s * (e.a.w + s * (e.b.x + s * e.b.y));
+    const float d = 1.0f + s * (e.b.z + s * e.b.w);
+    return t * e.a.y + (p * q) * fast_rcp(d);
+}
+
+// Entries of a row of mz samples: one per stencil base -3 .. mz + 1 (samples clamped to the row;
+// all of a base outside that range are the same edge sample, as they are at its ends).
+constexpr int kWenoPad = 5;
+FIA_HD int weno_entry_index(int base, int mz) { return clampi(base, -3, mz + 1) + 3; }
 
 // 3D WENO6, passes z then y then x (reference src/WENO6_interpolation_3d.cpp:7-258).  A pass
 // whose sample coordinate is on a grid node (SX/SY/SZ) is skipped: WENO6 at t = 0 returns f_2
