@@ -85,6 +85,8 @@ struct FluxSet {
     }
 };
 
+constexpr int kHostBounds = 6;
+
 struct fia_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -95,9 +97,11 @@ struct fia_ctx {
     DevBuf<unsigned> face_n;               // piece slots per face
     DevBuf<unsigned long long> face_start; // exclusive scan of face_n
     DevBuf<unsigned long long> scan_tmp;   // tile sums of the slot scan
-    DevBuf<unsigned long long> bounds;     // slot bounds of the families (device side)
-    unsigned long long *host_bounds = nullptr;   // pinned: [0] 0, [1] [2] family starts, [3] total
-    int *host_flags = nullptr;                   // pinned: twisted count, kernel error
+    // pinned, stored by the scan itself: [1] [2] family starts, [3] total slots, [4] twisted and [5]
+    // degenerate faces; [0] read-backs
+    unsigned long long *host_bounds = nullptr;
+    int *host_flags = nullptr;                   // pinned: twisted count, kernel error; [2] GenOver
+    hipEvent_t lists_read = nullptr;             // the twisted faces' pieces are stored
     double *host_scal = nullptr;                 // pinned: PCG scalars of two solves read back while iterating
     DevBuf<double> piece_c[3], piece_ay, piece_val;
     DevBuf<WenoHalf> weno_tab[2];          // z stencils of q and psi (WENO6 integral quadrature)
@@ -208,7 +212,7 @@ namespace {
 size_t ctx_bytes(const fia_ctx *c) {
     size_t b = c->psi.bytes() + c->twisted.bytes() + c->degen.bytes() + c->counters.bytes() + c->scal.bytes() + c->bits.bytes() +
                c->solid.bytes() + c->genI.bytes();
-    b += c->fsa.bytes() + c->fsb.bytes() + c->face_n.bytes() + c->face_start.bytes() + c->scan_tmp.bytes() + c->bounds.bytes() +
+    b += c->fsa.bytes() + c->fsb.bytes() + c->face_n.bytes() + c->face_start.bytes() + c->scan_tmp.bytes() +
          c->piece_ay.bytes() + c->piece_val.bytes() + c->weno_tab[0].bytes() + c->weno_tab[1].bytes();
     for (int a = 0; a < 3; ++a) b += c->piece_c[a].bytes() + c->gen_c[a].bytes();
     b += c->gen_n.bytes() + c->gen_start.bytes() + c->gen_ay.bytes() + c->gen_val.bytes();
@@ -279,6 +283,11 @@ __global__ void zero_ints_kernel(int *a, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = 0;
 }
+// the face lists' counts (counters[1], the first error, stays)
+__global__ void zero_lists_kernel(int *counters) {
+    if (threadIdx.x == 0) counters[0] = 0;
+    if (threadIdx.x == 2) counters[2] = 0;
+}
 __global__ void zero_uints_kernel(unsigned int *a, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = 0u;
@@ -329,6 +338,16 @@ fia_status do_vertices(fia_ctx *c, const CompGrid &g, const float *u, const floa
     return FIA_OK;
 }
 
+// lists of at most this many twisted faces store their pieces without a count (168 MB of records)
+constexpr size_t kGenListMost = (size_t)1 << 16;
+
+void bind_general(fia_ctx *c, FaceParams &p) {
+    p.gen_n = c->gen_n.p;
+    for (int a = 0; a < 3; ++a) p.gen_c[a] = c->gen_c[a].p;
+    p.gen_ay = c->gen_ay.p;
+    p.gen_val = c->gen_val.p;
+}
+
 fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, FluxSet &fs, const PassSpec &s,
                     int fam_mask, double h) {
     for (int f = 0; f < 3; ++f) {
@@ -348,8 +367,7 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     }
     HIP_TRY(c->twisted.ensure(g.faces(0) + g.faces(1) + g.faces(2)));
     HIP_TRY(c->degen.ensure(g.faces(0) + g.faces(1) + g.faces(2)));
-    hipLaunchKernelGGL(zero_ints_kernel, dim3(1), dim3(64), 0, c->stream, c->counters.p, 1);       // twisted count
-    hipLaunchKernelGGL(zero_ints_kernel, dim3(1), dim3(64), 0, c->stream, c->counters.p + 2, 1);   // degenerate count
+    hipLaunchKernelGGL(zero_lists_kernel, dim3(1), dim3(64), 0, c->stream, c->counters.p);
     HIP_TRY(hipGetLastError());
     FaceParams p;
     memset(&p, 0, sizeof(p));
@@ -394,32 +412,43 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     HIP_TRY(c->face_n.ensure(nf));
     HIP_TRY(c->face_start.ensure(nf));
     HIP_TRY(c->scan_tmp.ensure(scan_temp_words(nf)));
-    HIP_TRY(c->bounds.ensure(4));
     p.face_n = c->face_n.p;
     p.face_start = c->face_start.p;
     p.fam_base[0] = 0; p.fam_base[1] = g.faces(0); p.fam_base[2] = g.faces(0) + g.faces(1);
     int sp;
     HIP_TRY(span_begin(c, SK_FACE, sp));
     HIP_TRY(launch_face_count(p, c->stream));   // all families; inactive ones count zero
-    HIP_TRY(launch_scan(c->scan_tmp.p, c->face_n.p, c->face_start.p, nf, p, c->bounds.p, c->stream));
-    // slot bounds of the families into pinned host memory
-    HIP_TRY(hipMemcpyAsync(c->host_bounds, c->bounds.p, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                           c->stream));
-    // with the twisted and degenerate face counts (complete after the count kernels), which size
-    // the grids of their kernels
-    HIP_TRY(hipMemcpyAsync(c->host_flags, c->counters.p, 3 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    // the slot bounds of the families and the list lengths, which size the launches below, straight
+    // into pinned host memory
+    HIP_TRY(launch_scan(c->scan_tmp.p, c->face_n.p, c->face_start.p, nf, p, c->host_bounds, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    const int n_twisted = c->host_flags[0], n_degen = c->host_flags[2];
+    const int n_twisted = (int)c->host_bounds[4], n_degen = (int)c->host_bounds[5];
     unsigned long long fam_slots[4] = {0, c->host_bounds[1], c->host_bounds[2], c->host_bounds[3]};
     const unsigned long long nslots = fam_slots[3];
     if (!(fam_slots[1] <= fam_slots[2] && fam_slots[2] <= fam_slots[3]))
         return fail(FIA_ERR_DEVICE, "inconsistent piece slot bounds");
-    for (int a = 0; a < 3; ++a) HIP_TRY(c->piece_c[a].ensure(nslots));
-    HIP_TRY(c->piece_ay.ensure(nslots));
-    HIP_TRY(c->piece_val.ensure(nslots));
+    for (int a = 0; a < 3; ++a) HIP_TRY(c->piece_c[a].ensure_slack(nslots));
+    HIP_TRY(c->piece_ay.ensure_slack(nslots));
+    HIP_TRY(c->piece_val.ensure_slack(nslots));
     for (int a = 0; a < 3; ++a) p.piece_c[a] = c->piece_c[a].p;
     p.piece_ay = c->piece_ay.p;
     p.piece_val = c->piece_val.p;
+    // twisted faces first: their pieces into kGenStride records per face and orientation, and whether
+    // that held them, read back while the kernels below run
+    bool strided = n_twisted > 0 && !p.general_all && (size_t)n_twisted <= kGenListMost;
+    if (strided) {
+        const size_t pairs = 2 * (size_t)n_twisted, most = pairs * kGenStride;
+        HIP_TRY(c->gen_n.ensure_slack(pairs));
+        for (int a = 0; a < 3; ++a) HIP_TRY(c->gen_c[a].ensure_slack(most));
+        HIP_TRY(c->gen_ay.ensure_slack(most));
+        HIP_TRY(c->gen_val.ensure_slack(most));
+        bind_general(c, p);
+        p.gen_stride = kGenStride;
+        p.gen_over = c->host_flags + 2;
+        *p.gen_over = GEN_FITS;
+        HIP_TRY(launch_general_emit(p, n_twisted, c->stream));
+        HIP_TRY(hipEventRecord(c->lists_read, c->stream));
+    }
     // pieces: one-pass face kernels (segment cutter), then the degenerate faces (clipping pipeline)
     HIP_TRY(launch_seg_faces(p, c->stream));
     HIP_TRY(launch_faces_degenerate(p, n_degen, c->stream));
@@ -440,30 +469,45 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     if (weno_quad) HIP_TRY(span_end(c, sq));
     HIP_TRY(launch_face_sum(p, c->stream));
     if (n_twisted > 0) {
-        // twisted faces: pieces counted, then stored in records sized from the read-back total
-        HIP_TRY(c->gen_n.ensure(2 * (size_t)n_twisted));
-        HIP_TRY(c->gen_start.ensure(2 * (size_t)n_twisted + 1));
-        p.gen_n = c->gen_n.p;
-        p.gen_start = c->gen_start.p;
-        HIP_TRY(launch_general_count(p, n_twisted, c->stream));
-        HIP_TRY(hipMemcpyAsync(c->host_bounds, c->gen_start.p + 2 * (size_t)n_twisted, sizeof(unsigned long long),
-                               hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipMemcpyAsync(c->host_flags + 1, c->counters.p + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        const unsigned long long npieces = c->host_bounds[0];
-        if (c->host_flags[1] != 0) return check_kernel_errors(c);   // the cutter failed on a face
-        if (npieces > kGenMaxPieces)
-            return fail(FIA_ERR_CAPACITY, "twisted faces: " + std::to_string(npieces) + " pieces in one pass, more than "
-                                          "the general cutter's budget of " + std::to_string(kGenMaxPieces));
-        for (int a = 0; a < 3; ++a) HIP_TRY(c->gen_c[a].ensure(npieces));
-        HIP_TRY(c->gen_ay.ensure(npieces));
-        HIP_TRY(c->gen_val.ensure(npieces));
-        for (int a = 0; a < 3; ++a) p.gen_c[a] = c->gen_c[a].p;
-        p.gen_ay = c->gen_ay.p;
-        p.gen_val = c->gen_val.p;
+        unsigned long long npieces = 2ull * (unsigned long long)n_twisted * kGenStride;
+        if (strided) {
+            HIP_TRY(hipEventSynchronize(c->lists_read));
+            const int over = *(volatile int *)(c->host_flags + 2);
+            if (over == GEN_FAILED) return check_kernel_errors(c);   // the cutter failed on a face
+            if (over == GEN_MORE) strided = false;
+        }
+        if (!strided) {
+            // pieces counted, then stored in records sized from the read-back total
+            HIP_TRY(c->gen_n.ensure(2 * (size_t)n_twisted));
+            HIP_TRY(c->gen_start.ensure(2 * (size_t)n_twisted + 1));
+            p.gen_stride = 0;
+            p.gen_n = c->gen_n.p;
+            p.gen_start = c->gen_start.p;
+            HIP_TRY(launch_general_count(p, n_twisted, c->stream));
+            HIP_TRY(hipMemcpyAsync(c->host_bounds, c->gen_start.p + 2 * (size_t)n_twisted, sizeof(unsigned long long),
+                                   hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(hipMemcpyAsync(c->host_flags + 1, c->counters.p + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            npieces = c->host_bounds[0];
+            if (c->host_flags[1] != 0) return check_kernel_errors(c);   // the cutter failed on a face
+            if (npieces > kGenMaxPieces)
+                return fail(FIA_ERR_CAPACITY, "twisted faces: " + std::to_string(npieces) + " pieces in one pass, more than "
+                                              "the general cutter's budget of " + std::to_string(kGenMaxPieces));
+            for (int a = 0; a < 3; ++a) HIP_TRY(c->gen_c[a].ensure(npieces));
+            HIP_TRY(c->gen_ay.ensure(npieces));
+            HIP_TRY(c->gen_val.ensure(npieces));
+            bind_general(c, p);
+            HIP_TRY(launch_general_emit(p, n_twisted, c->stream));
+        }
         fs.dirty = true;   // from here on the set may hold corrections
         HIP_TRY(launch_general_pieces(p, n_twisted, npieces, c->stream));
-        if (c->timing) { c->acc.twisted_faces += n_twisted; c->acc.general_pieces += (long long)npieces; }
+        if (c->timing) {
+            std::vector<unsigned> n(2 * (size_t)n_twisted);
+            HIP_TRY(hipMemcpyAsync(n.data(), c->gen_n.p, n.size() * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            c->acc.twisted_faces += n_twisted;
+            for (unsigned k : n) c->acc.general_pieces += k;
+        }
     }
     HIP_TRY(span_end(c, sp));
     if (c->timing) { c->acc.face_launches += 1; c->acc.quad_launches += weno_quad ? 1 : 0; }
@@ -1016,25 +1060,29 @@ static fia_status ctx_create(int device, hipStream_t stream, fia_ctx **out) {
         c->stream = stream;
     }
     auto drop_stream = [&]() { if (c->own_stream) (void)hipStreamDestroy(c->stream); };
-    if (hipHostMalloc((void **)&c->host_bounds, 4 * sizeof(unsigned long long)) != hipSuccess ||
-        hipHostMalloc((void **)&c->host_flags, 4 * sizeof(int)) != hipSuccess ||
-        hipHostMalloc((void **)&c->host_scal, 2 * kPcgScalars * sizeof(double)) != hipSuccess) {
+    if (hipHostMalloc((void **)&c->host_bounds, kHostBounds * sizeof(unsigned long long), hipHostMallocCoherent) != hipSuccess ||
+        hipHostMalloc((void **)&c->host_flags, 4 * sizeof(int), hipHostMallocCoherent) != hipSuccess ||
+        hipHostMalloc((void **)&c->host_scal, 2 * kPcgScalars * sizeof(double)) != hipSuccess ||
+        hipEventCreateWithFlags(&c->lists_read, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
         if (c->host_bounds) (void)hipHostFree(c->host_bounds);
         if (c->host_flags) (void)hipHostFree(c->host_flags);
+        if (c->host_scal) (void)hipHostFree(c->host_scal);
         drop_stream();
         delete c;
         return fail(FIA_ERR_DEVICE, "cannot allocate pinned host memory");
     }
     if (io_scratch_init(dev) != hipSuccess) {
         (void)hipHostFree(c->host_bounds); (void)hipHostFree(c->host_flags); (void)hipHostFree(c->host_scal);
+        (void)hipEventDestroy(c->lists_read);
         drop_stream(); delete c;
         return fail(FIA_ERR_DEVICE, "cannot find the device scratch of the allocation-free entry points");
     }
-    memset(c->host_bounds, 0, 4 * sizeof(unsigned long long));
+    memset(c->host_bounds, 0, kHostBounds * sizeof(unsigned long long));
     memset(c->host_flags, 0, 4 * sizeof(int));
     memset(c->host_scal, 0, 2 * kPcgScalars * sizeof(double));
     if (ensure_common(c) != FIA_OK) {
         (void)hipHostFree(c->host_bounds); (void)hipHostFree(c->host_flags); (void)hipHostFree(c->host_scal);
+        (void)hipEventDestroy(c->lists_read);
         drop_stream(); delete c; return FIA_ERR_DEVICE;
     }
     *out = c;
@@ -1069,12 +1117,13 @@ fia_status fia_ctx_destroy(fia_ctx *c) {
     c->batch_states.release(); c->batch_map.release(); c->batch_scal.release();
     c->graphs.release();
     if (c->host_batch) (void)hipHostFree(c->host_batch);
-    c->bounds.release(); c->stats.release();
+    c->stats.release();
     for (auto &sp : c->spans) { (void)hipEventDestroy(sp.a); (void)hipEventDestroy(sp.b); }
     c->spans.clear();
     if (c->host_bounds) (void)hipHostFree(c->host_bounds);
     if (c->host_flags) (void)hipHostFree(c->host_flags);
     if (c->host_scal) (void)hipHostFree(c->host_scal);
+    if (c->lists_read) (void)hipEventDestroy(c->lists_read);
     if (c->own_stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return FIA_OK;

@@ -445,17 +445,32 @@ constexpr int kGenVerts = 32;
 constexpr int kGenStack = 8;
 constexpr int kGenTris = 40;
 
+// A polygon with the range of each colour over its vertices, kept as vertices are added.  The arrays
+// live in private scratch memory, where each access is waited for: polygons are built in place in a
+// pool and the stack holds their pool indices (as bytes of one word), so a vertex is written once and
+// read once, where copies between the stack and the polygon being cut took most of the time
+// (the twisted faces of a 32^3 step: 107 us to count and 108 to store them, now 28 in all).
 struct GenPoly {
     int n, dim;
+    double lo[2], hi[2];
     CutVert v[kGenVerts];
 };
-// copies a polygon's n live vertices only (the arrays live in private scratch memory, where a
-// whole-struct copy would move all kGenVerts entries every time the stack is pushed or popped)
-FIA_HD void gen_copy(GenPoly &d, const GenPoly &s) {
-    d.n = s.n;
-    d.dim = s.dim;
-    for (int i = 0; i < s.n; ++i) d.v[i] = s.v[i];
-}
+// a polygon being built: its pool entry and, in registers, what its header will hold
+struct GenBuild {
+    int at, n;
+    double lo[2], hi[2];
+    FIA_HD void open(int index) { at = index; n = 0; lo[0] = lo[1] = 1e300; hi[0] = hi[1] = -1e300; }
+    FIA_HD void add(GenPoly *pool, const CutVert &v) {
+        pool[at].v[n++] = v;
+        lo[0] = fmin(lo[0], v.cx); hi[0] = fmax(hi[0], v.cx);
+        lo[1] = fmin(lo[1], v.cz); hi[1] = fmax(hi[1], v.cz);
+    }
+    FIA_HD void close(GenPoly *pool, int dim) const {
+        GenPoly &p = pool[at];
+        p.n = n; p.dim = dim;
+        for (int a = 0; a < 2; ++a) { p.lo[a] = lo[a]; p.hi[a] = hi[a]; }
+    }
+};
 
 // centroid and |area| of a xi-eta polygon (reference src/facecutter.h:226-253)
 FIA_HD void gen_center(const double (*p)[2], int num, double &cx, double &cy, double &area) {
@@ -484,79 +499,98 @@ FIA_HD void gen_center(const double (*p)[2], int num, double &cx, double &cy, do
 // there, src/facecutter.h:190-203).
 template <class Emit>
 FIA_HD int general_cut(const double col[4][2], double min_area, Emit &emit) {
-    GenPoly stack[kGenStack];
+    constexpr int kPool = kGenStack + 3;   // the stack, the polygon being cut and the two being built
+    GenPoly pool[kPool];
+    unsigned free_set = (1u << kPool) - 1u;
+    unsigned long long stack = 0;          // pool index of entry k in byte k
     int sp = 0;
+    const auto take = [&]() {
+        const int i = __builtin_ctz(free_set);
+        free_set &= free_set - 1u;
+        return i;
+    };
+    const auto push = [&](int i) { stack |= (unsigned long long)i << (8 * sp++); };
+    GenBuild arr0, arr1;
     {
-        GenPoly &q = stack[sp++];
-        q.n = 4; q.dim = 0;
+        arr0.open(take());
         const double sq[4][2] = {{0, 0}, {1, 0}, {1, 1}, {0, 1}};
-        for (int i = 0; i < 4; ++i) { q.v[i].xi = sq[i][0]; q.v[i].eta = sq[i][1]; q.v[i].cx = col[i][0]; q.v[i].cz = col[i][1]; }
-    }
-    GenPoly cur, arr0, arr1;
-    while (sp > 0) {
-        gen_copy(cur, stack[--sp]);
-        const int dim = cur.dim, num = cur.n;
-        double lo = 1e300, hi = -1e300;
-        for (int n = 0; n < num; ++n) {
-            const double c = dim == 0 ? cur.v[n].cx : cur.v[n].cz;
-            lo = fmin(lo, c); hi = fmax(hi, c);
+        for (int i = 0; i < 4; ++i) {
+            CutVert c;
+            c.xi = sq[i][0]; c.eta = sq[i][1]; c.cx = col[i][0]; c.cz = col[i][1];
+            arr0.add(pool, c);
         }
+        arr0.close(pool, 0);
+        push(arr0.at);
+    }
+    while (sp > 0) {
+        const int top = (int)(stack >> (8 * --sp)) & 0xff;
+        stack &= (1ull << (8 * sp)) - 1ull;
+        GenPoly &cur = pool[top];
+        const int num = cur.n;
+        int dim = cur.dim;
         int first, last;
-        interior_integers(lo, hi, first, last);
+        interior_integers(cur.lo[dim], cur.hi[dim], first, last);
+        if (first > last && dim == 0) {   // cut along x to the end: on along z
+            dim = 1;
+            interior_integers(cur.lo[1], cur.hi[1], first, last);
+        }
         if (first <= last) {
             const double iso = first;
-            // arr0 is the piece on v[0]'s side, closed last; when that side is above the cut its
-            // stack slot is taken now, under the pieces below the cut
-            int reserved = -1;
-            if (!((dim == 0 ? cur.v[0].cx : cur.v[0].cz) - iso < 0.0)) {
+            const CutVert v0 = cur.v[0];
+            // arr0 is the piece on v[0]'s side, closed last; when that side is above the cut it
+            // goes on the stack now, under the pieces below the cut
+            const bool above = !((dim == 0 ? v0.cx : v0.cz) - iso < 0.0);
+            arr0.open(take());
+            if (above) {
                 if (sp >= kGenStack) return KE_CAP_STACK;
-                reserved = sp++;
+                push(arr0.at);
             }
-            arr0.n = 0; arr1.n = 0; arr0.dim = dim; arr1.dim = dim;
+            arr1.open(take());
             int slot = 0;
-            arr0.v[arr0.n++] = cur.v[0];
+            arr0.add(pool, v0);
+            CutVert vn = v0, vm = cur.v[1];
             for (int n = 0; n < num; ++n) {
-                const int m = (n + 1 == num) ? 0 : n + 1;
-                const double v0 = (dim == 0 ? cur.v[n].cx : cur.v[n].cz) - iso;
-                const double v1 = (dim == 0 ? cur.v[m].cx : cur.v[m].cz) - iso;
-                const bool neg0 = v0 < 0.0, neg1 = v1 < 0.0;
+                const CutVert after = cur.v[n + 2 < num ? n + 2 : num - 1];   // loaded a step ahead
+                const double d0 = (dim == 0 ? vn.cx : vn.cz) - iso;
+                const double d1 = (dim == 0 ? vm.cx : vm.cz) - iso;
+                const bool neg0 = d0 < 0.0, neg1 = d1 < 0.0;
                 if (neg0 != neg1) {
-                    const double inv = 1.0 / (v1 - v0);
-                    const double t0 = v1 * inv, t1 = -v0 * inv;
+                    const double inv = 1.0 / (d1 - d0);
+                    const double t0 = d1 * inv, t1 = -d0 * inv;
                     CutVert add;
-                    add.xi = t0 * cur.v[n].xi + t1 * cur.v[m].xi;
-                    add.eta = t0 * cur.v[n].eta + t1 * cur.v[m].eta;
-                    if (dim == 0) { add.cx = iso; add.cz = t0 * cur.v[n].cz + t1 * cur.v[m].cz; }
-                    else { add.cz = iso; add.cx = t0 * cur.v[n].cx + t1 * cur.v[m].cx; }
+                    add.xi = t0 * vn.xi + t1 * vm.xi;
+                    add.eta = t0 * vn.eta + t1 * vm.eta;
+                    if (dim == 0) { add.cx = iso; add.cz = t0 * vn.cz + t1 * vm.cz; }
+                    else { add.cz = iso; add.cx = t0 * vn.cx + t1 * vm.cx; }
                     if (slot == 0) {
-                        arr0.v[arr0.n++] = add;
-                        slot = 1; arr1.n = 0;
-                        if (t1 < 1.0) arr1.v[arr1.n++] = add;
+                        arr0.add(pool, add);
+                        slot = 1;
+                        if (t1 < 1.0) arr1.add(pool, add);
                     } else {
-                        arr1.v[arr1.n++] = add;
+                        arr1.add(pool, add);
+                        arr1.close(pool, dim);
                         if (sp >= kGenStack) return KE_CAP_STACK;
-                        gen_copy(stack[sp++], arr1);
+                        push(arr1.at);
+                        arr1.open(take());
                         slot = 0;
-                        if (t1 < 1.0) arr0.v[arr0.n++] = add;
+                        if (t1 < 1.0) arr0.add(pool, add);
                     }
                 }
                 if (n < num - 1) {
-                    GenPoly &dst = slot == 0 ? arr0 : arr1;
-                    dst.v[dst.n++] = cur.v[m];
+                    if (slot == 0) arr0.add(pool, vm);
+                    else arr1.add(pool, vm);
                 }
                 if (arr0.n >= kGenVerts - 2 || arr1.n >= kGenVerts - 2) return KE_CAP_VERTS;
+                vn = vm;
+                vm = n + 2 < num ? after : v0;
             }
             if (slot != 0) return KE_CUT;   // odd number of sign changes: cannot happen on a loop
-            if (reserved >= 0) {
-                gen_copy(stack[reserved], arr0);
-            } else {
+            arr0.close(pool, dim);
+            if (!above) {
                 if (sp >= kGenStack) return KE_CAP_STACK;
-                gen_copy(stack[sp++], arr0);
+                push(arr0.at);
             }
-        } else if (dim == 0) {
-            cur.dim = 1;
-            if (sp >= kGenStack) return KE_CAP_STACK;
-            gen_copy(stack[sp++], cur);
+            free_set |= 1u << arr1.at;
         } else if (num >= 3) {
             // subdivide (reference src/facecutter.h:255-324)
             double pts[kGenVerts][2];
@@ -580,6 +614,7 @@ FIA_HD int general_cut(const double col[4][2], double min_area, Emit &emit) {
                     }
                 } else {
                     if (area != 0.0) emit(pts, num, cx, cy);
+                    free_set |= 1u << top;
                     continue;
                 }
             }
@@ -615,6 +650,7 @@ FIA_HD int general_cut(const double col[4][2], double min_area, Emit &emit) {
                 }
             }
         }
+        free_set |= 1u << top;
     }
     return KE_NONE;
 }

@@ -24,6 +24,9 @@ template <class T> struct DevBuf {
         if (e == hipSuccess) n = want;
         return e;
     }
+    // for sizes that follow the data: an eighth more than asked when it has to grow, so that a
+    // slightly larger next call does not allocate (and so synchronise) again
+    hipError_t ensure_slack(size_t want) { return want <= n && p ? hipSuccess : ensure(want + want / 8); }
     void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
     size_t bytes() const { return n * sizeof(T); }
 };
@@ -138,6 +141,8 @@ struct FaceParams {
     double *gen_c[3];
     double *gen_ay;
     double *gen_val;
+    unsigned gen_stride;     // > 0: pair k's records start at k * gen_stride (gen_start unused)
+    int *gen_over;           // GenOver of that form (host memory)
     GaussTable gauss;
     // threads per block of the face kernels (count, cutter, sum, zero velocity) and of the
     // quadrature kernel: 64, 128 or 256, anything else 256.  Each face and piece is one thread's
@@ -150,6 +155,10 @@ struct FaceParams {
 // the general cutter's piece budget of one flux pass (records of 40 bytes): more pieces than this
 // report FIA_ERR_CAPACITY instead of running
 constexpr unsigned long long kGenMaxPieces = 1ull << 25;
+// records kept per face and orientation when the pieces are stored without a count (a power of two)
+constexpr unsigned kGenStride = 32;
+// whether every pair's pieces fit their records, some pair has more, or the cutter failed on one
+enum GenOver { GEN_FITS = 0, GEN_MORE = 1, GEN_FAILED = 2 };
 
 // errors reported by kernels through FaceParams::error
 // KE_CAPACITY: a caller's piece array (fia_split_faces); KE_CAP_*: the general cutter's polygon
@@ -172,7 +181,8 @@ size_t weno_table_halves(const FaceParams &p, size_t &psi_halves);
 hipError_t launch_weno_tables(const FaceParams &p, WenoHalf *q_tab, WenoHalf *psi_tab, hipStream_t s);
 hipError_t launch_face_sum(const FaceParams &p, hipStream_t s);
 // exclusive scan of the slot counts in (n faces) into out; bounds[1], bounds[2] = first slots of
-// families 1 and 2 (at p.fam_base), bounds[3] = total; tile_tmp holds scan_temp_words(n) words
+// families 1 and 2 (at p.fam_base), bounds[3] = total, bounds[4] = twisted and bounds[5] = degenerate
+// faces (host memory: the kernel stores them there itself); tile_tmp holds scan_temp_words(n) words
 size_t scan_temp_words(size_t n);
 hipError_t launch_scan(unsigned long long *tile_tmp, const unsigned *in, unsigned long long *out, size_t n,
                        const FaceParams &p, unsigned long long *bounds, hipStream_t s);
@@ -180,6 +190,8 @@ hipError_t launch_scan(unsigned long long *tile_tmp, const unsigned *in, unsigne
 // gen_start[2 count] = the total), then with the piece records sized from that total: the pieces
 // stored, integrated and summed into the faces' flux and corr (count: the listed faces)
 hipError_t launch_general_count(const FaceParams &p, int count, hipStream_t s);
+hipError_t launch_general_emit(const FaceParams &p, int count, hipStream_t s);
+// quadrature of the stored pieces (npieces record slots) and the sums
 hipError_t launch_general_pieces(const FaceParams &p, int count, unsigned long long npieces, hipStream_t s);
 // degenerate faces of the segment-cutter mode, cut per face into their slots by the pipeline
 hipError_t launch_faces_degenerate(const FaceParams &p, int count, hipStream_t s);

@@ -1251,7 +1251,8 @@ template <int FAM> __global__ void __launch_bounds__(kBlock) face_sum_kernel(Fac
 // the clipping pipeline cuts every (strip, band) piece of the face into its slot, with the
 // interpolated colours of the recursive cut, so the side an edge on a cut line goes to is decided
 // the same way.  A grid-stride loop over the queued faces (few, near walls or pinned vertices).
-FIA_HD void degenerate_body(const FaceParams &P, int t) {
+// Pieces first, first + step, ... of listed face t.
+FIA_HD void degenerate_pieces(const FaceParams &P, int t, int first, int step) {
     const unsigned code = P.degen[t];
     const int fam = (int)(code >> 30);
     const long id = (long)(code & ((1u << 30) - 1u));
@@ -1263,40 +1264,45 @@ FIA_HD void degenerate_body(const FaceParams &P, int t) {
     geom.init(v);
     int x0, nxc, z0, nzc;
     colour_ranges(col, x0, nxc, z0, nzc);
-    unsigned long long slot = P.face_start[P.fam_base[fam] + id];
-    for (int s = 0; s <= nxc; ++s) {
-        for (int m = 0; m <= nzc; ++m, ++slot) {
-            Pipeline pp;
-            pp.st[0].reset(s > 0, 0, (double)(x0 + s - 1), true);
-            pp.st[1].reset(s < nxc, 0, (double)(x0 + s), false);
-            pp.st[2].reset(m > 0, 1, (double)(z0 + m - 1), true);
-            pp.st[3].reset(m < nzc, 1, (double)(z0 + m), false);
-            pp.acc.reset();
-            const double sq[4][2] = {{0, 0}, {1, 0}, {1, 1}, {0, 1}};
-            for (int c = 0; c < 4; ++c) {
-                CutVert cv;
-                cv.xi = sq[c][0]; cv.eta = sq[c][1]; cv.cx = col[c][0]; cv.cz = col[c][1];
-                pp.push<0>(geom, cv);
-            }
-            pp.close<0>(geom);
-            double ay = 0.0, c3[3] = {0.0, 0.0, 0.0};
-            if (pp.acc.n >= 3 && pp.acc.area2 != 0.0) {
-                const double inv3a = 1.0 / (3.0 * pp.acc.area2);
-                double r[3];
-                geom.rel(pp.acc.mxi * inv3a, pp.acc.meta * inv3a, r);
-                c3[0] = geom.p0[0] + r[0]; c3[1] = geom.p0[1] + r[1]; c3[2] = geom.p0[2] + r[2];
-                ay = 0.5 * pp.acc.ay2;
-            }
-            P.piece_c[0][slot] = c3[0];
-            P.piece_c[1][slot] = c3[1];
-            P.piece_c[2][slot] = c3[2];
-            P.piece_ay[slot] = ay;
+    const unsigned long long slot0 = P.face_start[P.fam_base[fam] + id];
+    for (int q = first; q < (nxc + 1) * (nzc + 1); q += step) {
+        const int s = q / (nzc + 1), m = q - s * (nzc + 1);
+        const unsigned long long slot = slot0 + (unsigned long long)q;
+        Pipeline pp;
+        pp.st[0].reset(s > 0, 0, (double)(x0 + s - 1), true);
+        pp.st[1].reset(s < nxc, 0, (double)(x0 + s), false);
+        pp.st[2].reset(m > 0, 1, (double)(z0 + m - 1), true);
+        pp.st[3].reset(m < nzc, 1, (double)(z0 + m), false);
+        pp.acc.reset();
+        const double sq[4][2] = {{0, 0}, {1, 0}, {1, 1}, {0, 1}};
+        for (int c = 0; c < 4; ++c) {
+            CutVert cv;
+            cv.xi = sq[c][0]; cv.eta = sq[c][1]; cv.cx = col[c][0]; cv.cz = col[c][1];
+            pp.push<0>(geom, cv);
         }
+        pp.close<0>(geom);
+        double ay = 0.0, c3[3] = {0.0, 0.0, 0.0};
+        if (pp.acc.n >= 3 && pp.acc.area2 != 0.0) {
+            const double inv3a = 1.0 / (3.0 * pp.acc.area2);
+            double r[3];
+            geom.rel(pp.acc.mxi * inv3a, pp.acc.meta * inv3a, r);
+            c3[0] = geom.p0[0] + r[0]; c3[1] = geom.p0[1] + r[1]; c3[2] = geom.p0[2] + r[2];
+            ay = 0.5 * pp.acc.ay2;
+        }
+        P.piece_c[0][slot] = c3[0];
+        P.piece_c[1][slot] = c3[1];
+        P.piece_c[2][slot] = c3[2];
+        P.piece_ay[slot] = ay;
     }
 }
+FIA_HD void degenerate_body(const FaceParams &P, int t) { degenerate_pieces(P, t, 0, 1); }
+// kFaceLanes lanes share a face's pieces (most have two to six; the list is short, so the kernel is
+// one face's latency long)
+constexpr int kFaceLanes = 8;
 __global__ void __launch_bounds__(64) degenerate_kernel(FaceParams P) {
     const int count = *P.degen_count;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += gridDim.x * blockDim.x) degenerate_body(P, t);
+    for (int t = (blockIdx.x * blockDim.x + threadIdx.x) / kFaceLanes; t < count; t += gridDim.x * blockDim.x / kFaceLanes)
+        degenerate_pieces(P, t, (int)threadIdx.x % kFaceLanes, kFaceLanes);
 }
 // With fuse_value (no quadrature launch): the values of the degenerate faces' pieces from the
 // records degenerate_kernel stored.
@@ -1326,12 +1332,16 @@ __global__ void __launch_bounds__(64) degenerate_value_kernel(FaceParams P) {
 // cell's ('+' order v0 v1 v2 v3, orientation 0) goes to flux, the upper cell's (v0 v3 v2 v1,
 // orientation 1) enters through corr = upper + flux.  In steps, so that no thread integrates a
 // whole face alone:
-//   general_count_kernel  pieces of each orientation of each listed face (t: 2t, 2t + 1)
-//   general_scan_kernel   their exclusive scan (one block) and the total, read back to size
-//                         the piece records
-//   general_emit_kernel   the pieces again, each stored as a record (centre, y area) in its range
+// A pair is one orientation of one listed face (2t, 2t + 1); a pair is one thread's work.
+//   general_emit_kernel   each piece stored as a record (centre, y area) in its pair's kGenStride
+//                         records, and the pair's count
 //   general_piece_kernel  the quadrature of every piece, one thread per piece
 //   general_sum_kernel    each orientation's pieces summed in cut order into flux and corr
+// Where a pair has more pieces, or the list is long (minimal_area < 1 lists every face), the pieces
+// are counted first and stored in ranges of that size:
+//   general_count_kernel  pieces of each pair
+//   general_scan_kernel   their exclusive scan (one block) and the total, read back to size
+//                         the piece records
 // Ranges and order depend only on the faces, so the sums are deterministic.
 // ---------------------------------------------------------------------------------------------
 
@@ -1371,58 +1381,81 @@ FIA_HD void general_piece_record(const FaceGeom &geom, const double (*pts)[2], i
     ay = 0.5 * ay2;
 }
 
-FIA_HD void general_count_body(const FaceParams &P, int t) {
-    for (int o = 0; o < 2; ++o) {
-        int fam;
-        long id;
-        double v[4][3], col[4][2];
-        general_face(P, t, o, fam, id, v, col);
-        unsigned n = 0;
-        auto count = [&](const double (*)[2], int, double, double) { ++n; };
-        const int code = general_cut(col, P.min_area, count);
-        if (code != KE_NONE) { report(P.error, code); n = 0; }
-        P.gen_n[2 * t + o] = n;
-    }
+FIA_HD void general_count_pair(const FaceParams &P, int t, int o) {
+    int fam;
+    long id;
+    double v[4][3], col[4][2];
+    general_face(P, t, o, fam, id, v, col);
+    unsigned n = 0;
+    auto count = [&](const double (*)[2], int, double, double) { ++n; };
+    const int code = general_cut(col, P.min_area, count);
+    if (code != KE_NONE) { report(P.error, code); n = 0; }
+    P.gen_n[2 * t + o] = n;
 }
-__global__ void __launch_bounds__(64) general_count_kernel(FaceParams P) {
-    const int count = *P.twisted_count;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += gridDim.x * blockDim.x) general_count_body(P, t);
+FIA_HD void general_count_body(const FaceParams &P, int t) {
+    for (int o = 0; o < 2; ++o) general_count_pair(P, t, o);
 }
 
-FIA_HD void general_emit_body(const FaceParams &P, int t) {
-    for (int o = 0; o < 2; ++o) {
-        int fam;
-        long id;
-        double v[4][3], col[4][2];
-        general_face(P, t, o, fam, id, v, col);
-        FaceGeom geom;
-        geom.init(v);
-        const unsigned long long s0 = P.gen_start[2 * t + o];
-        const unsigned cap = P.gen_n[2 * t + o];
-        unsigned k = 0;
-        auto emit = [&](const double (*pts)[2], int num, double cxi, double ceta) {
-            if (k >= cap) return;   // the same cut as the count: never taken
+// the pieces of pair (t, o) stored; without counts (gen_stride) the pair's count too
+FIA_HD void general_emit_pair(const FaceParams &P, int t, int o) {
+    const int pair = 2 * t + o;
+    const bool strided = P.gen_stride > 0;
+    const unsigned long long s0 = strided ? (unsigned long long)pair * P.gen_stride : P.gen_start[pair];
+    const unsigned cap = strided ? P.gen_stride : P.gen_n[pair];
+    if (cap == 0) return;
+    int fam;
+    long id;
+    double v[4][3], col[4][2];
+    general_face(P, t, o, fam, id, v, col);
+    FaceGeom geom;
+    geom.init(v);
+    unsigned k = 0;
+    auto emit = [&](const double (*pts)[2], int num, double cxi, double ceta) {
+        if (k < cap) {
             double c3[3], ay;
             general_piece_record(geom, pts, num, cxi, ceta, c3, ay);
-            const unsigned long long q = s0 + k++;
+            const unsigned long long q = s0 + k;
             P.gen_c[0][q] = c3[0]; P.gen_c[1][q] = c3[1]; P.gen_c[2][q] = c3[2];
             P.gen_ay[q] = ay;
-        };
-        if (cap > 0) general_cut(col, P.min_area, emit);
+        }
+        ++k;
+    };
+    const int code = general_cut(col, P.min_area, emit);
+    if (strided) {
+        // (a failure outlasts GEN_MORE: the counted form would fail on the same face)
+        if (code != KE_NONE) { report(P.error, code); *P.gen_over = GEN_FAILED; k = 0; }
+        else if (k > cap) { if (*(volatile int *)P.gen_over == GEN_FITS) *P.gen_over = GEN_MORE; k = cap; }
+        P.gen_n[pair] = k;
     }
 }
-__global__ void __launch_bounds__(64) general_emit_kernel(FaceParams P) {
-    const int count = *P.twisted_count;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += gridDim.x * blockDim.x) general_emit_body(P, t);
+FIA_HD void general_emit_body(const FaceParams &P, int t) {
+    for (int o = 0; o < 2; ++o) general_emit_pair(P, t, o);
+}
+// Pairs over the waves: `lanes` of them per 64-lane block, one while the device has a SIMD for each
+// (lanes that cut different faces take turns on every branch).
+__global__ void __launch_bounds__(64) general_count_kernel(FaceParams P, int lanes) {
+    const int pairs = 2 * *P.twisted_count;
+    if ((int)threadIdx.x >= lanes) return;
+    for (int k = blockIdx.x * lanes + threadIdx.x; k < pairs; k += gridDim.x * lanes) general_count_pair(P, k >> 1, k & 1);
+}
+__global__ void __launch_bounds__(64) general_emit_kernel(FaceParams P, int lanes) {
+    const int pairs = 2 * *P.twisted_count;
+    if ((int)threadIdx.x >= lanes) return;
+    for (int k = blockIdx.x * lanes + threadIdx.x; k < pairs; k += gridDim.x * lanes) general_emit_pair(P, k >> 1, k & 1);
 }
 
 FIA_HD void general_piece_body(const FaceParams &P, unsigned long long q) {
+    if (P.gen_stride > 0 && (unsigned)(q % P.gen_stride) >= P.gen_n[q / P.gen_stride]) return;   // no piece
     const double ay = P.gen_ay[q];
     double val = 0.0;
     if (ay != 0.0) {
         const double c3[3] = {P.gen_c[0][q], P.gen_c[1][q], P.gen_c[2][q]};
-        int npts = 0;
-        val = piece_flux(P, c3, ay, npts);
+        int npts = 0, nevals = 0;
+        if (P.interp == IM_WENO6 && P.integral && P.gauss.n == 1)   // piece_quadrature_mode 1
+            val = P.weno_opt ? piece_flux_weno_integral<1, true>(P, c3, ay, npts, nevals)
+                             : piece_flux_weno_integral<1, false>(P, c3, ay, npts, nevals);
+        else
+            val = piece_flux(P, c3, ay, npts);
     }
     P.gen_val[q] = val;
 }
@@ -1434,7 +1467,8 @@ __global__ void __launch_bounds__(kBlock) general_piece_kernel(FaceParams P, uns
 FIA_HD void general_sum_body(const FaceParams &P, int t) {
     double f[2];
     for (int o = 0; o < 2; ++o) {
-        const unsigned long long s0 = P.gen_start[2 * t + o];
+        const unsigned long long s0 =
+            P.gen_stride > 0 ? (unsigned long long)(2 * t + o) * P.gen_stride : P.gen_start[2 * t + o];
         const unsigned n = P.gen_n[2 * t + o];
         double s = 0.0;
         for (unsigned k = 0; k < n; ++k) s += P.gen_val[s0 + k];
@@ -1892,7 +1926,11 @@ __global__ void __launch_bounds__(kBlock) scan_tiles_kernel(const unsigned *in, 
             out[k] = r;
             if (k == P.fam_base[1]) bounds[1] = r;
             if (k == P.fam_base[2]) bounds[2] = r;
-            if (k == n - 1) bounds[3] = r + sv[scan_pad(e)];
+            if (k == n - 1) {
+                bounds[3] = r + sv[scan_pad(e)];
+                bounds[4] = (unsigned long long)*P.twisted_count;
+                bounds[5] = (unsigned long long)*P.degen_count;
+            }
         }
     }
 }
@@ -1945,22 +1983,37 @@ hipError_t launch_seg_faces(const FaceParams &p, hipStream_t s) {
 
 hipError_t launch_faces_degenerate(const FaceParams &p, int count, hipStream_t s) {
     if (count <= 0) return hipSuccess;
-    hipLaunchKernelGGL(degenerate_kernel, dim3(list_blocks(count)), dim3(64), 0, s, p);
+    hipLaunchKernelGGL(degenerate_kernel, dim3(list_blocks((int)std::min<long>((long)count * kFaceLanes, INT32_MAX - 63))),
+                       dim3(64), 0, s, p);
     if (p.fuse_value) hipLaunchKernelGGL(degenerate_value_kernel, dim3(list_blocks(count)), dim3(64), 0, s, p);
     return hipGetLastError();
 }
 
+// lanes per wave and blocks of the pair kernels: at most kPairBlocks waves at once
+constexpr int kPairBlocks = 1024;
+static int pair_lanes(int pairs) { return std::min(64, (pairs + kPairBlocks - 1) / kPairBlocks); }
+static unsigned pair_blocks(int pairs) {
+    const int lanes = pair_lanes(pairs);
+    return (unsigned)std::min(kPairBlocks, (pairs + lanes - 1) / lanes);
+}
+
 hipError_t launch_general_count(const FaceParams &p, int count, hipStream_t s) {
     if (count <= 0) return hipSuccess;
-    hipLaunchKernelGGL(general_count_kernel, dim3(list_blocks(count)), dim3(64), 0, s, p);
-    hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(kBlock), 0, s, (const unsigned *)p.gen_n, p.gen_start,
-                       2 * count);
+    const int pairs = 2 * count;
+    hipLaunchKernelGGL(general_count_kernel, dim3(pair_blocks(pairs)), dim3(64), 0, s, p, pair_lanes(pairs));
+    hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(kBlock), 0, s, (const unsigned *)p.gen_n, p.gen_start, pairs);
+    return hipGetLastError();
+}
+
+hipError_t launch_general_emit(const FaceParams &p, int count, hipStream_t s) {
+    if (count <= 0) return hipSuccess;
+    const int pairs = 2 * count;
+    hipLaunchKernelGGL(general_emit_kernel, dim3(pair_blocks(pairs)), dim3(64), 0, s, p, pair_lanes(pairs));
     return hipGetLastError();
 }
 
 hipError_t launch_general_pieces(const FaceParams &p, int count, unsigned long long npieces, hipStream_t s) {
     if (count <= 0) return hipSuccess;
-    hipLaunchKernelGGL(general_emit_kernel, dim3(list_blocks(count)), dim3(64), 0, s, p);
     if (npieces > 0)
         hipLaunchKernelGGL(general_piece_kernel, dim3(grid_for(npieces, kBlock)), dim3(kBlock), 0, s, p, npieces);
     hipLaunchKernelGGL(general_sum_kernel, dim3(grid_for((size_t)count, kBlock)), dim3(kBlock), 0, s, p);
