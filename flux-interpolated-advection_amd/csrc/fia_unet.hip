@@ -6,9 +6,8 @@
 // one-voxel halo is staged in LDS 32 channels at a time and read by all 27 taps, one
 // v_mfma_f32_16x16x32_bf16 per 16 voxels x 16 output channels x 32 input channels.  A wave owns
 // 64 voxels (4 row blocks) and all output channels, so every A fragment feeds all column blocks.
-// The data gradient is the same kernel on the flipped, transposed weights.  The weight gradient stages 64-voxel tiles of the pre-activation gradient
-// and of the tap-shifted input in LDS and accumulates per tap and voxel chunk; chunks are then
-// summed in a fixed order (no atomics: training is deterministic).
+// The data gradient is the same kernel on the flipped, transposed weights; the weight and bias
+// gradients are a GEMM over the voxels (conv3_wgrad_kernel).
 //
 // MFMA operand layouts (64 lanes): 16x16x16 BF16: lane l holds A[l % 16][4 (l / 16) + i] and
 // B[4 (l / 16) + i][l % 16] for i < 4; 16x16x32 BF16: A[l % 16][8 (l / 16) + i] and
@@ -16,6 +15,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "fia_unet.hpp"
@@ -232,100 +232,169 @@ hipError_t launch_conv3(const ConvArgs &a, int mode, hipStream_t s) {
     return conv3_nb<2>(a, s);
 }
 
-// ---- weight gradient ---------------------------------------------------------------------------
+// ---- weight and bias gradient -------------------------------------------------------------------
+//
+// dW[t][co][ci] = sum over voxels v of D[v][co] I[v + t][ci]: a GEMM with K = voxels, whose operands
+// both need consecutive voxels in a lane.  A block takes a run of 4 x 4 x 16 voxel tiles and 16 input
+// channels: per tile it stages D, and I with a one-voxel halo in x and y, transposed to
+// [row of 16 z voxels][channel][voxel]; I once per z shift, so that every operand of every tap is one
+// aligned 16-byte LDS read.  The 27 taps and the bias (D times ones) are 28 products, seven per wave,
+// each wave reusing its D operands for its seven.  The runs' sums are added in a fixed order (no
+// atomics: training is deterministic).  Staging is bound by its loads' latency and the LDS reads;
+// one tap per block, restaging D and I for each and reading the operands voxel by voxel, took
+// 207 us a launch at 64^3 on average (now 18) and the bias a launch of its own of 51 us.
+constexpr int kWgX = 4, kWgY = 4, kWgZ = 16;
+constexpr int kWgRowsI = (kWgX + 2) * (kWgY + 2), kWgRowsD = kWgX * kWgY;
+constexpr int kWgTaps = 28, kWgPerWave = kWgTaps / 4;
+constexpr int kWgBlocks = 512;      // blocks aimed at: two per CU where LDS holds them
+constexpr int kWgMaxChunks = 256;   // runs whose sums are reduced
 
-constexpr int kWgVox = 64;        // voxels per LDS tile
-constexpr int kWgChunk = 4096;    // voxels per block
-constexpr int kWgMaxTiles = 6;    // 16x16 output tiles per wave (cout/16 * cin/16 <= 24)
-constexpr int kWgMaxCout = 64, kWgMaxCin = 112;
+static long wgrad_tiles(int nx, int ny, int nz) {
+    return (long)((nx + kWgX - 1) / kWgX) * ((ny + kWgY - 1) / kWgY) * ((nz + kWgZ - 1) / kWgZ);
+}
+size_t conv3_wgrad_words(int nx, int ny, int nz, int cin, int cout) {
+    return (size_t)conv3_wgrad_chunks(nx, ny, nz, cin) * kWgTaps * cin * cout;
+}
+int conv3_wgrad_chunks(int nx, int ny, int nz, int cin) {
+    const long want = std::min<long>(kWgMaxChunks, std::max(1, kWgBlocks / (cin / 16)));
+    return (int)std::min(want, wgrad_tiles(nx, ny, nz));
+}
 
-size_t conv3_wgrad_chunks(size_t n) { return (n + kWgChunk - 1) / kWgChunk; }
+// voxels first .. first + N - 1 (z) of row (x, y), channels [c, c + 8), zero outside the grid
+template <int N, class Load>
+__device__ __forceinline__ void wgrad_load(const ConvArgs &a, int x, int y, int first, i16x8 (&v)[N], Load load) {
+    const bool row = x >= 0 && x < a.nx && y >= 0 && y < a.ny;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int z = first + i;
+        v[i] = row && z >= 0 && z < a.nz ? load(z) : i16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+}
 
+template <int NB>
 __global__ void __launch_bounds__(256) conv3_wgrad_kernel(ConvArgs a, const uint16_t *dpre, float *part) {
-    __shared__ uint16_t sD[kWgVox][kWgMaxCout + 4];
-    __shared__ uint16_t sI[kWgVox][kWgMaxCin + 4];
-    const int t = blockIdx.y;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = lane & 15, kq = (lane >> 4) * 4;
-    const int cin = a.cA + a.cB, cout = a.cout;
-    const int nbi = cin / 16, ntiles = (cout / 16) * nbi;
-    const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
-    const long nvox = (long)a.nx * a.ny * a.nz;
-    const long vb = (long)blockIdx.x * kWgChunk, ve = min(nvox, vb + kWgChunk);
-    f32x4 acc[kWgMaxTiles];
+    constexpr int cout = NB * 16;
+    __shared__ alignas(16) uint16_t sD[kWgRowsD][cout][kWgZ];
+    __shared__ alignas(16) uint16_t sI[3][kWgRowsI][16][kWgZ];   // by z shift
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = lane & 15, grp = lane >> 4;
+    const int c0 = blockIdx.y * 16;
+    const int tx = (a.nx + kWgX - 1) / kWgX, ty = (a.ny + kWgY - 1) / kWgY, tz = (a.nz + kWgZ - 1) / kWgZ;
+    const long tiles = (long)tx * ty * tz;
+    const long first = tiles * blockIdx.x / gridDim.x, last = tiles * (blockIdx.x + 1) / gridDim.x;
+    f32x4 acc[kWgPerWave][NB];
 #pragma unroll
-    for (int s = 0; s < kWgMaxTiles; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long v0 = vb; v0 < ve; v0 += kWgVox) {
-        const int q4o = cout / 4, q4i = cin / 4;
-        for (int i = threadIdx.x; i < kWgVox * q4o; i += 256) {
-            const int r = i / q4o, c4 = (i % q4o) * 4;
-            const long v = v0 + r;
-            const bf16x4 val = v < ve ? *reinterpret_cast<const bf16x4 *>(dpre + v * cout + c4) : bf16x4{0, 0, 0, 0};
+    for (int j = 0; j < kWgPerWave; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sD[r][c4 + e] = (uint16_t)val[e];
-        }
-        for (int i = threadIdx.x; i < kWgVox * q4i; i += 256) {
-            const int r = i / q4i, c4 = (i % q4i) * 4;
-            const long v = v0 + r;
-            bf16x4 val = bf16x4{0, 0, 0, 0};
-            if (v < ve) {
-                const int z = (int)(v % a.nz) + dz, y = (int)((v / a.nz) % a.ny) + dy, x = (int)(v / ((long)a.ny * a.nz)) + dx;
-                if (x >= 0 && x < a.nx && y >= 0 && y < a.ny && z >= 0 && z < a.nz) val = load4(a, x, y, z, c4);
-            }
+        for (int n = 0; n < NB; ++n) acc[j][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (long tile = first; tile < last; ++tile) {
+        const int z0 = (int)(tile % tz) * kWgZ, y0 = (int)(tile / tz % ty) * kWgY, x0 = (int)(tile / ((long)tz * ty)) * kWgX;
+        __syncthreads();   // the previous tile's reads are done
+        // units of 8 voxels x 8 channels, transposed in registers; I's are 10 voxels, one output per shift
+        for (int u = threadIdx.x; u < kWgRowsI * 4; u += 256) {
+            const int c = (u & 1) * 8, half = (u >> 1) & 1, r = u >> 2;
+            const int x = x0 - 1 + r / (kWgY + 2), y = y0 - 1 + r % (kWgY + 2);
+            i16x8 v[10];
+            wgrad_load(a, x, y, z0 + 8 * half - 1, v, [&](int z) { return load8(a, x, y, z, c0 + c); });
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sI[r][c4 + e] = (uint16_t)val[e];
-        }
-        __syncthreads();
+            for (int s = 0; s < 3; ++s)
 #pragma unroll
-        for (int s = 0; s < kWgMaxTiles; ++s) {
-            const int tile = wave + 4 * s;
-            if (tile >= ntiles) continue;
-            const int ob = tile / nbi, ib = tile % nbi;
+                for (int e = 0; e < 8; ++e) {
+                    i16x8 o;
 #pragma unroll
-            for (int ks = 0; ks < kWgVox / 16; ++ks) {
-                bf16x4 A, B;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    A[e] = (short)sD[ks * 16 + kq + e][ob * 16 + row];
-                    B[e] = (short)sI[ks * 16 + kq + e][ib * 16 + row];
+                    for (int i = 0; i < 8; ++i) o[i] = v[s + i][e];
+                    *reinterpret_cast<i16x8 *>(&sI[s][r][c + e][8 * half]) = o;
                 }
-                acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A, B, acc[s], 0, 0, 0);
+        }
+        for (int u = threadIdx.x; u < kWgRowsD * (cout / 8) * 2; u += 256) {
+            const int c = u % (cout / 8) * 8, half = u / (cout / 8) & 1, r = u / (cout / 4);
+            const int x = x0 + r / kWgY, y = y0 + r % kWgY;
+            i16x8 v[8];
+            wgrad_load(a, x, y, z0 + 8 * half, v, [&](int z) {
+                return *reinterpret_cast<const i16x8 *>(dpre + vox(x, y, z, a.ny, a.nz) * cout + c);
+            });
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                i16x8 o;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) o[i] = v[i][e];
+                *reinterpret_cast<i16x8 *>(&sD[r][c + e][8 * half]) = o;
             }
         }
         __syncthreads();
-    }
+        // K = 32 voxels: rows y and y + 1 of the tile (lane groups 0, 1 and 2, 3)
+#pragma unroll 2
+        for (int k = 0; k < kWgRowsD / 2; ++k) {
+            const int x = k / (kWgY / 2), y = k % (kWgY / 2) * 2 + (grp >> 1);
+            bf16x8 A[NB];
 #pragma unroll
-    for (int s = 0; s < kWgMaxTiles; ++s) {
-        const int tile = wave + 4 * s;
-        if (tile >= ntiles) continue;
-        const int ob = tile / nbi, ib = tile % nbi;
+            for (int n = 0; n < NB; ++n)
+                A[n] = *reinterpret_cast<const bf16x8 *>(&sD[x * kWgY + y][n * 16 + row][8 * (grp & 1)]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int co = ob * 16 + kq + r, ci = ib * 16 + row;
-            part[(((size_t)blockIdx.x * 27 + t) * cout + co) * cin + ci] = acc[s][r];
+            for (int j = 0; j < kWgPerWave; ++j) {
+                const int t = wave * kWgPerWave + j;
+                bf16x8 B;
+                if (t < 27) {
+                    const int r = (x + t / 9) * (kWgY + 2) + y + t / 3 % 3;
+                    B = *reinterpret_cast<const bf16x8 *>(&sI[t % 3][r][row][8 * (grp & 1)]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) B[i] = (__bf16)1.0f;
+                }
+#pragma unroll
+                for (int n = 0; n < NB; ++n) acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[n], B, acc[j][n], 0, 0, 0);
+            }
         }
     }
+    // [chunk][input slice][tap][cout][16]
+    float *out = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * kWgTaps * cout * 16;
+#pragma unroll
+    for (int j = 0; j < kWgPerWave; ++j)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                out[((size_t)(wave * kWgPerWave + j) * cout + n * 16 + 4 * grp + r) * 16 + row] = acc[j][n][r];
 }
 
-// grad_w[i] += sum over chunks of part[chunk][i] (chunk order)
-__global__ void reduce_chunks_kernel(const float *part, size_t chunks, size_t per, float *grad_w) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= per) return;
+// grad_w[t][co][ci] and grad_b[co] += the chunks' sums: 64 values per block, each wave adds every
+// fourth chunk, then the four sums in wave order
+__global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float *part, int chunks, int cin, int cout, float *grad_w,
+                                                           float *grad_b) {
+    __shared__ float sh[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t per = (size_t)kWgTaps * cin * cout, i = (size_t)blockIdx.x * 64 + lane;
     float s = 0.f;
-    for (size_t c = 0; c < chunks; ++c) s += part[c * per + i];
-    grad_w[i] += s;
+    if (i < per) {
+#pragma unroll 8
+        for (int c = wave; c < chunks; c += 4) s += part[c * per + i];
+    }
+    sh[wave][lane] = s;
+    __syncthreads();
+    if (wave != 0 || i >= per) return;
+    s = ((sh[0][lane] + sh[1][lane]) + sh[2][lane]) + sh[3][lane];
+    const int e = (int)(i % 16), co = (int)(i / 16 % cout), t = (int)(i / (16 * (size_t)cout) % kWgTaps);
+    const int slice = (int)(i / (16 * (size_t)cout * kWgTaps));
+    if (t < 27) grad_w[((size_t)t * cout + co) * cin + slice * 16 + e] += s;
+    else if (slice == 0 && e == 0) grad_b[co] += s;
 }
 
-hipError_t launch_conv3_wgrad(const ConvArgs &a, const uint16_t *dpre, float *part, float *grad_w, hipStream_t s) {
+hipError_t launch_conv3_wgrad(const ConvArgs &a, const uint16_t *dpre, float *part, float *grad_w, float *grad_b,
+                              hipStream_t s) {
     const int cin = a.cA + a.cB;
-    if (a.cout > kWgMaxCout || cin > kWgMaxCin || (a.cout / 16) * (cin / 16) > 4 * kWgMaxTiles)
-        return hipErrorInvalidValue;
-    const long nvox = (long)a.nx * a.ny * a.nz;
-    const size_t chunks = conv3_wgrad_chunks((size_t)nvox);
-    hipLaunchKernelGGL(conv3_wgrad_kernel, dim3((unsigned)chunks, 27), dim3(256), 0, s, a, dpre, part);
-    const size_t per = (size_t)27 * a.cout * cin;
-    hipLaunchKernelGGL(reduce_chunks_kernel, dim3((unsigned)((per + 255) / 256)), dim3(256), 0, s, part, chunks, per,
-                       grad_w);
+    if (a.cout % 16 || cin % 16) return hipErrorInvalidValue;
+    const int chunks = conv3_wgrad_chunks(a.nx, a.ny, a.nz, cin);
+    const dim3 grid((unsigned)chunks, (unsigned)(cin / 16)), block(256);
+    switch (a.cout / 16) {
+    case 1: hipLaunchKernelGGL(conv3_wgrad_kernel<1>, grid, block, 0, s, a, dpre, part); break;
+    case 2: hipLaunchKernelGGL(conv3_wgrad_kernel<2>, grid, block, 0, s, a, dpre, part); break;
+    case 3: hipLaunchKernelGGL(conv3_wgrad_kernel<3>, grid, block, 0, s, a, dpre, part); break;
+    case 4: hipLaunchKernelGGL(conv3_wgrad_kernel<4>, grid, block, 0, s, a, dpre, part); break;
+    default: return hipErrorInvalidValue;
+    }
+    const size_t per = (size_t)kWgTaps * a.cout * cin;
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)((per + 63) / 64)), dim3(256), 0, s, part, chunks, cin, a.cout,
+                       grad_w, grad_b);
     return hipGetLastError();
 }
 
@@ -437,23 +506,6 @@ __global__ void relu_bwd_kernel(const float *g, const uint16_t *act, uint16_t *d
     const size_t i = (size_t)blockIdx.x * kEB + threadIdx.x;
     if (i >= n) return;
     dpre[i] = (act[i] & 0x7fffu) != 0 && !(act[i] & 0x8000u) ? f2bf(g[i]) : (uint16_t)0;
-}
-
-// bias gradient partials: part[chunk][c] = sum over the chunk's voxels of dpre[v][c]
-__global__ void bias_part_kernel(const uint16_t *dpre, size_t nvox, int C, float *part) {
-    const int c = threadIdx.x % C, lanes = blockDim.x / C, sub = threadIdx.x / C;
-    __shared__ float sh[256];
-    float s = 0.f;
-    const size_t vb = (size_t)blockIdx.x * kWgChunk, ve = min(nvox, vb + (size_t)kWgChunk);
-    if (sub < lanes)
-        for (size_t v = vb + sub; v < ve; v += lanes) s += bf2f(dpre[v * C + c]);
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    if ((int)threadIdx.x < C) {
-        float t = 0.f;
-        for (int k = 0; k < lanes; ++k) t += sh[k * C + threadIdx.x];
-        part[(size_t)blockIdx.x * C + threadIdx.x] = t;
-    }
 }
 
 // 1x1 output layer: y = w . act + b
@@ -752,8 +804,7 @@ hipError_t UNet::ensure_grid(int nx, int ny, int nz) {
         if ((e = gact_[i].ensure(nv * L.cout)) != hipSuccess) return e;
         gcat = std::max(gcat, nv * L.cin);
         dpre = std::max(dpre, nv * L.cout);
-        part = std::max(part, conv3_wgrad_chunks(nv) * 27 * L.cin * L.cout);
-        part = std::max(part, conv3_wgrad_chunks(nv) * L.cout);
+        part = std::max(part, conv3_wgrad_words(nx >> L.level, ny >> L.level, nz >> L.level, L.cin, L.cout));
     }
     part = std::max(part, (size_t)kRedBlocks * 17);
     for (int p = 0; p < 3; ++p) {
@@ -866,12 +917,9 @@ hipError_t UNet::backward(const float *dy, hipStream_t s) {
         hipLaunchKernelGGL(relu_bwd_kernel, dim3(eblocks(nv * L.cout)), dim3(kEB), 0, s, gact_[i].p, act_[i].p, dpre_.p,
                            nv * L.cout);
         const ConvArgs in = conv_in(i);
-        if ((e = launch_conv3_wgrad(in, dpre_.p, wpart_.p, grad_.p + unet_weight_offset(i), s)) != hipSuccess) return e;
-        const size_t chunks = conv3_wgrad_chunks(nv);
-        const int threads = std::min(256, (256 / L.cout) * L.cout);
-        hipLaunchKernelGGL(bias_part_kernel, dim3((unsigned)chunks), dim3(threads), 0, s, dpre_.p, nv, L.cout, wpart_.p);
-        hipLaunchKernelGGL(reduce_chunks_kernel, dim3(1), dim3(256), 0, s, wpart_.p, chunks, (size_t)L.cout,
-                           grad_.p + unet_bias_offset(i));
+        if ((e = launch_conv3_wgrad(in, dpre_.p, wpart_.p, grad_.p + unet_weight_offset(i), grad_.p + unet_bias_offset(i),
+                                    s)) != hipSuccess)
+            return e;
         if (i == 0) break;
         // data gradient: the same convolution on the flipped, transposed weights
         ConvArgs d;

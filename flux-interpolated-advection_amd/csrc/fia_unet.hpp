@@ -53,10 +53,11 @@ hipError_t launch_conv3(const ConvArgs &a, int mode, hipStream_t s);
 // per-cell flags of the fluid cells for the training loss: bits 0-5 = fluid neighbour at -x, +x,
 // -y, +y, -z, +z (0 on obstacle cells); solid may be null
 hipError_t launch_fluid_flags(const uint8_t *solid, int nx, int ny, int nz, uint8_t *flags, hipStream_t s);
-// weight gradient of a convolution: part (FP32, chunks * 27 * cout * cin) receives per-chunk sums,
-// then reduced in chunk order and added into grad_w [27][cout][cin]
-size_t conv3_wgrad_chunks(size_t vox);
-hipError_t launch_conv3_wgrad(const ConvArgs &in, const uint16_t *dpre, float *part, float *grad_w,
+// weight and bias gradient of a convolution, added into grad_w [27][cout][cin] and grad_b [cout]:
+// part (FP32, conv3_wgrad_words of them) receives the sums of conv3_wgrad_chunks runs of voxels
+int conv3_wgrad_chunks(int nx, int ny, int nz, int cin);
+size_t conv3_wgrad_words(int nx, int ny, int nz, int cin, int cout);
+hipError_t launch_conv3_wgrad(const ConvArgs &in, const uint16_t *dpre, float *part, float *grad_w, float *grad_b,
                               hipStream_t s);
 
 // The network: FP32 master parameters, their BF16 forward and transposed (data-gradient) copies,
