@@ -16,6 +16,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "fia_unet.hpp"
@@ -76,13 +77,13 @@ __device__ __forceinline__ bf16x4 load4(const ConvArgs &a, int x, int y, int z, 
 
 constexpr int kCB = 256;   // threads per convolution block (4 waves x 64 voxels)
 
-// Block tile of the convolution: 4 (x) x 4 (y) x 16 (z) voxels; wave w owns x-plane w of the tile,
-// its 4 row blocks are the tile's 4 y-rows of 16 z-voxels.  The input of the tile plus a one-voxel
-// halo (6 x 6 x 18 voxels) is staged in LDS for 32 input channels at a time and read by all 27
+// Block tile of the convolution: 4 (x) x M (y) x 16 (z) voxels; wave w owns x-plane w of the tile,
+// its M row blocks are the tile's y-rows of 16 z-voxels.  The input of the tile plus a one-voxel
+// halo (6 x (M + 2) x 18 voxels) is staged in LDS for 32 input channels at a time and read by all 27
 // taps.  Full 32-channel slices use v_mfma_f32_16x16x32_bf16 (lane l: A[l % 16][8 (l / 16) + i],
 // B[8 (l / 16) + i][l % 16], i < 8); a 16-channel tail uses the 16x16x16 form.
-constexpr int kTX = 4, kTY = 4, kTZ = 16;
-constexpr int kHX = kTX + 2, kHY = kTY + 2, kHZ = kTZ + 2, kHalo = kHX * kHY * kHZ;
+constexpr int kTX = 4, kTZ = 16;
+constexpr int kHX = kTX + 2, kHZ = kTZ + 2;
 constexpr int kSlice = 32, kSliceStride = kSlice + 8;   // LDS row: 32 channels + padding (bank spread)
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -101,9 +102,11 @@ __device__ __forceinline__ i16x8 load8(const ConvArgs &a, int x, int y, int z, i
 }
 
 // Stages input channels [c0, c0 + 8 groups) of the block's halo tile in LDS.
+template <int M>
 __device__ __forceinline__ void stage_slice(const ConvArgs &a, uint16_t *tile, int x0, int y0, int z0, int c0,
                                             int groups) {
-    for (int i = threadIdx.x; i < kHalo * groups; i += kCB) {
+    constexpr int kHY = M + 2;
+    for (int i = threadIdx.x; i < kHX * kHY * kHZ * groups; i += kCB) {
         const int g = i % groups, v = i / groups;
         const int hz = v % kHZ, hy = (v / kHZ) % kHY, hx = v / (kHZ * kHY);
         const int x = x0 - 1 + hx, y = y0 - 1 + hy, z = z0 - 1 + hz;
@@ -113,80 +116,80 @@ __device__ __forceinline__ void stage_slice(const ConvArgs &a, uint16_t *tile, i
     }
 }
 
-// All 27 taps over one staged slice: K = 32 channels (FULL, 16x16x32) or 16 (16x16x16).
-template <int NB, bool FULL>
-__device__ __forceinline__ void slice_taps(const ConvArgs &a, const uint16_t *tile, int c0, int cin, int wave, int row,
-                                           int grp, f32x4 (&acc)[4][NB]) {
+// All 27 taps over one staged slice: K = 32 channels (FULL, 16x16x32) or 16 (16x16x16), for the NB
+// column blocks from output channel n0.  The next tap's weights are loaded a tap ahead (from L2; at
+// one wave per SIMD their latency was most of a tap).
+template <int NB, bool FULL, int M>
+__device__ __forceinline__ void slice_taps(const ConvArgs &a, const uint16_t *tile, int c0, int cin, int n0, int wave,
+                                           int row, int grp, f32x4 (&acc)[M][NB]) {
+    constexpr int kHY = M + 2, kPer = FULL ? 8 : 4;   // channels per lane
+    using Frag = typename std::conditional<FULL, bf16x8, bf16x4>::type;
+    const uint16_t *wt = a.w + c0 + (size_t)(n0 + row) * cin + kPer * grp;
+    const size_t tap = (size_t)a.cout * cin;
+    Frag B[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) B[n] = *reinterpret_cast<const Frag *>(wt + (size_t)(n * 16) * cin);
+#pragma unroll 1
     for (int t = 0; t < 27; ++t) {
         const int dx = t / 9, dy = (t / 3) % 3, dz = t % 3;   // halo offsets 0..2
-        const uint16_t *wt = a.w + (size_t)t * a.cout * cin + c0;
-        if (FULL) {
-            bf16x8 A[4];
+        const uint16_t *wn = wt + (size_t)min(t + 1, 26) * tap;
+        Frag next[NB], A[M];
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const int v = ((wave + dx) * kHY + (m + dy)) * kHZ + (row + dz);
-                A[m] = *reinterpret_cast<const bf16x8 *>(&tile[v * kSliceStride + 8 * grp]);
-            }
+        for (int n = 0; n < NB; ++n) next[n] = *reinterpret_cast<const Frag *>(wn + (size_t)(n * 16) * cin);
 #pragma unroll
-            for (int n = 0; n < NB; ++n) {
-                const bf16x8 B = *reinterpret_cast<const bf16x8 *>(wt + (size_t)(n * 16 + row) * cin + 8 * grp);
+        for (int m = 0; m < M; ++m) {
+            const int v = ((wave + dx) * kHY + (m + dy)) * kHZ + (row + dz);
+            A[m] = *reinterpret_cast<const Frag *>(&tile[v * kSliceStride + kPer * grp]);
+        }
 #pragma unroll
-                for (int m = 0; m < 4; ++m)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], B, acc[m][n], 0, 0, 0);
-            }
-        } else {
-            bf16x4 A[4];
+        for (int n = 0; n < NB; ++n) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const int v = ((wave + dx) * kHY + (m + dy)) * kHZ + (row + dz);
-                A[m] = *reinterpret_cast<const bf16x4 *>(&tile[v * kSliceStride + 4 * grp]);
-            }
-#pragma unroll
-            for (int n = 0; n < NB; ++n) {
-                const bf16x4 B = *reinterpret_cast<const bf16x4 *>(wt + (size_t)(n * 16 + row) * cin + 4 * grp);
-#pragma unroll
-                for (int m = 0; m < 4; ++m)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[m], B, acc[m][n], 0, 0, 0);
+            for (int m = 0; m < M; ++m) {
+                if constexpr (FULL) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], B[n], acc[m][n], 0, 0, 0);
+                else acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[m], B[n], acc[m][n], 0, 0, 0);
             }
         }
+#pragma unroll
+        for (int n = 0; n < NB; ++n) B[n] = next[n];
     }
 }
 
-template <int NB, int MODE>
+// blockIdx.y: the block's NB column blocks of output channels
+template <int NB, int MODE, int M>
 __global__ void __launch_bounds__(kCB) conv3_kernel(ConvArgs a) {
-    __shared__ uint16_t tile[kHalo * kSliceStride];
+    __shared__ uint16_t tile[kHX * (M + 2) * kHZ * kSliceStride];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = lane & 15, grp = lane >> 4;
-    const int tx = (a.nx + kTX - 1) / kTX, ty = (a.ny + kTY - 1) / kTY;
+    const int tx = (a.nx + kTX - 1) / kTX, ty = (a.ny + M - 1) / M;
     const int bx = blockIdx.x % tx, by = (blockIdx.x / tx) % ty, bz = blockIdx.x / (tx * ty);
-    const int x0 = bx * kTX, y0 = by * kTY, z0 = bz * kTZ;
+    const int x0 = bx * kTX, y0 = by * M, z0 = bz * kTZ, n0 = blockIdx.y * NB * 16;
     const int cin = a.cA + a.cB;
-    f32x4 acc[4][NB];
+    f32x4 acc[M][NB];
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < M; ++m)
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int full = cin / kSlice * kSlice;
     for (int c0 = 0; c0 < full; c0 += kSlice) {
         __syncthreads();   // the previous slice's reads are done
-        stage_slice(a, tile, x0, y0, z0, c0, kSlice / 8);
+        stage_slice<M>(a, tile, x0, y0, z0, c0, kSlice / 8);
         __syncthreads();
-        slice_taps<NB, true>(a, tile, c0, cin, wave, row, grp, acc);
+        slice_taps<NB, true, M>(a, tile, c0, cin, n0, wave, row, grp, acc);
     }
     if (full < cin) {   // a 16-channel tail
         __syncthreads();
-        stage_slice(a, tile, x0, y0, z0, full, 2);
+        stage_slice<M>(a, tile, x0, y0, z0, full, 2);
         __syncthreads();
-        slice_taps<NB, false>(a, tile, full, cin, wave, row, grp, acc);
+        slice_taps<NB, false, M>(a, tile, full, cin, n0, wave, row, grp, acc);
     }
     // D[i][j] in lane l: j = l % 16 (output channel), i = 4 (l / 16) + r (z-voxel of the row block)
     const int x = x0 + wave;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < M; ++m) {
         const int y = y0 + m;
 #pragma unroll
         for (int n = 0; n < NB; ++n) {
-            const int co = n * 16 + row;
+            const int co = n0 + n * 16 + row;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int z = z0 + 4 * grp + r;
@@ -197,27 +200,42 @@ __global__ void __launch_bounds__(kCB) conv3_kernel(ConvArgs a) {
                     val += a.bias[co];
                     if (a.relu) val = fmaxf(val, 0.f);
                     static_cast<uint16_t *>(a.out)[v * a.cout + co] = f2bf(val);
-                } else if (MODE == 1) {
-                    static_cast<float *>(a.out)[v * a.cout + co] = val;
                 } else {
-                    static_cast<float *>(a.out)[v * a.cout + co] += val;
+                    static_cast<float *>(a.out)[v * a.cout + co] = val;
                 }
             }
         }
     }
 }
 
+// One block computes every output channel of its tile while that gives each CU a block; below that
+// each takes 16 channels, and below that one y-row as well: a level of 8^3 voxels is 4 blocks of
+// 64 channels (60 us, nearly all latency) or 64 of 16 (18 us).  Every output sums the same
+// products in the same order in all forms.
 template <int MODE>
 static hipError_t conv3_nb(const ConvArgs &a, hipStream_t s) {
-    const long tiles = (long)((a.nx + kTX - 1) / kTX) * ((a.ny + kTY - 1) / kTY) * ((a.nz + kTZ - 1) / kTZ);
-    const dim3 grid((unsigned)tiles);
-    switch (a.cout / 16) {
-    case 1: hipLaunchKernelGGL((conv3_kernel<1, MODE>), grid, dim3(kCB), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((conv3_kernel<2, MODE>), grid, dim3(kCB), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((conv3_kernel<3, MODE>), grid, dim3(kCB), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((conv3_kernel<4, MODE>), grid, dim3(kCB), 0, s, a); break;
-    case 5: hipLaunchKernelGGL((conv3_kernel<5, MODE>), grid, dim3(kCB), 0, s, a); break;
-    case 7: hipLaunchKernelGGL((conv3_kernel<7, MODE>), grid, dim3(kCB), 0, s, a); break;
+    constexpr long kFill = 256;
+    const auto tiles = [&](int m) {
+        return (long)((a.nx + kTX - 1) / kTX) * ((a.ny + m - 1) / m) * ((a.nz + kTZ - 1) / kTZ);
+    };
+    const int nb = a.cout / 16;
+    const long big = tiles(4);
+    if (big < kFill && big * nb < kFill) {
+        hipLaunchKernelGGL((conv3_kernel<1, MODE, 1>), dim3((unsigned)tiles(1), (unsigned)nb), dim3(kCB), 0, s, a);
+        return hipGetLastError();
+    }
+    if (big < kFill) {
+        hipLaunchKernelGGL((conv3_kernel<1, MODE, 4>), dim3((unsigned)big, (unsigned)nb), dim3(kCB), 0, s, a);
+        return hipGetLastError();
+    }
+    const dim3 grid((unsigned)big);
+    switch (nb) {
+    case 1: hipLaunchKernelGGL((conv3_kernel<1, MODE, 4>), grid, dim3(kCB), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((conv3_kernel<2, MODE, 4>), grid, dim3(kCB), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((conv3_kernel<3, MODE, 4>), grid, dim3(kCB), 0, s, a); break;
+    case 4: hipLaunchKernelGGL((conv3_kernel<4, MODE, 4>), grid, dim3(kCB), 0, s, a); break;
+    case 5: hipLaunchKernelGGL((conv3_kernel<5, MODE, 4>), grid, dim3(kCB), 0, s, a); break;
+    case 7: hipLaunchKernelGGL((conv3_kernel<7, MODE, 4>), grid, dim3(kCB), 0, s, a); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -227,9 +245,7 @@ hipError_t launch_conv3(const ConvArgs &a, int mode, hipStream_t s) {
     if (a.cout % 16 || (a.cA + a.cB) % 16 || a.cA % 16 || a.nx <= 0 || a.ny <= 0 || a.nz <= 0)
         return hipErrorInvalidValue;
     if (a.upA && (a.nx % 2 || a.ny % 2 || a.nz % 2)) return hipErrorInvalidValue;
-    if (mode == 0) return conv3_nb<0>(a, s);
-    if (mode == 1) return conv3_nb<1>(a, s);
-    return conv3_nb<2>(a, s);
+    return mode == 0 ? conv3_nb<0>(a, s) : conv3_nb<1>(a, s);
 }
 
 // ---- weight and bias gradient -------------------------------------------------------------------

@@ -48,7 +48,7 @@ struct ConvArgs {
     int relu;                      // forward: ReLU on the output
 };
 
-// mode 0: BF16 output with bias (+ ReLU); 1: FP32 output; 2: FP32 output added to what is there
+// mode 0: BF16 output with bias (+ ReLU); 1: FP32 output
 hipError_t launch_conv3(const ConvArgs &a, int mode, hipStream_t s);
 // per-cell flags of the fluid cells for the training loss: bits 0-5 = fluid neighbour at -x, +x,
 // -y, +y, -z, +z (0 on obstacle cells); solid may be null
