@@ -685,6 +685,15 @@ static fia_status pressure_system(fia_ctx *c, const fia_grid3d *g, const GridVie
     return assemble_system(c, g, gv, solid ? c->solid.p : nullptr, c->pcg_b.p, c->pcg_flags.p, pg);
 }
 
+// Whether a Jacobi solve with the device to itself runs the fused sweep.  By default it does: one
+// launch and one pass over the partial sums per iteration instead of two (fused and two-sweep
+// iterations: 32^3 12.9 and 15.2 us, 64^3 12.7 and 16.2, 128^3 26.0 and 36.6, 160^3 42.9 and 59.7,
+// 256^3 137 and 203); a shape tuned for one of the two-sweep update forms keeps it under 4M cells.
+static bool fused_choice(const fia_tuning &t, size_t cells) {
+    if (t.pcg_fused >= 0) return t.pcg_fused == 1;
+    return t.pcg_recompute < 0 || cells >= ((size_t)1 << 22);
+}
+
 // Buffers B (allocated here for the grid of pg) bound into a CG state over the system (b, flags).
 // batched: the solve joins fia_scenes_step_batched's launches, which run the two-kernel iteration.
 // shared: other scenes' solves share the device (a step of several scenes): the tiles are sized by
@@ -694,10 +703,7 @@ static fia_status bind_solve(fia_ctx::PcgBufs &B, const PcgGrid &pg, const doubl
                              PcgState &ps, bool mg, const fia_tuning &tu, bool batched, bool shared) {
     const size_t n = (size_t)pg.nx * pg.ny * pg.nz;
     ps.nblocks = pcg_blocks(n);
-    // fused by default from 4M cells (256^3: 191 against 203 us per iteration at the best chunking;
-    // 128^3: even)
-    ps.fused = !mg && !batched && !shared &&
-               (tu.pcg_fused == 1 || (tu.pcg_fused == -1 && n >= ((size_t)1 << 22)));
+    ps.fused = !mg && !batched && !shared && fused_choice(tu, n);
     pcg_direction_tiling(pg.nx, pg.ny, pg.nz, ps, tu.pcg_chunk_x, tu.pcg_recompute, shared);
     HIP_TRY(B.x.ensure(n)); HIP_TRY(B.r.ensure(n)); HIP_TRY(B.p0.ensure(n)); HIP_TRY(B.p1.ensure(n));
     HIP_TRY(B.part.ensure(pcg_partial_words(ps))); HIP_TRY(B.scal.ensure(kPcgScalars));
@@ -1328,7 +1334,7 @@ fia_status fia_ctx_autotune(fia_ctx *c, const fia_grid3d *g, const uint8_t *soli
     const size_t ncells = (size_t)pg.nx * pg.ny * pg.nz;
     auto launch_key = [&](const fia_tuning &t) {
         PcgState ps;
-        ps.fused = !use_mg && (t.pcg_fused == 1 || (t.pcg_fused == -1 && ncells >= ((size_t)1 << 22)));
+        ps.fused = !use_mg && fused_choice(t, ncells);
         pcg_direction_tiling(pg.nx, pg.ny, pg.nz, ps, t.pcg_chunk_x, t.pcg_recompute);
         return std::make_pair(ps.dir_chunk_x, ps.fused ? 2 : (int)ps.recompute_q);
     };

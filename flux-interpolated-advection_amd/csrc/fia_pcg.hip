@@ -23,8 +23,8 @@
 // streaming; the update reads 4 (p) + 8 x 2 (x, r) + 1, plus 8 (q) when streaming, and writes 16
 // (x, r): 70 bytes streaming, 54 recomputing.  Recomputing pays where the tiles sweep
 // long x chunks (large grids); on small grids, whose chunks are a few planes, the halo planes
-// cost more than q and the streaming form is faster.  Under Jacobi on grids of at least 4 M
-// cells one kernel per iteration replaces the two (pcg_fused_kernel, below: 35 bytes per cell
+// cost more than q and the streaming form is faster.  Under Jacobi, for a solve that has the
+// device to itself, one kernel per iteration replaces the two (pcg_fused_kernel, below: 35 bytes per cell
 // and iteration), and a geometric multigrid V-cycle can replace the Jacobi preconditioner.
 //
 // Reductions without fences: every block writes its partial sums with plain stores, and every
@@ -1504,6 +1504,29 @@ int pcg_resident_blocks(bool fused) {
     return v;
 }
 
+// A fused sweep whose vectors stay in the last-level cache (45 bytes a cell) is bound by its blocks'
+// chain of planes, not by memory, and the round need not be full: with 1, 2 or 3 blocks on every CU
+// a sweep of c planes per block took about 10.2 + 2.25 c, 13.4 + 2.85 c and 13.3 + 4.3 c us (grids of
+// 64^3 to 160^3).  The least of the three: 128^3 runs chunks of 4 planes, 512 blocks, in 26.0 us an
+// iteration against 28.2 for the full round's 3 planes and 29.0 for 256 blocks of 8.  Larger grids
+// are bound by memory and fill the round (256^3).
+constexpr size_t kCachedCells = (size_t)1 << 22;
+static long fused_chunks(int nx, long tiles, int resident) {
+    constexpr double fixed[3] = {10.2, 13.4, 13.3}, plane[3] = {2.25, 2.85, 4.3};
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        return std::max<long>(1, std::min<long>(nx, resident / tiles));
+    long best = 1;
+    double least = 1e300;
+    for (int k = 1; k <= 3 && k * cus <= resident; ++k) {
+        const long chunks = std::max<long>(1, std::min<long>(nx, (long)k * cus / tiles));
+        const double t = fixed[k - 1] + plane[k - 1] * (double)((nx + chunks - 1) / chunks);
+        if (t < least) { least = t; best = chunks; }
+    }
+    return best;
+}
+
 // Tiling of the tile sweeps: kTileZ x kTileY column tiles, x cut into chunks so that the launch
 // has about as many blocks as fit on the device at once (one full round: on 256^3 a 22-plane
 // chunk, 768 blocks at 3 per CU, ran the iteration in 191-203 us against 236-246 us for 16-plane
@@ -1517,7 +1540,9 @@ void pcg_direction_tiling(int nx, int ny, int nz, PcgState &st, int chunk_x, int
     const int resident = shared ? 0 : pcg_resident_blocks(st.fused);
     // chunks per tile column: as many as fit in one round of resident blocks (rounded down: a few
     // blocks over the round would run alone in a second one)
-    const long want = resident > 0 ? std::max<long>(1, std::min<long>(nx, resident / tiles))
+    const bool cached = resident > 0 && st.fused && (size_t)nx * ny * nz < kCachedCells;
+    const long want = cached ? fused_chunks(nx, tiles, resident)
+                    : resident > 0 ? std::max<long>(1, std::min<long>(nx, resident / tiles))
                                    : std::max<long>(1, std::min<long>(nx, ((long)target_blocks((size_t)nx * ny * nz) +
                                                                            tiles - 1) / tiles));
     st.dir_chunk_x = chunk_x > 0 ? std::min(chunk_x, nx) : (int)((nx + want - 1) / want);
