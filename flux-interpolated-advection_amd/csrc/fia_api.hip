@@ -120,8 +120,8 @@ struct fia_ctx {
     DevBuf<uint8_t> pcg_flags;    // per-cell neighbour flags of the pressure system
     struct PcgBufs {              // one CG solve: x, r, p (two buffers), q (streaming update), z and r.z
                                   // partials (multigrid), partials, scalars
-        DevBuf<double> x, r, r_alt, q, z, part_mg, part, scal;
-        DevBuf<float> p0, p1;   // the search direction
+        DevBuf<double> x, r, r_alt, q, part_mg, part, scal;
+        DevBuf<float> p0, p1, z;   // the search direction
         size_t bytes() const {
             return x.bytes() + r.bytes() + r_alt.bytes() + p0.bytes() + p1.bytes() + q.bytes() + z.bytes() +
                    part_mg.bytes() + part.bytes() + scal.bytes();
@@ -136,13 +136,15 @@ struct fia_ctx {
     struct MgBufs {
         DevBuf<float4> op[kMgMaxLevels];
         DevBuf<float> b[kMgMaxLevels], x[kMgMaxLevels], xs[kMgMaxLevels];
+        DevBuf<float> dense;   // the coarsest level's map
         size_t bytes() const {
-            size_t t = 0;
+            size_t t = dense.bytes();
             for (int l = 0; l < kMgMaxLevels; ++l) t += op[l].bytes() + b[l].bytes() + x[l].bytes() + xs[l].bytes();
             return t;
         }
         void release() {
             for (int l = 0; l < kMgMaxLevels; ++l) { op[l].release(); b[l].release(); x[l].release(); xs[l].release(); }
+            dense.release();
         }
     } mgb;
     MgHier mgh;
@@ -659,11 +661,10 @@ static fia_status assemble_system(fia_ctx *c, const fia_grid3d *g, const GridVie
     pg.nx = g->nx; pg.ny = g->ny; pg.nz = g->nz; pg.solid = solid_dev; pg.pin = (long)n - 1;
     if (solid_dev) {
         // last fluid cell is pinned (the reference pins the last cell, which has no obstacles)
-        std::vector<uint8_t> hs(n);
-        HIP_TRY(hipMemcpyAsync(hs.data(), solid_dev, n, hipMemcpyDeviceToHost, c->stream));
+        long long *last = (long long *)c->host_bounds;   // [0], a read-back
+        HIP_TRY(launch_last_fluid(solid_dev, n, last, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
-        long pin = -1;
-        for (long i = (long)n - 1; i >= 0; --i) if (!hs[i]) { pin = i; break; }
+        const long pin = (long)*(volatile long long *)last;
         if (pin < 0) return fail(FIA_ERR_INVALID_ARG, "every cell is solid");
         pg.pin = pin;
         HIP_TRY(launch_zero_solid_faces(pg, gv.u, gv.v, gv.w, c->stream));
@@ -718,6 +719,7 @@ static fia_status bind_solve(fia_ctx::PcgBufs &B, const PcgGrid &pg, const doubl
     ps.part_mg = mg ? B.part_mg.p : nullptr;
     ps.mg_lv = nullptr;
     ps.mg_levels = 0;
+    ps.mg_tail = 0;
     ps.scal = B.scal.p; ps.part_start = B.part.p; ps.part_dir = B.part.p + 3 * (size_t)ps.nblocks;
     ps.part_update = ps.part_dir + ps.dir_blocks;
     ps.part_fused = ps.fused ? ps.part_update + 2 * (size_t)ps.upd_blocks : nullptr;
@@ -730,7 +732,7 @@ static fia_status bind_solve(fia_ctx::PcgBufs &B, const PcgGrid &pg, const doubl
 static fia_status mg_setup(hipStream_t stream, fia_ctx::MgBufs &B, MgHier &h, const PcgState &ps) {
     mg_shape(ps.g.nx, ps.g.ny, ps.g.nz, h);
     const MgLevel &top = h.lv[h.levels - 1];
-    if ((size_t)top.nx * top.ny * top.nz > 256) return fail(FIA_ERR_UNSUPPORTED, "grid too large for the multigrid levels");
+    if ((size_t)top.nx * top.ny * top.nz > (size_t)kMgCoarsestCells) return fail(FIA_ERR_UNSUPPORTED, "grid too large for the multigrid levels");
     for (int l = 0; l < h.levels; ++l) {
         MgLevel &L = h.lv[l];
         const size_t n = (size_t)L.nx * L.ny * L.nz;
@@ -743,6 +745,9 @@ static fia_status mg_setup(hipStream_t stream, fia_ctx::MgBufs &B, MgHier &h, co
             L.op = B.op[l].p; L.xs = B.xs[l].p;
         }
     }
+    const size_t coarsest = (size_t)top.nx * top.ny * top.nz;
+    HIP_TRY(B.dense.ensure(coarsest * coarsest));
+    h.lv[h.levels - 1].dense = B.dense.p;
     HIP_TRY(launch_mg_build(ps, h, stream));
     return FIA_OK;
 }
@@ -887,6 +892,7 @@ fia_status scene_solve_setup(fia_ctx *cw, fia_ctx *main, int s, fia_scene *sc, f
         HIP_TRY(hipMemcpyAsync(sv.lv_dev.p, sv.mgh.lv, sizeof(sv.mgh.lv), hipMemcpyHostToDevice, cw->stream));
         sa.mg_lv = sv.lv_dev.p;
         sa.mg_levels = sv.mgh.levels;
+        sa.mg_tail = mg_tail_level(sv.mgh);
         mg = &sv.mgh;
     }
     if (net) {
@@ -896,6 +902,7 @@ fia_status scene_solve_setup(fia_ctx *cw, fia_ctx *main, int s, fia_scene *sc, f
             return st;
         sb.mg_lv = sa.mg_lv;
         sb.mg_levels = sa.mg_levels;
+        sb.mg_tail = sa.mg_tail;
         LearnedStart ls;
         if ((st = learned_start(cw, net, sv.pg, sa, sb, tol2, std::min(5, max_iters), cw->host_scal,
                                 cw->host_scal + kPcgScalars, ls, mg)) != FIA_OK)
@@ -951,7 +958,7 @@ fia_status scenes_solve_run(fia_ctx *c, fia_scene *scenes, const int *idx, int m
             down_off[l] = (int)map.size();
             for (int j = 0; j < m; ++j) {
                 const MgHier &h = c->solves[idx[j]].mgh;
-                if (l + 1 < h.levels)
+                if (l < mg_tail_level(h))
                     for (int k = 0; k < mg_down_tiles(h.lv[l]); ++k) map.push_back(make_int2(j, k));
             }
             mb.down_blocks[l] = (int)map.size() - down_off[l];
@@ -960,7 +967,7 @@ fia_status scenes_solve_run(fia_ctx *c, fia_scene *scenes, const int *idx, int m
             up_off[l] = (int)map.size();
             for (int j = 0; j < m; ++j) {
                 const MgHier &h = c->solves[idx[j]].mgh;
-                if (l + 1 < h.levels) {
+                if (l < mg_tail_level(h)) {
                     const size_t n = (size_t)h.lv[l].nx * h.lv[l].ny * h.lv[l].nz;
                     for (size_t k = 0; k < (n + 255) / 256; ++k) map.push_back(make_int2(j, (int)k));
                 }

@@ -260,10 +260,11 @@ struct PcgState {
                           // runs iteration k after testing iteration k - 1
     // multigrid preconditioner (null for Jacobi): z = M r written by the last V-cycle kernel, with
     // dir_blocks partial sums of r.z in part_mg
-    double *z;
+    float *z;
     double *part_mg;
     const MgLevel *mg_lv;   // the solve's levels in device memory (batched V-cycles), mg_levels of them
     int mg_levels;
+    int mg_tail;            // mg_tail_level of those levels
     int it;             // iterations enqueued since the start (selects the p buffer)
 };
 int pcg_blocks(size_t n);
@@ -287,7 +288,10 @@ struct MgLevel {
     float *b;         // right-hand side (level 0: the residual of the first sweep; it reads r)
     float *x;         // pre-smoothed iterate (the coarsest level: its solution)
     float *xs;        // post-smoothed iterate (levels 1 .. L-2)
+    float *dense;     // the coarsest level: its sweeps as a matrix, column e at dense + e cells
 };
+constexpr int kMgCoarsestCells = 256;   // most cells of the coarsest level
+constexpr int kMgTailCells = 5120;      // most cells of the tail's smoothed levels together
 struct MgHier {
     int levels = 0;
     MgLevel lv[kMgMaxLevels];
@@ -298,7 +302,7 @@ __host__ __device__ inline int mg_down_tiles(const MgLevel &F) {
     return ((F.nz + kMgTileZ - 1) / kMgTileZ) * ((F.ny + 1) / 2) * ((F.nx + 1) / 2);
 }
 // block maps (solve, block of that solve's launch) of a batched V-cycle: level 1's restriction,
-// and per level l >= 1 the down and up launches of the solves that have level l + 1
+// and per level l >= 1 the down and up launches of the solves whose tail starts below it
 struct MgBatch {
     const int2 *r0_map;
     int r0_blocks;
@@ -307,6 +311,9 @@ struct MgBatch {
     const int2 *up_map[kMgMaxLevels];
     int up_blocks[kMgMaxLevels];
 };
+// the first level of the V-cycle's tail, the levels that one block runs: at least 1, at most the
+// coarsest
+int mg_tail_level(const MgHier &h);
 // dims of every level for a grid (coarsest: at most 256 cells or kMgMaxLevels levels)
 void mg_shape(int nx, int ny, int nz, MgHier &h);
 // coarse operators of levels 1 .. L-1 from the solve's flag bytes
@@ -392,6 +399,8 @@ class PcgGraphCache {
 };
 hipError_t launch_project(const PcgGrid &g, const double *p, double h, float *u, float *v, float *w,
                           float *pressure_out, hipStream_t s);
+// *out (host memory the device can store to) = the last cell that is not solid, -1 for none
+hipError_t launch_last_fluid(const uint8_t *solid, size_t n, long long *out, hipStream_t s);
 hipError_t launch_zero_solid_faces(const PcgGrid &g, float *u, float *v, float *w, hipStream_t s);
 
 // context accessors and the calling thread's error message (fia_api.hip), for other host files

@@ -34,6 +34,7 @@
 // reads a scalar that another block of the same kernel writes.  Once converged every later kernel
 // of the solve returns at once, so the host only polls now and then (after a 1-block check).
 #include <atomic>
+#include <type_traits>
 
 #include "fia_internal.hpp"
 #include "fia_math.hpp"
@@ -290,31 +291,33 @@ __device__ __forceinline__ bool in_grid(const PcgGrid &g, int x, int y, int z) {
 __device__ __forceinline__ size_t clamped_cell(const PcgGrid &g, int x, int y, int z) {
     return idx3(min(max(x, 0), g.nx - 1), min(max(y, 0), g.ny - 1), min(max(z, 0), g.nz - 1), g.ny, g.nz);
 }
-struct DirRaw {
+template <bool MG> struct DirRaw {
     unsigned f;
-    double r;
+    typename std::conditional<MG, float, double>::type r;
     float p;
 };
-struct DirOp {
-    using Raw = DirRaw;
+template <bool MG> struct DirOp {
+    using Raw = DirRaw<MG>;
     const PcgState &st;
     const float *__restrict__ pold;
     float *__restrict__ pnew;
     double beta;
-    // Jacobi: r (z = r / diag on the fly); multigrid: the V-cycle's z
+    // Jacobi: r (z = r / diag on the fly); multigrid: the V-cycle's z (FP32, as the cycle computes it)
     __device__ __forceinline__ Raw load(int x, int y, int z, bool) const {
         const size_t c = clamped_cell(st.g, x, y, z);
-        const double *rz = st.z ? st.z : st.r;
         const unsigned f = st.flags[c];
-        const double r = rz[c];
+        decltype(Raw::r) r;
+        if constexpr (MG) r = st.z[c];
+        else r = st.r[c];
         const float p = pold[c];
         const bool in = in_grid(st.g, x, y, z);
-        return Raw{in ? f : 0u, in ? r : 0.0, in ? p : 0.0f};
+        return Raw{in ? f : 0u, in ? r : 0, in ? p : 0.0f};
     }
     // the direction rounded to FP32 here, before the stencil: q = L p and p.q are those of the
     // stored p, which the update reads back
     __device__ __forceinline__ double value(const Raw &a) const {
-        return (double)(float)((st.z ? a.r : a.r * inv_diag(a.f)) + beta * (double)a.p);
+        if constexpr (MG) return (double)(float)((double)a.r + beta * (double)a.p);
+        else return (double)(float)(a.r * inv_diag(a.f) + beta * (double)a.p);
     }
     __device__ __forceinline__ void cell(size_t c, const Raw &, double v, double q, double *acc) const {
         pnew[c] = (float)v;
@@ -465,7 +468,7 @@ __device__ __forceinline__ void tile_sweep(const PcgState &st, int blk, const Op
     }
 }
 
-__device__ __forceinline__ void pcg_direction_body(const PcgState &st, int blk, int k) {
+template <bool MG> __device__ __forceinline__ void pcg_direction_body(const PcgState &st, int blk, int k) {
     const float *__restrict__ pold = st.p[k & 1];
     float *__restrict__ pnew = st.p[(k + 1) & 1];
     // the converged flag read with the partials (one round trip), tested before any write
@@ -486,7 +489,7 @@ __device__ __forceinline__ void pcg_direction_body(const PcgState &st, int blk, 
     }
     if (done) return;
     double acc[1] = {0.0};
-    tile_sweep(st, blk, DirOp{st, pold, pnew, beta}, acc);
+    tile_sweep(st, blk, DirOp<MG>{st, pold, pnew, beta}, acc);
     write_partials<1>(acc, st.part_dir, st.dir_blocks, blk);
 }
 
@@ -943,6 +946,26 @@ __global__ void project_kernel(PcgGrid g, const double *p, double h, float *u, f
         w[idx3(i, j, k, ny, nz + 1)] = (float)((double)w[idx3(i, j, k, ny, nz + 1)] - (p[c] - p[c - 1]) / h);
 }
 
+// Index of the last fluid cell, -1 for none, stored to *out (host memory): one block reads the mask
+// from its end, 16 KB a step, and stops at the first step that has one (nearly always the first).
+constexpr int kLastThreads = 1024, kLastBytes = 16;
+__global__ void __launch_bounds__(kLastThreads) last_fluid_kernel(const uint8_t *solid, long n, long long *out) {
+    __shared__ long long best;
+    if (threadIdx.x == 0) best = -1;
+    __syncthreads();
+    for (long end = n; end > 0; end -= (long)kLastThreads * kLastBytes) {
+        const long hi = end - (long)threadIdx.x * kLastBytes, lo = max(0L, hi - kLastBytes);
+        long long mine = -1;
+        for (long c = lo; c < hi; ++c)
+            if (!solid[c]) mine = c;
+        if (mine >= 0) atomicMax(&best, mine);
+        __syncthreads();
+        if (best >= 0) break;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = best;
+}
+
 __global__ void zero_solid_faces_kernel(PcgGrid g, float *u, float *v, float *w) {
     const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long n = (long)g.nx * g.ny * g.nz;
@@ -975,7 +998,6 @@ __global__ void pcg_guess_kernel(PcgState st, const float *p_in) {
 constexpr float kMgOmega = 0.9f;
 constexpr int kMgCoarseSweeps = 48;
 constexpr float kMgCorrScale = 1.8f;
-constexpr int kMgCoarsestCells = 256;
 
 // A cell of a level: unknown, diagonal and the weights to its six neighbours (-x, +x, -y, +y, -z,
 // +z).  Level 0 reads the flag byte (weight 1 to each fluid neighbour, the diagonal counts them);
@@ -1052,89 +1074,44 @@ __global__ void __launch_bounds__(kPB) mg_build_kernel(PcgState st, MgLevel F, M
     C.op[I] = make_float4(d, wp[0], wp[1], wp[2]);
 }
 
-// b and L x of a cell at level l (level 0: b = r, FP64 in memory)
-__device__ __forceinline__ float mg_b(const PcgState &st, const MgLevel &L, int l, size_t c) {
-    return l == 0 ? (float)st.r[c] : L.b[c];
-}
+// The first smoothing sweep from zero, x = w b / d (0 on a cell that is not an unknown).
+__device__ __forceinline__ float mg_presmooth(float b, float d) { return d > 0.0f ? kMgOmega * b / d : 0.0f; }
 
-// Down the V-cycle at level l, one thread per cell of a 2 x 2 x 64 tile (32 aggregates of level
-// l + 1 along z): every unknown cell gets the first smoothing sweep from zero, x = w b / d, and
-// its residual b - L x (the neighbours' x recomputed from their b); each aggregate's right-hand
-// side is the sum of its eight children's residuals, added in a fixed order through LDS.
-// The down step's residual of cell (i, j, k) of a level l >= 1 (x = w b / d on every unknown),
-// with every load issued at once: the cell's operator record and those of its -x, -y, -z
-// neighbours (the weights), and each neighbour's record and right-hand side, from indices clamped
-// into the grid.  A neighbour that is outside, not an unknown, or joined by a zero weight adds
-// (its term) * 0 with a denominator that cannot be 0; the others add what the tested form adds.
-__device__ __forceinline__ float mg_down_cell_coarse(const MgLevel &F, int i, int j, int k) {
+// Down the V-cycle at level l >= 1, one thread per cell of a 2 x 2 x 64 tile (32 aggregates of level
+// l + 1 along z): the residual b - L x of the pre-smoothed x, which the step that made b stored with
+// it; each aggregate's right-hand side is the sum of its eight children's residuals, added in a fixed
+// order through LDS, and stored with its own pre-smoothed x.
+// The residual of cell (i, j, k), with every load issued at once: the cell's operator record and those
+// of its -x, -y, -z neighbours (the weights), and each neighbour's x from an index clamped into the
+// grid.  A neighbour that is outside has weight 0, one that is not an unknown has x = 0.
+__device__ __forceinline__ float mg_residual_cell(const MgLevel &F, int i, int j, int k) {
     const int sx = F.ny * F.nz, sy = F.nz;
     const int c = (i * F.ny + j) * F.nz + k;
     const float4 o = F.op[c];
     const float4 oxm = F.op[i > 0 ? c - sx : c], oym = F.op[j > 0 ? c - sy : c], ozm = F.op[k > 0 ? c - 1 : c];
-    const float bc = F.b[c];
-    const float w[6] = {oxm.y * (float)(i > 0), o.y, oym.z * (float)(j > 0), o.z, ozm.w * (float)(k > 0), o.w};
-    float dn[6], bn[6];
-    bool in[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        int ni, nj, nk;
-        mg_neighbour(q, i, j, k, ni, nj, nk);
-        in[q] = ni >= 0 && nj >= 0 && nk >= 0 && ni < F.nx && nj < F.ny && nk < F.nz;
-        const int cn = (clampi(ni, 0, F.nx - 1) * F.ny + clampi(nj, 0, F.ny - 1)) * F.nz + clampi(nk, 0, F.nz - 1);
-        dn[q] = F.op[cn].x;
-        bn[q] = F.b[cn];
-    }
-    if (!(o.x > 0.0f)) {
-        F.x[c] = 0.0f;
-        return 0.0f;
-    }
-    const float d = o.x;
-    const float xc = kMgOmega * bc / d;
-    F.x[c] = xc;
-    float lx = d * xc;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        const bool use = w[q] != 0.0f && in[q] && dn[q] > 0.0f;
-        const float dq = dn[q] + (use ? 0.0f : 1.0f);
-        lx -= (w[q] * (kMgOmega * bn[q] / dq)) * (float)use;
-    }
+    const float bc = F.b[c], xc = F.x[c];
+    const float x0 = F.x[i > 0 ? c - sx : c], x1 = F.x[i + 1 < F.nx ? c + sx : c];
+    const float x2 = F.x[j > 0 ? c - sy : c], x3 = F.x[j + 1 < F.ny ? c + sy : c];
+    const float x4 = F.x[k > 0 ? c - 1 : c], x5 = F.x[k + 1 < F.nz ? c + 1 : c];
+    if (!(o.x > 0.0f)) return 0.0f;
+    float lx = o.x * xc;
+    lx -= (i > 0 ? oxm.y : 0.0f) * x0;
+    lx -= (i + 1 < F.nx ? o.y : 0.0f) * x1;
+    lx -= (j > 0 ? oym.z : 0.0f) * x2;
+    lx -= (j + 1 < F.ny ? o.z : 0.0f) * x3;
+    lx -= (k > 0 ? ozm.w : 0.0f) * x4;
+    lx -= (k + 1 < F.nz ? o.w : 0.0f) * x5;
     return bc - lx;
 }
 
-__device__ __forceinline__ void mg_down_body(const PcgState &st, const MgLevel &F, const MgLevel &C, int l, int blk) {
+__device__ __forceinline__ void mg_down_body(const PcgState &st, const MgLevel &F, const MgLevel &C, int blk) {
     if (solve_done(st.scal)) return;
     __shared__ float res[kPB];
     const int tz = threadIdx.x % kMgTileZ, ty = (threadIdx.x / kMgTileZ) & 1, tx = threadIdx.x / (2 * kMgTileZ);
     const int tiles_z = (F.nz + kMgTileZ - 1) / kMgTileZ, tiles_y = (F.ny + 1) / 2;
     const int bz = blk % tiles_z, by = (blk / tiles_z) % tiles_y, bx = blk / (tiles_z * tiles_y);
     const int i = 2 * bx + tx, j = 2 * by + ty, k = bz * kMgTileZ + tz;
-    float rc = 0.0f;
-    if (l >= 1) {
-        if (i < F.nx && j < F.ny && k < F.nz) rc = mg_down_cell_coarse(F, i, j, k);
-    } else if (i < F.nx && j < F.ny && k < F.nz) {
-        const size_t c = idx3(i, j, k, F.ny, F.nz);
-        const MgCell a = mg_get(st, F, l, i, j, k);
-        if (a.unknown) {
-            const float bc = mg_b(st, F, l, c);
-            const float xc = kMgOmega * bc / a.d;
-            F.x[c] = xc;
-            float lx = a.d * xc;
-#pragma unroll
-            for (int q = 0; q < 6; ++q) {
-                if (a.w[q] == 0.0f) continue;
-                int ni, nj, nk;
-                mg_neighbour(q, i, j, k, ni, nj, nk);
-                if (ni < 0 || nj < 0 || nk < 0 || ni >= F.nx || nj >= F.ny || nk >= F.nz) continue;
-                const MgCell b = mg_get(st, F, l, ni, nj, nk);
-                if (!b.unknown) continue;
-                lx -= a.w[q] * (kMgOmega * mg_b(st, F, l, idx3(ni, nj, nk, F.ny, F.nz)) / b.d);
-            }
-            rc = bc - lx;
-        } else {
-            F.x[c] = 0.0f;
-        }
-    }
-    res[threadIdx.x] = rc;
+    res[threadIdx.x] = i < F.nx && j < F.ny && k < F.nz ? mg_residual_cell(F, i, j, k) : 0.0f;
     __syncthreads();
     if (threadIdx.x < kMgTileZ / 2) {
         const int az = threadIdx.x;
@@ -1148,18 +1125,21 @@ __device__ __forceinline__ void mg_down_body(const PcgState &st, const MgLevel &
 #pragma unroll
                     for (int cz = 0; cz < 2; ++cz) sum += res[cx * 2 * kMgTileZ + cy * kMgTileZ + 2 * az + cz];
             const size_t ci = idx3(I, J, K, C.ny, C.nz);
-            C.b[ci] = C.op[ci].x > 0.0f ? sum : 0.0f;
+            const float d = C.op[ci].x;
+            C.b[ci] = d > 0.0f ? sum : 0.0f;
+            C.x[ci] = mg_presmooth(sum, d);
         }
     }
 }
-__global__ void __launch_bounds__(kPB) mg_down_kernel(PcgState st, MgLevel F, MgLevel C, int l) {
-    mg_down_body(st, F, C, l, blockIdx.x);
+__global__ void __launch_bounds__(kPB) mg_down_kernel(PcgState st, MgLevel F, MgLevel C) {
+    mg_down_body(st, F, C, blockIdx.x);
 }
 
 // The coarsest level (at most kMgCoarsestCells cells, one per thread): kMgCoarseSweeps damped
-// Jacobi sweeps from zero, in LDS.
-__device__ __forceinline__ void mg_coarsest_body(const PcgState &st, const MgLevel &L) {
-    if (solve_done(st.scal)) return;
+// Jacobi sweeps from zero, in LDS.  Block e runs them on the unit vector of cell e: the sweeps are
+// one linear map of the right-hand side, and its columns, built once per system, serve every cycle
+// (48 sweeps of one block took 17 us a cycle, half of a small grid's coarse levels).
+__global__ void __launch_bounds__(kMgCoarsestCells) mg_dense_kernel(MgLevel L) {
     __shared__ float xs[2][kMgCoarsestCells];
     const int n = L.nx * L.ny * L.nz;
     const int c = threadIdx.x;
@@ -1169,7 +1149,7 @@ __device__ __forceinline__ void mg_coarsest_body(const PcgState &st, const MgLev
     if (c < n) {
         k = c % L.nz; j = (c / L.nz) % L.ny; i = c / (L.ny * L.nz);
         a = mg_cell(L, i, j, k);
-        bc = L.b[c];
+        bc = c == (int)blockIdx.x ? 1.0f : 0.0f;
     }
     xs[0][c] = 0.0f;
     __syncthreads();
@@ -1191,37 +1171,14 @@ __device__ __forceinline__ void mg_coarsest_body(const PcgState &st, const MgLev
         __syncthreads();
         cur ^= 1;
     }
-    if (c < n) L.x[c] = xs[cur][c];
+    if (c < n) L.dense[(size_t)blockIdx.x * n + c] = xs[cur][c];
 }
-__global__ void __launch_bounds__(kPB) mg_coarsest_kernel(PcgState st, MgLevel L) { mg_coarsest_body(st, L); }
 
-// Up the V-cycle at level l: x' = x + the aggregate's correction, then one smoothing sweep
-// x'' = x' + w (b - L x') / d (the neighbours' x' recomputed the same way).
-__device__ __forceinline__ float mg_up_cell(const PcgState &st, const MgLevel &F, const float *corr, int cny, int cnz,
-                                            int l, size_t c, float bc) {
-    const int k = (int)(c % F.nz), j = (int)((c / F.nz) % F.ny), i = (int)(c / ((size_t)F.ny * F.nz));
-    const MgCell a = mg_get(st, F, l, i, j, k);
-    if (!a.unknown) return 0.0f;
-    const float xc = F.x[c] + kMgCorrScale * corr[idx3(i >> 1, j >> 1, k >> 1, cny, cnz)];
-    float lx = a.d * xc;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        if (a.w[q] == 0.0f) continue;
-        int ni, nj, nk;
-        mg_neighbour(q, i, j, k, ni, nj, nk);
-        if (ni < 0 || nj < 0 || nk < 0 || ni >= F.nx || nj >= F.ny || nk >= F.nz) continue;
-        const size_t cn = idx3(ni, nj, nk, F.ny, F.nz);
-        if (!mg_unknown(st, F, l, cn)) continue;
-        lx -= a.w[q] * (F.x[cn] + kMgCorrScale * corr[idx3(ni >> 1, nj >> 1, nk >> 1, cny, cnz)]);
-    }
-    return xc + kMgOmega * (bc - lx) / a.d;
-}
-// The same on a level l >= 1 with every load issued at once (as mg_down_cell_coarse): the
-// operator records for the cell's weights, its x and correction, and each neighbour's record, x
-// and correction from indices clamped into the grid; a neighbour that is outside, not an unknown
-// or joined by a zero weight adds its term times 0 (every value finite).
-__device__ __forceinline__ float mg_up_cell_coarse(const MgLevel &F, const float *corr, int cny, int cnz, int c,
-                                                   float bc) {
+// Up the V-cycle at a level l >= 1: x' = x + the aggregate's correction, then one smoothing sweep
+// x'' = x' + w (b - L x') / d (the neighbours' x' recomputed the same way), with every load issued at
+// once (as mg_residual_cell): a neighbour that is outside has weight 0; one that is not an unknown has
+// no face to this cell, so its weight is 0 too.
+__device__ __forceinline__ float mg_up_cell(const MgLevel &F, const float *corr, int cny, int cnz, int c, float bc) {
     const int k = c % F.nz, j = (c / F.nz) % F.ny, i = c / (F.ny * F.nz);
     const int sx = F.ny * F.nz, sy = F.nz;
     const float4 o = F.op[c];
@@ -1253,18 +1210,145 @@ __device__ __forceinline__ float mg_up_cell_coarse(const MgLevel &F, const float
     }
     return xc + kMgOmega * (bc - lx) / o.x;
 }
-// levels >= 1: one thread per cell, writes xs
+// one thread per cell, writes xs
 __device__ __forceinline__ void mg_up_body(const PcgState &st, const MgLevel &F, const float *corr, int cny, int cnz,
-                                           int l, int blk) {
+                                           int blk) {
     if (solve_done(st.scal)) return;
     const size_t n = (size_t)F.nx * F.ny * F.nz;
     const size_t c = (size_t)blk * kPB + threadIdx.x;
-    if (c < n) F.xs[c] = l >= 1 ? mg_up_cell_coarse(F, corr, cny, cnz, (int)c, F.b[c]) : mg_up_cell(st, F, corr, cny, cnz, l, c, F.b[c]);
+    if (c < n) F.xs[c] = mg_up_cell(F, corr, cny, cnz, (int)c, F.b[c]);
 }
-__global__ void __launch_bounds__(kPB) mg_up_kernel(PcgState st, MgLevel F, const float *corr, int cny, int cnz,
-                                                    int l) {
-    mg_up_body(st, F, corr, cny, cnz, l, blockIdx.x);
+__global__ void __launch_bounds__(kPB) mg_up_kernel(PcgState st, MgLevel F, const float *corr, int cny, int cnz) {
+    mg_up_body(st, F, corr, cny, cnz, blockIdx.x);
 }
+// The V-cycle's tail: its levels from `first` on (mg_tail_level: the smoothed ones hold at most
+// kMgTailCells cells together) in one block, in LDS.  As launches of their own each was 4 us of
+// latency (the coarsest 17), five of them on a 256^3 grid (34 us); one block takes 17 us for all of them.  Each cell's
+// arithmetic is that of the level kernels.
+constexpr int kTailThreads = 1024;
+// cell index -> (i, j, k) in a level of at most kMgTailCells cells, by multiplications (c nz < 2^32)
+struct TailCells {
+    int ny, nz;
+    unsigned my, mz;
+    __device__ __forceinline__ explicit TailCells(const MgLevel &L)
+        : ny(L.ny), nz(L.nz), my(0xffffffffu / (unsigned)L.ny + 1u), mz(0xffffffffu / (unsigned)L.nz + 1u) {}
+    __device__ __forceinline__ void at(int c, int &i, int &j, int &k) const {
+        const int q = nz == 1 ? c : (int)__umulhi((unsigned)c, mz);
+        i = ny == 1 ? q : (int)__umulhi((unsigned)q, my);
+        j = q - i * ny;
+        k = c - q * nz;
+    }
+};
+__device__ __forceinline__ void mg_tail_body(const PcgState &st, const MgLevel *lv, int levels, int first) {
+    __shared__ float4 op[kMgTailCells];
+    __shared__ float b[kMgTailCells], x[kMgTailCells], res[kMgTailCells];
+    __shared__ float cb[kMgCoarsestCells], part[kTailThreads];
+    if (solve_done(st.scal)) return;
+    const int tid = threadIdx.x, last = levels - 1;
+    const MgLevel &B = lv[last];
+    const int nb = B.nx * B.ny * B.nz;
+    int off = 0;
+    for (int l = first; l < last; ++l) {
+        const int n = lv[l].nx * lv[l].ny * lv[l].nz;
+        for (int c = tid; c < n; c += kTailThreads) {
+            op[off + c] = lv[l].op[c];
+            if (l == first) { b[c] = lv[l].b[c]; x[c] = lv[l].x[c]; }
+        }
+        off += n;
+    }
+    if (first == last && tid < nb) cb[tid] = B.b[tid];
+    __syncthreads();
+    off = 0;
+    for (int l = first; l < last; ++l) {
+        MgLevel F = lv[l];
+        const MgLevel &C = lv[l + 1];
+        F.op = op + off; F.b = b + off; F.x = x + off;
+        const int n = F.nx * F.ny * F.nz, nc = C.nx * C.ny * C.nz;
+        const TailCells cells(F), coarse(C);
+        for (int c = tid; c < n; c += kTailThreads) {
+            int i, j, k;
+            cells.at(c, i, j, k);
+            res[c] = mg_residual_cell(F, i, j, k);
+        }
+        __syncthreads();
+        for (int a = tid; a < nc; a += kTailThreads) {
+            int I, J, K;
+            coarse.at(a, I, J, K);
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int i = 2 * I + (e >> 2), j = 2 * J + ((e >> 1) & 1), k = 2 * K + (e & 1);
+                const bool in = i < F.nx && j < F.ny && k < F.nz;
+                const float v = res[(min(i, F.nx - 1) * F.ny + min(j, F.ny - 1)) * F.nz + min(k, F.nz - 1)];
+                sum += in ? v : 0.0f;
+            }
+            if (l + 1 == last) {
+                cb[a] = C.op[a].x > 0.0f ? sum : 0.0f;
+            } else {
+                const float d = op[off + n + a].x;
+                b[off + n + a] = d > 0.0f ? sum : 0.0f;
+                x[off + n + a] = mg_presmooth(sum, d);
+            }
+        }
+        __syncthreads();
+        off += n;
+    }
+    // the coarsest level: its dense map, groups of threads over a share of its columns each
+    const int width = nb <= 64 ? 64 : nb <= 128 ? 128 : 256, groups = kTailThreads / width;
+    {
+        const int c = tid % width, g = tid / width;
+        float sum = 0.0f;
+        if (c < nb) {
+#pragma unroll 4
+            for (int e = g; e < nb; e += groups) sum += B.dense[e * nb + c] * cb[e];
+        }
+        part[tid] = sum;
+    }
+    __syncthreads();
+    if (tid < nb) {
+        float sum = part[tid];
+        for (int g = 1; g < groups; ++g) sum += part[g * width + tid];
+        cb[tid] = sum;
+        if (first == last) B.x[tid] = sum;
+    }
+    __syncthreads();
+    for (int l = last - 1; l >= first; --l) {
+        MgLevel F = lv[l];
+        const MgLevel &C = lv[l + 1];
+        const int n = F.nx * F.ny * F.nz;
+        const float *corr = l + 1 == last ? cb : x + off;
+        off -= n;
+        F.op = op + off; F.b = b + off; F.x = x + off;
+        const TailCells cells(F);
+        // the corrected x of every cell first, then the smoothing sweep into res
+        for (int c = tid; c < n; c += kTailThreads) {
+            int i, j, k;
+            cells.at(c, i, j, k);
+            if (F.op[c].x > 0.0f) x[off + c] = x[off + c] + kMgCorrScale * corr[((i >> 1) * C.ny + (j >> 1)) * C.nz + (k >> 1)];
+        }
+        __syncthreads();
+        for (int c = tid; c < n; c += kTailThreads) {
+            int i, j, k;
+            cells.at(c, i, j, k);
+            const float d = F.op[c].x;
+            const float v = d > 0.0f ? x[off + c] + kMgOmega * mg_residual_cell(F, i, j, k) / d : 0.0f;
+            if (l == first) lv[l].xs[c] = v;
+            else res[c] = v;
+        }
+        if (l == first) break;
+        __syncthreads();
+        for (int c = tid; c < n; c += kTailThreads) x[off + c] = res[c];
+        __syncthreads();
+    }
+}
+__global__ void __launch_bounds__(kTailThreads) mg_tail_kernel(PcgState st, MgHier h, int first) {
+    mg_tail_body(st, h.lv, h.levels, first);
+}
+__global__ void __launch_bounds__(kTailThreads) mg_tail_batch_kernel(const PcgState *__restrict__ sts) {
+    const PcgState &st = sts[blockIdx.x];
+    mg_tail_body(st, st.mg_lv, st.mg_levels, st.mg_tail);
+}
+
 // Level 0 of the V-cycle on the solve's tiles (tile_sweep: the 2.5-D sweep of the CG kernels).
 // Down: v = x = w r / d (the first smoothing sweep from zero), stored, and the residual r - L x
 // into the level's residual buffer (b), summed over the 2 x 2 x 2 aggregates by
@@ -1323,11 +1407,11 @@ struct MgUp0Op {
         return (a.f & kPcgUnknown) ? (double)(a.x + kMgCorrScale * a.corr) : 0.0;
     }
     __device__ __forceinline__ void cell(size_t c, const Raw &a, double v, double q, double *acc) const {
-        double zc = 0.0;
+        float zc = 0.0f;
         if (a.f & kPcgUnknown)
-            zc = (double)((float)v + kMgOmega * (float)(a.r - q) / (float)__builtin_popcount(a.f & 63u));
+            zc = (float)v + kMgOmega * (float)(a.r - q) / (float)__builtin_popcount(a.f & 63u);
         st.z[c] = zc;
-        acc[0] += a.r * zc;
+        acc[0] += a.r * (double)zc;
     }
 };
 __device__ __forceinline__ void mg_down0_body(const PcgState &st, float *x, float *res, int blk) {
@@ -1338,7 +1422,7 @@ __device__ __forceinline__ void mg_down0_body(const PcgState &st, float *x, floa
 __global__ void __launch_bounds__(kPB) mg_down0_kernel(PcgState st, float *x, float *res) {
     mg_down0_body(st, x, res, blockIdx.x);
 }
-// b of level 1: the sum of each aggregate's children's residuals (fixed order)
+// b of level 1, the sum of each aggregate's children's residuals (fixed order), and its pre-smoothed x
 __device__ __forceinline__ void mg_restrict0_body(const PcgState &st, const MgLevel &F, const MgLevel &C, int blk) {
     if (solve_done(st.scal)) return;
     const size_t n = (size_t)C.nx * C.ny * C.nz;
@@ -1357,7 +1441,9 @@ __device__ __forceinline__ void mg_restrict0_body(const PcgState &st, const MgLe
     float sum = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) sum += v[e] * m[e];
-    C.b[I] = C.op[I].x > 0.0f ? sum : 0.0f;
+    const float d = C.op[I].x;
+    C.b[I] = d > 0.0f ? sum : 0.0f;
+    C.x[I] = mg_presmooth(sum, d);
 }
 __global__ void __launch_bounds__(kPB) mg_restrict0_kernel(PcgState st, MgLevel F, MgLevel C) {
     mg_restrict0_body(st, F, C, blockIdx.x);
@@ -1393,18 +1479,14 @@ __global__ void __launch_bounds__(kPB) mg_down_batch_kernel(const PcgState *__re
                                                             const int2 *__restrict__ map, int l) {
     const int2 m = map[blockIdx.x];
     const PcgState &st = sts[m.x];
-    mg_down_body(st, st.mg_lv[l], st.mg_lv[l + 1], l, m.y);
-}
-__global__ void __launch_bounds__(kPB) mg_coarsest_batch_kernel(const PcgState *__restrict__ sts) {
-    const PcgState &st = sts[blockIdx.x];
-    mg_coarsest_body(st, st.mg_lv[st.mg_levels - 1]);
+    mg_down_body(st, st.mg_lv[l], st.mg_lv[l + 1], m.y);
 }
 __global__ void __launch_bounds__(kPB) mg_up_batch_kernel(const PcgState *__restrict__ sts,
                                                           const int2 *__restrict__ map, int l) {
     const int2 m = map[blockIdx.x];
     const PcgState &st = sts[m.x];
     const MgLevel &C = st.mg_lv[l + 1];
-    mg_up_body(st, st.mg_lv[l], l + 1 == st.mg_levels - 1 ? C.x : C.xs, C.ny, C.nz, l, m.y);
+    mg_up_body(st, st.mg_lv[l], l + 1 == st.mg_levels - 1 ? C.x : C.xs, C.ny, C.nz, m.y);
 }
 __global__ void __launch_bounds__(kPB) mg_up0_batch_kernel(const PcgState *__restrict__ sts,
                                                            const int2 *__restrict__ map) {
@@ -1418,8 +1500,8 @@ __global__ void __launch_bounds__(kPB) mg_up0_batch_kernel(const PcgState *__res
 __global__ void __launch_bounds__(kPB) pcg_start_kernel(PcgState st, double tol2) {
     pcg_start_body(st, blockIdx.x, tol2);
 }
-__global__ void __launch_bounds__(kPB) pcg_direction_kernel(PcgState st, int k) {
-    pcg_direction_body(st, blockIdx.x, k);
+template <bool MG> __global__ void __launch_bounds__(kPB) pcg_direction_kernel(PcgState st, int k) {
+    pcg_direction_body<MG>(st, blockIdx.x, k);
 }
 template <bool RECOMPUTE> __global__ void __launch_bounds__(kPB) pcg_update_kernel(PcgState st, int k) {
     pcg_update_body<RECOMPUTE>(st, blockIdx.x, k);
@@ -1445,10 +1527,11 @@ __global__ void __launch_bounds__(kPB) pcg_fused_flush_kernel(PcgState st) {
 
 // ... or many solves per launch, all at the same iteration: map[b] = (s, j) says that block b of
 // the launch is block j of solve s, so each solve's arithmetic is exactly that of its own launch.
+template <bool MG>
 __global__ void __launch_bounds__(kPB) pcg_direction_batch_kernel(const PcgState *__restrict__ st,
                                                                   const int2 *__restrict__ map, int k) {
     const int2 m = map[blockIdx.x];
-    pcg_direction_body(st[m.x], m.y, k);
+    pcg_direction_body<MG>(st[m.x], m.y, k);
 }
 template <bool RECOMPUTE>
 __global__ void __launch_bounds__(kPB) pcg_update_batch_kernel(const PcgState *__restrict__ st,
@@ -1495,7 +1578,7 @@ int pcg_resident_blocks(bool fused) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, pcg_fused_kernel<true>, kPB, 0) != hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, pcg_fused_kernel<false>, kPB, 0) != hipSuccess)
             return 0;
-    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, pcg_direction_kernel, kPB, 0) != hipSuccess ||
+    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, pcg_direction_kernel<false>, kPB, 0) != hipSuccess ||
                hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, pcg_update_kernel<true>, kPB, 0) != hipSuccess) {
         return 0;
     }
@@ -1596,7 +1679,8 @@ hipError_t launch_pcg_iterations(PcgState &st, int count, hipStream_t s, const M
         return hipGetLastError();
     }
     for (int k = 0; k < count; ++k) {
-        hipLaunchKernelGGL(pcg_direction_kernel, dim3(st.dir_blocks), dim3(kPB), 0, s, st, st.it);
+        if (st.z) hipLaunchKernelGGL(pcg_direction_kernel<true>, dim3(st.dir_blocks), dim3(kPB), 0, s, st, st.it);
+        else hipLaunchKernelGGL(pcg_direction_kernel<false>, dim3(st.dir_blocks), dim3(kPB), 0, s, st, st.it);
         if (st.recompute_q) hipLaunchKernelGGL(pcg_update_kernel<true>, dim3(st.upd_blocks), dim3(kPB), 0, s, st, st.it);
         else hipLaunchKernelGGL(pcg_update_kernel<false>, dim3(st.upd_blocks), dim3(kPB), 0, s, st, st.it);
         if (mg) {
@@ -1619,7 +1703,12 @@ hipError_t launch_pcg_check(const PcgState &st, hipStream_t s) {
 hipError_t launch_pcg_batch_iterations(PcgBatch &b, int count, hipStream_t s, const MgBatch *mb) {
     if (b.n == 0) return hipSuccess;
     for (int k = 0; k < count; ++k) {
-        hipLaunchKernelGGL(pcg_direction_batch_kernel, dim3(b.dir_blocks), dim3(kPB), 0, s, b.states, b.dir_map, b.it);
+        if (mb)
+            hipLaunchKernelGGL(pcg_direction_batch_kernel<true>, dim3(b.dir_blocks), dim3(kPB), 0, s, b.states, b.dir_map,
+                               b.it);
+        else
+            hipLaunchKernelGGL(pcg_direction_batch_kernel<false>, dim3(b.dir_blocks), dim3(kPB), 0, s, b.states, b.dir_map,
+                               b.it);
         if (b.stream_blocks)
             hipLaunchKernelGGL(pcg_update_batch_kernel<false>, dim3(b.stream_blocks), dim3(kPB), 0, s, b.states,
                                b.stream_map, b.it);
@@ -1651,13 +1740,15 @@ static bool same_launch(const PcgState &a, const PcgState &b) {
            a.nblocks == b.nblocks && a.dir_blocks == b.dir_blocks &&
            a.dir_tiles_y == b.dir_tiles_y && a.dir_tiles_z == b.dir_tiles_z && a.dir_chunk_x == b.dir_chunk_x &&
            a.dir_chunks == b.dir_chunks && a.recompute_q == b.recompute_q && a.upd_blocks == b.upd_blocks &&
-           a.z == b.z && a.part_mg == b.part_mg && a.mg_lv == b.mg_lv && a.mg_levels == b.mg_levels;
+           a.z == b.z && a.part_mg == b.part_mg && a.mg_lv == b.mg_lv && a.mg_levels == b.mg_levels &&
+           a.mg_tail == b.mg_tail;
 }
 static bool same_launch(const MgHier &a, const MgHier &b) {
     if (a.levels != b.levels) return false;
     for (int l = 0; l < a.levels; ++l) {
         const MgLevel &x = a.lv[l], &y = b.lv[l];
-        if (x.nx != y.nx || x.ny != y.ny || x.nz != y.nz || x.op != y.op || x.b != y.b || x.x != y.x || x.xs != y.xs)
+        if (x.nx != y.nx || x.ny != y.ny || x.nz != y.nz || x.op != y.op || x.b != y.b || x.x != y.x || x.xs != y.xs ||
+            x.dense != y.dense)
             return false;
     }
     return true;
@@ -1774,16 +1865,29 @@ void mg_shape(int nx, int ny, int nz, MgHier &h) {
     while (h.levels < kMgMaxLevels) {
         MgLevel &L = h.lv[h.levels++];
         L.nx = x; L.ny = y; L.nz = z;
-        L.op = nullptr; L.b = nullptr; L.x = nullptr; L.xs = nullptr;
+        L.op = nullptr; L.b = nullptr; L.x = nullptr; L.xs = nullptr; L.dense = nullptr;
         if (h.levels >= 2 && (size_t)x * y * z <= (size_t)kMgCoarsestCells) break;
         x = (x + 1) / 2; y = (y + 1) / 2; z = (z + 1) / 2;
     }
+}
+int mg_tail_level(const MgHier &h) {
+    int first = h.levels - 1;
+    size_t cells = 0;
+    while (first > 1) {
+        const MgLevel &L = h.lv[first - 1];
+        cells += (size_t)L.nx * L.ny * L.nz;
+        if (cells > (size_t)kMgTailCells) break;
+        --first;
+    }
+    return first;
 }
 hipError_t launch_mg_build(const PcgState &st, const MgHier &h, hipStream_t s) {
     for (int l = 0; l + 1 < h.levels; ++l) {
         const size_t n = (size_t)h.lv[l + 1].nx * h.lv[l + 1].ny * h.lv[l + 1].nz;
         hipLaunchKernelGGL(mg_build_kernel, dim3(blocks(n)), dim3(kPB), 0, s, st, h.lv[l], h.lv[l + 1], l);
     }
+    const MgLevel &B = h.lv[h.levels - 1];
+    hipLaunchKernelGGL(mg_dense_kernel, dim3(B.nx * B.ny * B.nz), dim3(kMgCoarsestCells), 0, s, B);
     return hipGetLastError();
 }
 hipError_t launch_mg_vcycle(const PcgState &st, const MgHier &h, hipStream_t s) {
@@ -1793,12 +1897,13 @@ hipError_t launch_mg_vcycle(const PcgState &st, const MgHier &h, hipStream_t s) 
         const size_t n1 = (size_t)h.lv[1].nx * h.lv[1].ny * h.lv[1].nz;
         hipLaunchKernelGGL(mg_restrict0_kernel, dim3(blocks(n1)), dim3(kPB), 0, s, st, h.lv[0], h.lv[1]);
     }
-    for (int l = 1; l + 1 < L; ++l) {
+    const int first = mg_tail_level(h);
+    for (int l = 1; l < first; ++l) {
         const MgLevel &F = h.lv[l];
-        hipLaunchKernelGGL(mg_down_kernel, dim3((unsigned)mg_down_tiles(F)), dim3(kPB), 0, s, st, F, h.lv[l + 1], l);
+        hipLaunchKernelGGL(mg_down_kernel, dim3((unsigned)mg_down_tiles(F)), dim3(kPB), 0, s, st, F, h.lv[l + 1]);
     }
-    hipLaunchKernelGGL(mg_coarsest_kernel, dim3(1), dim3(kPB), 0, s, st, h.lv[L - 1]);
-    for (int l = L - 2; l >= 0; --l) {
+    hipLaunchKernelGGL(mg_tail_kernel, dim3(1), dim3(kTailThreads), 0, s, st, h, first);
+    for (int l = first - 1; l >= 0; --l) {
         const MgLevel &C = h.lv[l + 1];
         const float *corr = l + 1 == L - 1 ? C.x : C.xs;
         if (l == 0) {
@@ -1806,7 +1911,7 @@ hipError_t launch_mg_vcycle(const PcgState &st, const MgHier &h, hipStream_t s) 
                                C.nz);
         } else {
             const size_t n = (size_t)h.lv[l].nx * h.lv[l].ny * h.lv[l].nz;
-            hipLaunchKernelGGL(mg_up_kernel, dim3(blocks(n)), dim3(kPB), 0, s, st, h.lv[l], corr, C.ny, C.nz, l);
+            hipLaunchKernelGGL(mg_up_kernel, dim3(blocks(n)), dim3(kPB), 0, s, st, h.lv[l], corr, C.ny, C.nz);
         }
     }
     return hipGetLastError();
@@ -1818,7 +1923,7 @@ hipError_t launch_mg_batch_vcycle(const PcgBatch &b, const MgBatch &mb, hipStrea
     for (int l = 1; l < kMgMaxLevels; ++l)
         if (mb.down_blocks[l])
             hipLaunchKernelGGL(mg_down_batch_kernel, dim3(mb.down_blocks[l]), dim3(kPB), 0, s, b.states, mb.down_map[l], l);
-    hipLaunchKernelGGL(mg_coarsest_batch_kernel, dim3(b.n), dim3(kPB), 0, s, b.states);
+    hipLaunchKernelGGL(mg_tail_batch_kernel, dim3(b.n), dim3(kTailThreads), 0, s, b.states);
     for (int l = kMgMaxLevels - 1; l >= 1; --l)
         if (mb.up_blocks[l])
             hipLaunchKernelGGL(mg_up_batch_kernel, dim3(mb.up_blocks[l]), dim3(kPB), 0, s, b.states, mb.up_map[l], l);
@@ -1829,6 +1934,10 @@ hipError_t launch_project(const PcgGrid &g, const double *p, double h, float *u,
                           float *pressure_out, hipStream_t s) {
     const size_t n = (size_t)g.nx * g.ny * g.nz;
     hipLaunchKernelGGL(project_kernel, dim3(blocks(n)), dim3(kPB), 0, s, g, p, h, u, v, w, pressure_out);
+    return hipGetLastError();
+}
+hipError_t launch_last_fluid(const uint8_t *solid, size_t n, long long *out, hipStream_t s) {
+    hipLaunchKernelGGL(last_fluid_kernel, dim3(1), dim3(kLastThreads), 0, s, solid, (long)n, out);
     return hipGetLastError();
 }
 hipError_t launch_zero_solid_faces(const PcgGrid &g, float *u, float *v, float *w, hipStream_t s) {
