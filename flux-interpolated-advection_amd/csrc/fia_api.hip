@@ -285,10 +285,12 @@ __global__ void zero_ints_kernel(int *a, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = 0;
 }
-// the face lists' counts (counters[1], the first error, stays)
-__global__ void zero_lists_kernel(int *counters) {
-    if (threadIdx.x == 0) counters[0] = 0;
-    if (threadIdx.x == 2) counters[2] = 0;
+// the face lists' counts (counters[1], the first error, stays) and the scan's tile sums
+__global__ void zero_lists_kernel(int *counters, unsigned long long *sums, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) counters[0] = 0;
+    if (i == 2) counters[2] = 0;
+    if (i < n) sums[i] = 0;
 }
 __global__ void zero_uints_kernel(unsigned int *a, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -369,8 +371,6 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     }
     HIP_TRY(c->twisted.ensure(g.faces(0) + g.faces(1) + g.faces(2)));
     HIP_TRY(c->degen.ensure(g.faces(0) + g.faces(1) + g.faces(2)));
-    hipLaunchKernelGGL(zero_lists_kernel, dim3(1), dim3(64), 0, c->stream, c->counters.p);
-    HIP_TRY(hipGetLastError());
     FaceParams p;
     memset(&p, 0, sizeof(p));
     p.g = g; p.q = q; p.psi = c->psi.p;
@@ -419,7 +419,11 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     p.fam_base[0] = 0; p.fam_base[1] = g.faces(0); p.fam_base[2] = g.faces(0) + g.faces(1);
     int sp;
     HIP_TRY(span_begin(c, SK_FACE, sp));
-    HIP_TRY(launch_face_count(p, c->stream));   // all families; inactive ones count zero
+    const int tiles = (int)scan_temp_words(nf);
+    hipLaunchKernelGGL(zero_lists_kernel, dim3((unsigned)((tiles + 255) / 256)), dim3(256), 0, c->stream, c->counters.p,
+                       c->scan_tmp.p, tiles);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(launch_face_count(p, c->scan_tmp.p, c->stream));   // all families; inactive ones count zero
     // the slot bounds of the families and the list lengths, which size the launches below, straight
     // into pinned host memory
     HIP_TRY(launch_scan(c->scan_tmp.p, c->face_n.p, c->face_start.p, nf, p, c->host_bounds, c->stream));

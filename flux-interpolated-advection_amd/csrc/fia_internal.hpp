@@ -169,7 +169,8 @@ enum KernelError {
 
 hipError_t launch_psi(const PsiParams &p, hipStream_t s);
 hipError_t launch_vertices(const VertexParams &p, hipStream_t s);
-hipError_t launch_face_count(const FaceParams &p, hipStream_t s);
+// slot counts of every face, added up by tile of the scan in tile_sum (scan_temp_words, zero before)
+hipError_t launch_face_count(const FaceParams &p, unsigned long long *tile_sum, hipStream_t s);
 // segment cutter: the face kernels of the three families (pieces into the slots of the scan)
 hipError_t launch_seg_faces(const FaceParams &p, hipStream_t s);
 // 1 or 2: the WENO6 integral quadrature with that many Gauss points per half (piece_kernel<1|2>);
@@ -182,9 +183,9 @@ hipError_t launch_weno_tables(const FaceParams &p, WenoHalf *q_tab, WenoHalf *ps
 hipError_t launch_face_sum(const FaceParams &p, hipStream_t s);
 // exclusive scan of the slot counts in (n faces) into out; bounds[1], bounds[2] = first slots of
 // families 1 and 2 (at p.fam_base), bounds[3] = total, bounds[4] = twisted and bounds[5] = degenerate
-// faces (host memory: the kernel stores them there itself); tile_tmp holds scan_temp_words(n) words
+// faces (host memory: the kernel stores them there itself); tile_sum: launch_face_count's
 size_t scan_temp_words(size_t n);
-hipError_t launch_scan(unsigned long long *tile_tmp, const unsigned *in, unsigned long long *out, size_t n,
+hipError_t launch_scan(unsigned long long *tile_sum, const unsigned *in, unsigned long long *out, size_t n,
                        const FaceParams &p, unsigned long long *bounds, hipStream_t s);
 // the twisted faces' pieces: count per face and orientation, and their scan (p.gen_n, p.gen_start;
 // gen_start[2 count] = the total), then with the piece records sized from that total: the pieces

@@ -5,8 +5,9 @@
 //                     column's y range in eight segments (one wave each), FP64 sums
 //                     (psi_weno_held_kernel: the WENO6 integral rule with the segment held)
 //   vertex_kernel     backtraced displacement of every lattice vertex, one thread per vertex
-//   face_count_kernel slots of every face (x strips x z bands); twisted and degenerate faces listed
-//   scan_*            exclusive scan of the slot counts (three kernels over tiles)
+//   face_count_kernel slots of every face (x strips x z bands) and their sums by tile of the scan;
+//                     twisted and degenerate faces listed
+//   scan_*            exclusive scan of the slot counts
 //   seg_face_kernel   boundary-segment cutter, one thread per face (multi-cut faces piece by piece)
 //   degenerate_kernel clipping pipeline for faces with a corner colour on an interior integer
 //   zero_velocity_face_kernel  the zero-velocity correction pass: the undeformed y faces' pieces
@@ -749,7 +750,7 @@ template <int FAM> FIA_HD bool seg_one_pass(int nxc, int nzc) {
 // ones, or all when minimal_area < 1) are queued and get no slots; a non-finite face reports an
 // error and gets none (zero flux).  Degenerate faces keep their slots and are queued for the
 // clipping pipeline (degenerate_kernel).
-template <int FAM> FIA_HD void face_count_body(const FaceParams &P, long id) {
+template <int FAM> FIA_HD unsigned face_count_body(const FaceParams &P, long id) {
     unsigned n = 0;
     if (P.fam_mask & (1 << FAM)) {
         int i, j, k;
@@ -767,13 +768,52 @@ template <int FAM> FIA_HD void face_count_body(const FaceParams &P, long id) {
         }
     }
     P.face_n[P.fam_base[FAM] + id] = n;
-}
-template <int FAM> __global__ void __launch_bounds__(kBlock) face_count_kernel(FaceParams P) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (long)P.g.faces(FAM)) return;
-    face_count_body<FAM>(P, id);
+    return n;
 }
 
+// The family kernels run as one launch over the three families' blocks in turn: on small grids a
+// launch is several us long whatever its size.  Block blk of the launch -> family, block in it.
+FIA_HD int family_block(const CompGrid &g, unsigned threads, unsigned blk, unsigned &in) {
+    in = blk;
+    for (int f = 0; f < 2; ++f) {
+        const unsigned n = (unsigned)((g.faces(f) + threads - 1) / threads);
+        if (in < n) return f;
+        in -= n;
+    }
+    return 2;
+}
+
+constexpr int kScanItems = 16;
+constexpr int kScanTile = kBlock * kScanItems;
+
+// Adds the wave's slot counts (consecutive faces, n of face gid per lane) to the sums of the scan's
+// tiles, which a wave's faces straddle at most once.
+__device__ __forceinline__ void add_tile_sums(unsigned long long *tile_sum, size_t gid, unsigned n) {
+    const unsigned tile = (unsigned)(gid / kScanTile), t0 = __shfl(tile, 0, 64);
+    unsigned long long a = tile == t0 ? n : 0u, b = tile == t0 ? 0u : n;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_down(a, off, 64);
+        b += __shfl_down(b, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        if (a) atomicAdd(tile_sum + t0, a);
+        if (b) atomicAdd(tile_sum + t0 + 1, b);
+    }
+}
+template <int FAM, bool SUMS>
+__device__ __forceinline__ void face_count_block(const FaceParams &P, unsigned blk, unsigned long long *tile_sum) {
+    const long id = (long)blk * blockDim.x + threadIdx.x;
+    const unsigned n = id < (long)P.g.faces(FAM) ? face_count_body<FAM>(P, id) : 0u;
+    if constexpr (SUMS) add_tile_sums(tile_sum, P.fam_base[FAM] + (size_t)id, n);
+}
+template <bool SUMS> __global__ void __launch_bounds__(kBlock) face_count_kernel(FaceParams P, unsigned long long *tile_sum) {
+    unsigned blk;
+    const int fam = family_block(P.g, blockDim.x, blockIdx.x, blk);
+    if (fam == 0) face_count_block<0, SUMS>(P, blk, tile_sum);
+    else if (fam == 1) face_count_block<1, SUMS>(P, blk, tile_sum);
+    else face_count_block<2, SUMS>(P, blk, tile_sum);
+}
 
 // Value of a piece under the non-integral rule with linear or 1Dy_linear psi: piece_flux's
 // non-integral branch for those two methods, each with its method fixed at compile time.
@@ -867,14 +907,17 @@ template <int FAM> FIA_HD void seg_piece_body(const FaceParams &P, long id, unsi
 // x and z faces (one cut direction each) fit 128 VGPRs, four waves per SIMD, with one spilled value
 // in the piece-by-piece phase (1.03 -> 0.86 ms per launch at 256^3); the y faces (two cut
 // directions) need 160 and keep three waves (bound to 128 they spill 126 values)
-template <int FAM>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FAM == 1 ? 1 : 4))) seg_face_kernel(FaceParams P) {
-    __shared__ unsigned s_face[kBlock];   // the block's faces cut piece by piece (index in the family)
-    __shared__ unsigned s_end[kBlock];    // their slot counts, then the inclusive prefix of them
-    __shared__ int s_count;
+struct SegShared {
+    unsigned face[kBlock];   // the block's faces cut piece by piece (index in the family)
+    unsigned end[kBlock];    // their slot counts, then the inclusive prefix of them
+    int count;
+};
+template <int FAM> __device__ __forceinline__ void seg_face_block(const FaceParams &P, unsigned blk, SegShared &sh) {
+    unsigned *s_face = sh.face, *s_end = sh.end;
+    int &s_count = sh.count;
     if (threadIdx.x == 0) s_count = 0;
     __syncthreads();
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blk * blockDim.x + threadIdx.x;
     if (id < (long)P.g.faces(FAM)) {
         const unsigned n = seg_face_body<FAM>(P, id);
         if (n != 0) {
@@ -901,6 +944,20 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FAM
         }
         seg_piece_body<FAM>(P, (long)s_face[lo], p - (lo > 0 ? s_end[lo - 1] : 0u));
     }
+}
+template <int FAM>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FAM == 1 ? 1 : 4))) seg_face_kernel(FaceParams P) {
+    __shared__ SegShared sh;
+    seg_face_block<FAM>(P, blockIdx.x, sh);
+}
+// the three families in one launch, at the y faces' registers (the families not computed hold no slots)
+__global__ void __launch_bounds__(kBlock) seg_faces_kernel(FaceParams P) {
+    __shared__ SegShared sh;
+    unsigned blk;
+    const int fam = family_block(P.g, blockDim.x, blockIdx.x, blk);
+    if (fam == 0) seg_face_block<0>(P, blk, sh);
+    else if (fam == 1) seg_face_block<1>(P, blk, sh);
+    else seg_face_block<2>(P, blk, sh);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1241,10 +1298,14 @@ template <int FAM> FIA_HD void face_sum_body(const FaceParams &P, long id) {
     for (unsigned q = 0; q < n; ++q) f += P.piece_val[s0 + q];
     P.flux[FAM][id] = f;
 }
-template <int FAM> __global__ void __launch_bounds__(kBlock) face_sum_kernel(FaceParams P) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (long)P.g.faces(FAM)) return;
-    face_sum_body<FAM>(P, id);
+__global__ void __launch_bounds__(kBlock) face_sum_kernel(FaceParams P) {
+    unsigned blk;
+    const int fam = family_block(P.g, blockDim.x, blockIdx.x, blk);
+    const long id = (long)blk * blockDim.x + threadIdx.x;
+    if (!(P.fam_mask & (1 << fam)) || id >= (long)P.g.faces(fam)) return;
+    if (fam == 0) face_sum_body<0>(P, id);
+    else if (fam == 1) face_sum_body<1>(P, id);
+    else face_sum_body<2>(P, id);
 }
 
 // Degenerate faces of the segment-cutter mode (a corner colour exactly on an interior integer):
@@ -1704,12 +1765,77 @@ hipError_t launch_vertices(const VertexParams &p, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_face_count(const FaceParams &p, hipStream_t s) {
+// Grids under this many faces are bound by launches: the cutters of the three families run as one
+// launch, at the y faces' 157 registers, and the count kernel adds up the scan's tile sums with
+// atomics instead of a kernel that reads the counts (density step, merged and separate: 16^3 335 and
+// 430 us, 32^3 328 and 388, 64^3 651 and 702, 80^3 938 and 962, 96^3 1,379 and 1,357, 256^3 21.3 and
+// 19.8 ms).
+constexpr size_t kMergeFaces = (size_t)1 << 21;
+
+// block-wide exclusive scan of one value per thread (kBlock threads, 64-wide waves); total out
+__device__ __forceinline__ unsigned long long block_exclusive_scan(unsigned long long x, unsigned long long &total) {
+    __shared__ unsigned long long wsum[kBlock / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long incl = x;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned long long y = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += y;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    unsigned long long before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) {
+        if (w < wave) before += wsum[w];
+        all += wsum[w];
+    }
+    __syncthreads();   // wsum may be reused by the caller's next scan
+    total = all;
+    return before + incl - x;
+}
+
+__global__ void __launch_bounds__(kBlock) scan_tile_sums_kernel(const unsigned *in, size_t n,
+                                                                unsigned long long *tile_sum) {
+    // the tile read striped over the block (coalesced); the sum does not depend on the order
+    const size_t tile0 = (size_t)blockIdx.x * kScanTile;
+    unsigned long long s = 0;
+    if (tile0 + kScanTile <= n) {
+        // a full tile (all but the last): no bounds tests, so the loads are issued together (a
+        // load under a test is compiled into a branch and waited for at once)
+        unsigned v[kScanItems];
+#pragma unroll
+        for (int i = 0; i < kScanItems; ++i) v[i] = in[tile0 + (size_t)i * kBlock + threadIdx.x];
+#pragma unroll
+        for (int i = 0; i < kScanItems; ++i) s += v[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < kScanItems; ++i) {
+            const size_t k = tile0 + (size_t)i * kBlock + threadIdx.x;
+            if (k < n) s += in[k];
+        }
+    }
+    unsigned long long total;
+    (void)block_exclusive_scan(s, total);
+    if (threadIdx.x == 0) tile_sum[blockIdx.x] = total;
+}
+
+static unsigned family_blocks(const CompGrid &g, int threads) {
+    return grid_for(g.faces(0), threads) + grid_for(g.faces(1), threads) + grid_for(g.faces(2), threads);
+}
+
+hipError_t launch_face_count(const FaceParams &p, unsigned long long *tile_sum, hipStream_t s) {
     // every family writes its entries so the scan sees no stale counts
     const int b = block_or_default(p.face_block);
-    hipLaunchKernelGGL(face_count_kernel<0>, dim3(grid_for(p.g.faces(0), b)), dim3(b), 0, s, p);
-    hipLaunchKernelGGL(face_count_kernel<1>, dim3(grid_for(p.g.faces(1), b)), dim3(b), 0, s, p);
-    hipLaunchKernelGGL(face_count_kernel<2>, dim3(grid_for(p.g.faces(2), b)), dim3(b), 0, s, p);
+    const dim3 grid(family_blocks(p.g, b));
+    const size_t nf = p.g.faces(0) + p.g.faces(1) + p.g.faces(2);
+    if (nf < kMergeFaces) {
+        hipLaunchKernelGGL(face_count_kernel<true>, grid, dim3(b), 0, s, p, tile_sum);
+    } else {
+        hipLaunchKernelGGL(face_count_kernel<false>, grid, dim3(b), 0, s, p, tile_sum);
+        hipLaunchKernelGGL(scan_tile_sums_kernel, dim3((unsigned)scan_temp_words(nf)), dim3(kBlock), 0, s,
+                           (const unsigned *)p.face_n, nf, tile_sum);
+    }
     return hipGetLastError();
 }
 
@@ -1774,68 +1900,18 @@ hipError_t launch_pieces(const FaceParams &p, unsigned long long nslots, hipStre
 
 hipError_t launch_face_sum(const FaceParams &p, hipStream_t s) {
     const int b = block_or_default(p.face_block);
-    if (p.fam_mask & 1) hipLaunchKernelGGL(face_sum_kernel<0>, dim3(grid_for(p.g.faces(0), b)), dim3(b), 0, s, p);
-    if (p.fam_mask & 2) hipLaunchKernelGGL(face_sum_kernel<1>, dim3(grid_for(p.g.faces(1), b)), dim3(b), 0, s, p);
-    if (p.fam_mask & 4) hipLaunchKernelGGL(face_sum_kernel<2>, dim3(grid_for(p.g.faces(2), b)), dim3(b), 0, s, p);
+    hipLaunchKernelGGL(face_sum_kernel, dim3(family_blocks(p.g, b)), dim3(b), 0, s, p);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------------------------
-// Exclusive scan of the per-face slot counts into 64-bit starts.  Three plain kernels over tiles
-// of kScanTile counts: tile sums, one block scanning the tile sums, then each tile scanned in
-// LDS and offset.  No block waits on another block's progress.  The last kernel also writes the
-// slot bounds of the three families (bounds[f] = start of family f, bounds[3] = total).
+// Exclusive scan of the per-face slot counts into 64-bit starts, over tiles of kScanTile counts whose
+// sums launch_face_count left: each tile is scanned in LDS from the sum of the tiles before it,
+// which its block adds up itself on grids of at most kScanDirect tiles, or one block has scanned for
+// all.  No block waits on another block's progress.  The last tile also writes the slot bounds of the
+// three families (bounds[f] = start of family f, bounds[3] = total) and the list lengths.
 // ---------------------------------------------------------------------------------------------
-constexpr int kScanItems = 16;
-constexpr int kScanTile = kBlock * kScanItems;
-
-// block-wide exclusive scan of one value per thread (kBlock threads, 64-wide waves); total out
-__device__ __forceinline__ unsigned long long block_exclusive_scan(unsigned long long x, unsigned long long &total) {
-    __shared__ unsigned long long wsum[kBlock / 64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned long long incl = x;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned long long y = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += y;
-    }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    unsigned long long before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) {
-        if (w < wave) before += wsum[w];
-        all += wsum[w];
-    }
-    __syncthreads();   // wsum may be reused by the caller's next scan
-    total = all;
-    return before + incl - x;
-}
-
-__global__ void __launch_bounds__(kBlock) scan_tile_sums_kernel(const unsigned *in, size_t n,
-                                                                unsigned long long *tile_sum) {
-    // the tile read striped over the block (coalesced); the sum does not depend on the order
-    const size_t tile0 = (size_t)blockIdx.x * kScanTile;
-    unsigned long long s = 0;
-    if (tile0 + kScanTile <= n) {
-        // a full tile (all but the last): no bounds tests, so the loads are issued together (a
-        // load under a test is compiled into a branch and waited for at once)
-        unsigned v[kScanItems];
-#pragma unroll
-        for (int i = 0; i < kScanItems; ++i) v[i] = in[tile0 + (size_t)i * kBlock + threadIdx.x];
-#pragma unroll
-        for (int i = 0; i < kScanItems; ++i) s += v[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < kScanItems; ++i) {
-            const size_t k = tile0 + (size_t)i * kBlock + threadIdx.x;
-            if (k < n) s += in[k];
-        }
-    }
-    unsigned long long total;
-    (void)block_exclusive_scan(s, total);
-    if (threadIdx.x == 0) tile_sum[blockIdx.x] = total;
-}
+constexpr size_t kScanDirect = 2048;   // 2,048 sums are 8 loads a thread, less than a launch
 
 // one block: tile_sum[0..ntiles) -> exclusive prefix in place
 __global__ void __launch_bounds__(kBlock) scan_tile_offsets_kernel(unsigned long long *tile_sum, int ntiles) {
@@ -1879,6 +1955,8 @@ __device__ __forceinline__ int scan_pad(int e) { return e + e / kScanItems; }
 
 // Each tile is loaded striped over the block (coalesced), transposed in LDS so that every thread
 // scans kScanItems consecutive counts, and its starts stored striped again.
+// DIRECT: tile_off holds the tiles' sums, else their exclusive prefix.
+template <bool DIRECT>
 __global__ void __launch_bounds__(kBlock) scan_tiles_kernel(const unsigned *in, size_t n,
                                                             const unsigned long long *tile_off,
                                                             unsigned long long *out, FaceParams P,
@@ -1909,8 +1987,15 @@ __global__ void __launch_bounds__(kBlock) scan_tiles_kernel(const unsigned *in, 
         v[i] = sv[scan_pad(threadIdx.x * kScanItems + i)];
         s += v[i];
     }
-    unsigned long long total;
-    unsigned long long run = tile_off[blockIdx.x] + block_exclusive_scan(s, total);
+    unsigned long long total, before = 0;
+    if constexpr (DIRECT) {
+        unsigned long long t = 0;
+        for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlock) t += tile_off[i];
+        (void)block_exclusive_scan(t, before);
+    } else {
+        before = tile_off[blockIdx.x];
+    }
+    unsigned long long run = before + block_exclusive_scan(s, total);
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
         so[scan_pad(threadIdx.x * kScanItems + i)] = run;
@@ -1937,14 +2022,18 @@ __global__ void __launch_bounds__(kBlock) scan_tiles_kernel(const unsigned *in, 
 
 size_t scan_temp_words(size_t n) { return (n + kScanTile - 1) / kScanTile; }
 
-hipError_t launch_scan(unsigned long long *tile_tmp, const unsigned *in, unsigned long long *out, size_t n,
+hipError_t launch_scan(unsigned long long *tile_sum, const unsigned *in, unsigned long long *out, size_t n,
                        const FaceParams &p, unsigned long long *bounds, hipStream_t s) {
     const size_t ntiles = scan_temp_words(n);
     if (ntiles == 0 || ntiles > (size_t)INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(scan_tile_sums_kernel, dim3((unsigned)ntiles), dim3(kBlock), 0, s, in, n, tile_tmp);
-    hipLaunchKernelGGL(scan_tile_offsets_kernel, dim3(1), dim3(kBlock), 0, s, tile_tmp, (int)ntiles);
-    hipLaunchKernelGGL(scan_tiles_kernel, dim3((unsigned)ntiles), dim3(kBlock), 0, s, in, n,
-                       (const unsigned long long *)tile_tmp, out, p, bounds);
+    if (ntiles <= kScanDirect) {
+        hipLaunchKernelGGL(scan_tiles_kernel<true>, dim3((unsigned)ntiles), dim3(kBlock), 0, s, in, n,
+                           (const unsigned long long *)tile_sum, out, p, bounds);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(scan_tile_offsets_kernel, dim3(1), dim3(kBlock), 0, s, tile_sum, (int)ntiles);
+    hipLaunchKernelGGL(scan_tiles_kernel<false>, dim3((unsigned)ntiles), dim3(kBlock), 0, s, in, n,
+                       (const unsigned long long *)tile_sum, out, p, bounds);
     return hipGetLastError();
 }
 
@@ -1975,6 +2064,10 @@ static unsigned list_blocks(int count) { return (unsigned)std::min(1024, (count 
 
 hipError_t launch_seg_faces(const FaceParams &p, hipStream_t s) {
     const int b = block_or_default(p.face_block);
+    if (p.fam_mask == 7 && p.g.faces(0) + p.g.faces(1) + p.g.faces(2) < kMergeFaces) {
+        hipLaunchKernelGGL(seg_faces_kernel, dim3(family_blocks(p.g, b)), dim3(b), 0, s, p);
+        return hipGetLastError();
+    }
     if (p.fam_mask & 1) hipLaunchKernelGGL(seg_face_kernel<0>, dim3(grid_for(p.g.faces(0), b)), dim3(b), 0, s, p);
     if (p.fam_mask & 2) hipLaunchKernelGGL(seg_face_kernel<1>, dim3(grid_for(p.g.faces(1), b)), dim3(b), 0, s, p);
     if (p.fam_mask & 4) hipLaunchKernelGGL(seg_face_kernel<2>, dim3(grid_for(p.g.faces(2), b)), dim3(b), 0, s, p);
