@@ -397,7 +397,9 @@ FIA_HD bool load_face(const FaceParams &P, int fam, int i, int j, int k, double 
 // (cells^2), in units of q (reference quadrature src/polygon_3D.cpp:57-77 and 257-487,
 // consumers src/calc_density_in_cell_from_quadrature_point_list_for_integrate_density.cpp:119-201
 // and src/calc_density_in_cell_from_quadrature_point_list.cpp:98-132).
-FIA_HD double piece_flux(const FaceParams &P, const double c[3], double ay, int &npts) {
+// IM: the quadrature points' interpolation fixed at compile time (the code of the other rules, and
+// its registers, left out), or -1.
+template <int IM = -1> FIA_HD double piece_flux(const FaceParams &P, const double c[3], double ay, int &npts) {
     const int mx = P.g.m[0], my = P.g.m[1], mz = P.g.m[2];
     const double ex = 0.5 * P.g.e[0], ey = 0.5 * P.g.e[1], ez = 0.5 * P.g.e[2];
     // field offsets in the physical frame: q at G cell centres, psi on G y-faces
@@ -405,7 +407,7 @@ FIA_HD double piece_flux(const FaceParams &P, const double c[3], double ay, int 
     const double opx = 0.5 - ex, opy = -ey, opz = 0.5 - ez;
     const Loader<double> PS{P.psi, mx, my + 1, mz};
     // the quadrature points' interpolation ("WENO6-optimized": the ISPC variant)
-    const int im = (P.interp == IM_WENO6 && P.weno_opt) ? IM_WENO6_OPT : P.interp;
+    const int im = IM >= 0 ? IM : (P.interp == IM_WENO6 && P.weno_opt) ? IM_WENO6_OPT : P.interp;
     if (!P.integral) {
         return ay * interp_point<double>(PS, im, c[0], c[1], c[2], opx, opy, opz, P.kappa_psi);
     }
@@ -1038,9 +1040,21 @@ FIA_HD double zero_velocity_weno4(const FaceParams &P, int j, const double xl[2]
     return flux;
 }
 
+// The value of piece q = (x strip a, z band b) of a face whose strips and bands are given, by the
+// general quadrature or (LINEAR) the non-integral rule of linear and 1Dy_linear psi alone.
+template <bool LINEAR>
+FIA_HD double zero_velocity_piece(const FaceParams &P, double y, const double xl[2], const double xh[2],
+                                  const double zl[2], const double zh[2], int a, int b) {
+    const double c3[3] = {0.5 * (xl[a] + xh[a]), y, 0.5 * (zl[b] + zh[b])};
+    const double ay = (xh[a] - xl[a]) * (zh[b] - zl[b]);
+    int npts = 0;
+    if constexpr (LINEAR) return piece_value_linear(P, c3, ay);
+    else return piece_flux(P, c3, ay, npts);
+}
+
 // FAST: WENO6 non-integral rule with both axes cut in two (the host decides from the split and the
 // grid's staggering); otherwise the general quadrature per piece.
-template <bool FAST> FIA_HD void zero_velocity_face_body(const FaceParams &P, long id) {
+template <bool FAST, bool LINEAR = false> FIA_HD void zero_velocity_face_body(const FaceParams &P, long id) {
     int i, j, k;
     decode_face(P.g, 1, id, i, j, k);
     const double x0 = i - 0.5 * P.g.e[0], y = j - 0.5 * P.g.e[1], z0 = k - 0.5 * P.g.e[2];
@@ -1053,20 +1067,18 @@ template <bool FAST> FIA_HD void zero_velocity_face_body(const FaceParams &P, lo
         return;
     } else {
         double f = 0.0;
-        int npts = 0;
 #pragma unroll 1
         for (int q = 0; q < nx * nz; ++q) {
             const int a = q / nz, b = q - a * nz;   // x strips outer, z bands inner
-            const double c3[3] = {0.5 * (xl[a] + xh[a]), y, 0.5 * (zl[b] + zh[b])};
-            f += piece_flux(P, c3, (xh[a] - xl[a]) * (zh[b] - zl[b]), npts);
+            f += zero_velocity_piece<LINEAR>(P, y, xl, xh, zl, zh, a, b);
         }
         P.flux[1][id] = f;
     }
 }
-template <bool FAST> __global__ void __launch_bounds__(kBlock) zero_velocity_face_kernel(FaceParams P) {
+template <bool FAST, bool LINEAR = false> __global__ void __launch_bounds__(kBlock) zero_velocity_face_kernel(FaceParams P) {
     const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= (long)P.g.faces(1)) return;
-    zero_velocity_face_body<FAST>(P, id);
+    zero_velocity_face_body<FAST, LINEAR>(P, id);
 }
 
 // Work counters: block sum in LDS, then one atomic per counter and block on one of kStatSlots
@@ -1093,7 +1105,10 @@ __device__ __forceinline__ void add_stats(unsigned long long *stats, int a, int 
 
 // Phase 3: quadrature of every piece slot, one thread per slot (the expensive WENO work runs
 // converged regardless of how many pieces each face has).  QM selects the quadrature: the
-// WENO6 integral rule with NG = QM Gauss points per half (1 or 2), or any mode (QM = 0).
+// WENO6 integral rule with NG = QM Gauss points per half (1 or 2), the linear rule (kPieceLinear, an
+// eighth of the work: at any mode's 213 registers its loads waited on two waves per SIMD,
+// 180 us on 93x61x118, 85 now), or any mode (QM = 0).
+constexpr int kPieceLinear = -1;
 template <int QM, bool OPT = false>
 FIA_HD void piece_body(const FaceParams &P, unsigned long long q, int &npieces, int &npts, int &nevals) {
     const double ay = P.piece_ay[q];
@@ -1101,6 +1116,7 @@ FIA_HD void piece_body(const FaceParams &P, unsigned long long q, int &npieces, 
     if (ay != 0.0) {
         const double c3[3] = {P.piece_c[0][q], P.piece_c[1][q], P.piece_c[2][q]};
         if constexpr (QM == 0) val = piece_flux(P, c3, ay, npts);
+        else if constexpr (QM == kPieceLinear) val = piece_flux<IM_LINEAR>(P, c3, ay, npts);
         else val = piece_flux_weno_integral<QM, OPT>(P, c3, ay, npts, nevals);
         npieces = 1;
     }
@@ -1114,7 +1130,7 @@ piece_kernel(FaceParams P, unsigned long long nslots) {
     const unsigned long long q = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
     int npieces = 0, npts = 0, nevals = 0;
     if (q < nslots) piece_body<QM, OPT>(P, q, npieces, npts, nevals);
-    if (QM != 0 && P.stats) add_stats(P.stats, npieces, npts, nevals);   // counted for the WENO6 rule only
+    if (QM > 0 && P.stats) add_stats(P.stats, npieces, npts, nevals);   // counted for the WENO6 rule only
 }
 
 // The table quadrature, one block per brick of faces.  Read from memory, a piece's 42 rows of 32
@@ -1892,6 +1908,8 @@ hipError_t launch_pieces(const FaceParams &p, unsigned long long nslots, hipStre
         hipLaunchKernelGGL((piece_kernel<1, false>), grid, dim3(b), 0, s, p, nslots);
     } else if (qm == 2) {
         hipLaunchKernelGGL((piece_kernel<2, false>), grid, dim3(b), 0, s, p, nslots);
+    } else if (p.interp == IM_LINEAR) {
+        hipLaunchKernelGGL((piece_kernel<kPieceLinear, false>), grid, dim3(b), 0, s, p, nslots);
     } else {
         hipLaunchKernelGGL((piece_kernel<0, false>), grid, dim3(b), 0, s, p, nslots);
     }
@@ -2053,6 +2071,8 @@ hipError_t launch_zero_velocity_faces(const FaceParams &p, hipStream_t s) {
     // general quadrature per piece)
     if (p.interp == IM_WENO6 && !p.weno_opt && !p.integral && zero_velocity_cuts_both(p))
         hipLaunchKernelGGL(zero_velocity_face_kernel<true>, grid, dim3(b), 0, s, p);
+    else if (p.fuse_value)   // linear or 1Dy_linear psi, not integral
+        hipLaunchKernelGGL((zero_velocity_face_kernel<false, true>), grid, dim3(b), 0, s, p);
     else
         hipLaunchKernelGGL(zero_velocity_face_kernel<false>, grid, dim3(b), 0, s, p);
     return hipGetLastError();
