@@ -1651,12 +1651,12 @@ fia_status fia_cfl_time_step(fia_ctx *c, const fia_grid3d *g, double now_time, i
     HIP_TRY(hipGetLastError());
     const size_t nu = (size_t)(g->nx + 1) * g->ny * g->nz, nv = (size_t)g->nx * (g->ny + 1) * g->nz,
                  nw = (size_t)g->nx * g->ny * (g->nz + 1);
-    HIP_TRY(launch_absmax(gv.u, nu, c->bits.p, c->stream));
-    HIP_TRY(launch_absmax(gv.v, nv, c->bits.p, c->stream));
-    HIP_TRY(launch_absmax(gv.w, nw, c->bits.p, c->stream));
-    unsigned int bits = 0;
-    HIP_TRY(hipMemcpyAsync(&bits, c->bits.p, 4, hipMemcpyDeviceToHost, c->stream));
+    const float *const fields[3] = {gv.u, gv.v, gv.w};
+    const size_t sizes[3] = {nu, nv, nw};
+    HIP_TRY(launch_absmax(fields, sizes, c->bits.p, c->stream));
+    HIP_TRY(hipMemcpyAsync(c->host_flags + 3, c->bits.p, 4, hipMemcpyDeviceToHost, c->stream));   // pinned
     HIP_TRY(hipStreamSynchronize(c->stream));
+    const unsigned int bits = (unsigned int)c->host_flags[3];
     float m;
     memcpy(&m, &bits, 4);
     if (m != m) return fail(FIA_ERR_NONFINITE, "velocity contains NaN");

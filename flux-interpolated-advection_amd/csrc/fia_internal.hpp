@@ -216,7 +216,8 @@ hipError_t launch_interpolate(const float *field, int mx, int my, int mz, double
                               hipStream_t s);
 hipError_t launch_split_faces(const double *quads_cells, size_t n, int split, double min_area, int max_pieces,
                               int *count, double *cen, double *area, int *error, hipStream_t s);
-hipError_t launch_absmax(const float *a, size_t n, unsigned int *out_bits, hipStream_t s);
+// bit pattern of the largest |value| of three arrays, into *out_bits (0 before)
+hipError_t launch_absmax(const float *const a[3], const size_t n[3], unsigned int *out_bits, hipStream_t s);
 
 // Jacobi-PCG (FP64 vectors, FP64 reductions in a fixed order)
 struct PcgGrid {

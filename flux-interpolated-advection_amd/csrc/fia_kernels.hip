@@ -1750,18 +1750,25 @@ __global__ void __launch_bounds__(64) split_faces_kernel(const double *quads, si
     if (over) atomicCAS(error, 0, over);
 }
 
-__global__ void absmax_kernel(const float *a, size_t n, unsigned int *out_bits) {
-    float m = 0.0f;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float v = fabsf(a[i]);
-        m = (v > m || v != v) ? v : m;
-    }
-    // wave reduction then one atomic per wave; |x| bit patterns order like the floats
-    for (int off = 32; off > 0; off >>= 1) {
-        const float o = __shfl_down(m, off, 64);
-        m = (o > m || o != o) ? o : m;
-    }
-    if ((threadIdx.x & 63) == 0) atomicMax(out_bits, __float_as_uint(m));
+// Largest |value| of three arrays as its bit pattern (bit patterns of |x| order like the floats, NaN
+// above all): one atomic per block, of a few blocks per CU (one per wave of 2,048 blocks queued on one
+// address, 62 us a launch of a 64^3 array).
+struct AbsMaxArgs {
+    const float *a[3];
+    size_t n[3];
+};
+__global__ void __launch_bounds__(kBlock) absmax_kernel(AbsMaxArgs A, unsigned int *out_bits) {
+    __shared__ unsigned wave_max[kBlock / 64];
+    unsigned m = 0;
+    for (int f = 0; f < 3; ++f)
+        for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < A.n[f]; i += (size_t)gridDim.x * kBlock)
+            m = max(m, __float_as_uint(A.a[f][i]) & 0x7fffffffu);
+    for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_down((int)m, off, 64));
+    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < kBlock / 64; ++w) m = max(m, wave_max[w]);
+    atomicMax(out_bits, m);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2171,10 +2178,11 @@ hipError_t launch_split_faces(const double *quads, size_t n, int split, double m
     return hipGetLastError();
 }
 
-hipError_t launch_absmax(const float *a, size_t n, unsigned int *out_bits, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    const unsigned blocks = (unsigned)std::min<size_t>(grid_for(n, kBlock), 2048);
-    hipLaunchKernelGGL(absmax_kernel, dim3(blocks), dim3(kBlock), 0, s, a, n, out_bits);
+hipError_t launch_absmax(const float *const a[3], const size_t n[3], unsigned int *out_bits, hipStream_t s) {
+    AbsMaxArgs A;
+    for (int f = 0; f < 3; ++f) { A.a[f] = a[f]; A.n[f] = n[f]; }
+    const unsigned blocks = (unsigned)std::min<size_t>(grid_for(std::max(n[0], std::max(n[1], n[2])), kBlock), 1024);
+    hipLaunchKernelGGL(absmax_kernel, dim3(std::max(1u, blocks)), dim3(kBlock), 0, s, A, out_bits);
     return hipGetLastError();
 }
 
