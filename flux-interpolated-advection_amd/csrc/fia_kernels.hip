@@ -788,26 +788,32 @@ FIA_HD int family_block(const CompGrid &g, unsigned threads, unsigned blk, unsig
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kBlock * kScanItems;
 
-// Adds the wave's slot counts (consecutive faces, n of face gid per lane) to the sums of the scan's
-// tiles, which a wave's faces straddle at most once.
-__device__ __forceinline__ void add_tile_sums(unsigned long long *tile_sum, size_t gid, unsigned n) {
-    const unsigned tile = (unsigned)(gid / kScanTile), t0 = __shfl(tile, 0, 64);
+// Adds the block's slot counts (consecutive faces, n of face gid per thread, first: thread 0's) to the
+// sums of the scan's tiles, which a block's faces straddle at most once: at most two atomics a block
+// (one per wave, 64 to a tile at about the same time, took longer than the counting).
+__device__ __forceinline__ void add_tile_sums(unsigned long long *tile_sum, size_t first, size_t gid, unsigned n) {
+    __shared__ unsigned long long sums[2][kBlock / 64];
+    const unsigned t0 = (unsigned)(first / kScanTile), tile = (unsigned)(gid / kScanTile);
     unsigned long long a = tile == t0 ? n : 0u, b = tile == t0 ? 0u : n;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         a += __shfl_down(a, off, 64);
         b += __shfl_down(b, off, 64);
     }
-    if ((threadIdx.x & 63) == 0) {
-        if (a) atomicAdd(tile_sum + t0, a);
-        if (b) atomicAdd(tile_sum + t0 + 1, b);
+    const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0) { sums[0][wave] = a; sums[1][wave] = b; }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned long long t = 0;
+        for (int w = 0; w < waves; ++w) t += sums[threadIdx.x][w];
+        if (t) atomicAdd(tile_sum + t0 + threadIdx.x, t);
     }
 }
 template <int FAM, bool SUMS>
 __device__ __forceinline__ void face_count_block(const FaceParams &P, unsigned blk, unsigned long long *tile_sum) {
     const long id = (long)blk * blockDim.x + threadIdx.x;
     const unsigned n = id < (long)P.g.faces(FAM) ? face_count_body<FAM>(P, id) : 0u;
-    if constexpr (SUMS) add_tile_sums(tile_sum, P.fam_base[FAM] + (size_t)id, n);
+    if constexpr (SUMS) add_tile_sums(tile_sum, P.fam_base[FAM] + (size_t)blk * blockDim.x, P.fam_base[FAM] + (size_t)id, n);
 }
 template <bool SUMS> __global__ void __launch_bounds__(kBlock) face_count_kernel(FaceParams P, unsigned long long *tile_sum) {
     unsigned blk;
@@ -1790,9 +1796,9 @@ hipError_t launch_vertices(const VertexParams &p, hipStream_t s) {
 
 // Grids under this many faces are bound by launches: the cutters of the three families run as one
 // launch, at the y faces' 157 registers, and the count kernel adds up the scan's tile sums with
-// atomics instead of a kernel that reads the counts (density step, merged and separate: 16^3 335 and
-// 430 us, 32^3 328 and 388, 64^3 651 and 702, 80^3 938 and 962, 96^3 1,379 and 1,357, 256^3 21.3 and
-// 19.8 ms).
+// atomics instead of a kernel that reads the counts (density step, merged and separate: 16^3 330 and
+// 430 us, 32^3 320 and 388, 64^3 626 and 702, 80^3 911 and 962, 96^3 1,347 and 1,342, 104^3 1,757 and
+// 1,740).
 constexpr size_t kMergeFaces = (size_t)1 << 21;
 
 // block-wide exclusive scan of one value per thread (kBlock threads, 64-wide waves); total out
