@@ -5,6 +5,7 @@
 //                     column's y range in eight segments (one wave each), FP64 sums
 //                     (psi_weno_held_kernel: the WENO6 integral rule with the segment held)
 //   vertex_kernel     backtraced displacement of every lattice vertex, one thread per vertex
+//                     (vertex_weno_kernel: the WENO6 rule, tiles of (y, z) marched along x)
 //   face_count_kernel slots of every face (x strips x z bands) and their sums by tile of the scan;
 //                     twisted and degenerate faces listed
 //   scan_*            exclusive scan of the slot counts
@@ -294,7 +295,18 @@ __global__ void __launch_bounds__(64 * kPsiSegs) __attribute__((amdgpu_waves_per
 // ---------------------------------------------------------------------------------------------
 // vertex backtrace (reference src/calc_backtraced_face_3D.cpp:9-159)
 // ---------------------------------------------------------------------------------------------
-FIA_HD void vertex_body(const VertexParams &P, long id) {
+// clamps the position p + d of axis a to [-e_a/2, n_a + e_a/2] (reference :131-159) as a bound on d
+FIA_HD float clamp_displacement(const CompGrid &g, int a, double p, float d) {
+    const float lo = (float)(-0.5 * g.e[a] - p);
+    const float hi = (float)(g.n[a] + 0.5 * g.e[a] - p);
+    if (!(d >= lo)) d = (d != d) ? d : lo;   // NaN passes through and is caught by the face kernel
+    if (d > hi) d = hi;
+    return d;
+}
+
+// METHOD: the interpolation, where it is known at compile time (else -1: P.interp)
+template <int METHOD = -1> FIA_HD void vertex_body(const VertexParams &P, long id) {
+    const int method = METHOD < 0 ? P.interp : METHOD;
     const int ly = P.g.m[1] + 1, lz = P.g.m[2] + 1;
     const int k = (int)(id % lz), j = (int)((id / lz) % ly), i = (int)(id / ((long)ly * lz));
     const int lat[3] = {i, j, k};
@@ -309,27 +321,115 @@ FIA_HD void vertex_body(const VertexParams &P, long id) {
     if (!pinned) {
         const int nx = P.g.n[0], ny = P.g.n[1], nz = P.g.n[2];
         const Loader<float> U{P.u, nx + 1, ny, nz}, V{P.v, nx, ny + 1, nz}, W{P.w, nx, ny, nz + 1};
-        const float vu = interp_point<float>(U, P.interp, p[0], p[1], p[2], 0.0, 0.5, 0.5, 1.0f);
-        const float vv = interp_point<float>(V, P.interp, p[0], p[1], p[2], 0.5, 0.0, 0.5, 1.0f);
-        const float vw = interp_point<float>(W, P.interp, p[0], p[1], p[2], 0.5, 0.5, 0.0, 1.0f);
+        const float vu = interp_point<float>(U, method, p[0], p[1], p[2], 0.0, 0.5, 0.5, 1.0f);
+        const float vv = interp_point<float>(V, method, p[0], p[1], p[2], 0.5, 0.0, 0.5, 1.0f);
+        const float vw = interp_point<float>(W, method, p[0], p[1], p[2], 0.5, 0.5, 0.0, 1.0f);
         d[0] = -P.dt_over_h * vu;
         d[1] = -P.dt_over_h * vv;
         d[2] = -P.dt_over_h * vw;
     }
     for (int a = 0; a < 3; ++a) {
-        // clamp the position to [-e_a/2, n_a + e_a/2] (reference :131-159) as a bound on d
-        const float lo = (float)(-0.5 * P.g.e[a] - p[a]);
-        const float hi = (float)(P.g.n[a] + 0.5 * P.g.e[a] - p[a]);
-        float v = d[a];
-        if (!(v >= lo)) v = (v != v) ? v : lo;   // NaN passes through and is caught by the face kernel
-        if (v > hi) v = hi;
-        P.disp[a][id] = v;
+        P.disp[a][id] = clamp_displacement(P.g, a, p[a], d[a]);
     }
 }
-__global__ void __launch_bounds__(kBlock) vertex_kernel(VertexParams P) {
+// Compiled for the linear rules each alone (76 and 41 registers; every rule in one took 162, which
+// leave three waves per SIMD): 1Dy_linear 292 -> 110 us at 256^3.
+template <int METHOD> __global__ void __launch_bounds__(kBlock) vertex_kernel(VertexParams P) {
     const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= (long)(P.g.m[0] + 1) * (P.g.m[1] + 1) * (P.g.m[2] + 1)) return;
-    vertex_body(P, id);
+    vertex_body<METHOD>(P, id);
+}
+
+// WENO6 displacements.  Every lattice vertex lies on a sample or half way between two along each axis
+// of a velocity component, the same for all vertices, and the passes (z, y, x, as weno3d) of
+// neighbouring vertices have most of their rows in common: a vertex on its own takes 21 stencil
+// evaluations on the cell lattice and 45 on a face component's, VALU bound.  Here each pass is
+// taken once per row: a block marches along x over a 16 x 16 tile of (y, z); a plane's z passes go
+// through LDS to the y passes (21 rows for 16), and a thread holds its last six y values for the x
+// pass.  One component per blockIdx.y; 256^3, three components: 1,027 -> 250 us (cell
+// lattice), 1,594 -> 244 (face components).
+constexpr int kVtxTile = 16;
+__global__ void __launch_bounds__(kVtxTile * kVtxTile) vertex_weno_kernel(VertexParams P, int tiles_y, int tiles_z,
+                                                                          int chunk) {
+    __shared__ float zs[2][(kVtxTile + 5) * kVtxTile];
+    const int comp = blockIdx.y, tid = threadIdx.x, z = tid % kVtxTile, y = tid / kVtxTile;
+    const int bz = blockIdx.x % tiles_z, by = (blockIdx.x / tiles_z) % tiles_y, bx = blockIdx.x / (tiles_z * tiles_y);
+    const int lx = P.g.m[0] + 1, ly = P.g.m[1] + 1, lz = P.g.m[2] + 1;
+    const int i0 = bx * chunk, i1 = min(lx, i0 + chunk), j0 = by * kVtxTile, j = j0 + y, k = bz * kVtxTile + z;
+    const float *__restrict__ F = comp == 0 ? P.u : (comp == 1 ? P.v : P.w);
+    float *__restrict__ out = P.disp[0];
+    if (comp == 1) out = P.disp[1];
+    if (comp == 2) out = P.disp[2];
+    // sample coordinate of lattice index l along axis a: l + base_a, plus a half if half_a
+    int m[3], base[3];
+    bool half[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int e = P.g.e[a], o = a != comp;
+        m[a] = P.g.n[a] + (a == comp);
+        half[a] = (e + o) & 1;
+        base[a] = -((e + o + 1) >> 1);
+    }
+    const WenoCoef wc(0.5f, 1.0f);
+    // offsets in a plane of the six samples of this thread's z pass (row j0 + y - 2 if the y pass
+    // follows, row j otherwise) or, with z on a sample, of its y pass (or of its one sample)
+    const bool zy = half[2] && half[1];
+    const int jr = (zy ? j0 + y - 2 : j) + base[1], kz = k + base[2];
+    const unsigned mz = (unsigned)m[2], row = (unsigned)clampi(jr, 0, m[1] - 1) * mz;
+    unsigned off[6];
+#pragma unroll
+    for (int r = 0; r < 6; ++r)
+        off[r] = half[2] ? row + (unsigned)clampi(kz - 2 + r, 0, m[2] - 1)
+                         : (unsigned)clampi(half[1] ? jr - 2 + r : jr, 0, m[1] - 1) * mz +
+                               (unsigned)clampi(kz, 0, m[2] - 1);
+    // the tile's last five rows of z passes
+    const bool second = zy && y < 5;
+    const unsigned step = (unsigned)clampi(jr + kVtxTile, 0, m[1] - 1) * mz - row;
+    const int planes = i1 - i0 + (half[0] ? 5 : 0), first = i0 + base[0] - (half[0] ? 2 : 0);
+    float yv[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p = 0; p < planes; ++p) {
+        const float *__restrict__ plane = F + (size_t)clampi(first + p, 0, m[0] - 1) * m[1] * m[2];
+        float f[6], v;
+        if (half[2] || half[1]) {
+#pragma unroll
+            for (int r = 0; r < 6; ++r) f[r] = plane[off[r]];
+            v = weno6<float>(f, wc);
+            if (zy) {
+                float *rows = zs[p & 1];
+                rows[tid] = v;
+                if (second) {
+#pragma unroll
+                    for (int r = 0; r < 6; ++r) f[r] = plane[off[r] + step];
+                    rows[tid + kVtxTile * kVtxTile] = weno6<float>(f, wc);
+                }
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < 6; ++r) f[r] = rows[tid + r * kVtxTile];
+                v = weno6<float>(f, wc);
+            }
+        } else {
+            v = plane[off[0]];
+        }
+        if (half[0]) {
+#pragma unroll
+            for (int r = 0; r < 5; ++r) yv[r] = yv[r + 1];
+            yv[5] = v;
+            if (p < 5) continue;
+            v = weno6<float>(yv, wc);
+        }
+        const int i = i0 + p - (half[0] ? 5 : 0);
+        if (j < ly && k < lz) {
+            const int lat[3] = {i, j, k};
+            float d = -P.dt_over_h * v;
+            double pos = 0.0;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                if (a == P.g.comp && (lat[a] <= 1 || lat[a] >= P.g.n[a])) d = 0.0f;
+                if (a == comp) pos = lat[a] - 0.5 * P.g.e[a];
+            }
+            out[idx3(i, j, k, ly, lz)] = clamp_displacement(P.g, comp, pos, d);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1789,8 +1889,29 @@ hipError_t launch_psi(const PsiParams &p, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Planes of x per block of the WENO6 kernel: long chunks repeat less of the five planes before a chunk,
+// short ones fill the chip: as many as leave kVtxBlocks blocks, four at least (256^3 with 2,048, 4,096
+// and 8,192 blocks: 272, 250 and 243 us, 128^3 with 4,096 and 8,192: 48 and 52; at least 2, 4 and 8
+// planes on 75x96x50: 18, 17 and 21 us).
+constexpr unsigned kVtxBlocks = 4096;
+
 hipError_t launch_vertices(const VertexParams &p, hipStream_t s) {
-    hipLaunchKernelGGL(vertex_kernel, dim3(grid_for(p.g.lattice(), kBlock)), dim3(kBlock), 0, s, p);
+    const int lx = p.g.m[0] + 1, ly = p.g.m[1] + 1, lz = p.g.m[2] + 1;
+    // in-plane byte offsets of the WENO6 kernel are 32 bits
+    if (p.interp == IM_WENO6 && (size_t)ly * lz < ((size_t)1 << 29)) {
+        const int ty = (ly + kVtxTile - 1) / kVtxTile, tz = (lz + kVtxTile - 1) / kVtxTile;
+        const size_t tiles = (size_t)ty * tz;
+        size_t chunk = (size_t)lx * tiles * 3 / kVtxBlocks;
+        chunk = std::min<size_t>(std::max<size_t>(chunk, 4), 64);
+        const size_t blocks = tiles * (((size_t)lx + chunk - 1) / chunk);
+        hipLaunchKernelGGL(vertex_weno_kernel, dim3((unsigned)blocks, 3), dim3(kVtxTile * kVtxTile), 0, s, p, ty, tz,
+                           (int)chunk);
+        return hipGetLastError();
+    }
+    const dim3 grid(grid_for(p.g.lattice(), kBlock));
+    if (p.interp == IM_LINEAR) hipLaunchKernelGGL(vertex_kernel<IM_LINEAR>, grid, dim3(kBlock), 0, s, p);
+    else if (p.interp == IM_1DY_LINEAR) hipLaunchKernelGGL(vertex_kernel<IM_1DY_LINEAR>, grid, dim3(kBlock), 0, s, p);
+    else hipLaunchKernelGGL(vertex_kernel<-1>, grid, dim3(kBlock), 0, s, p);
     return hipGetLastError();
 }
 
