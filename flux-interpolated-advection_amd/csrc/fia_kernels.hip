@@ -1103,47 +1103,61 @@ FIA_HD int unit_interval_pieces(double a, bool cut, double off, double lo[2], do
     return 1;
 }
 
-// WENO6 psi of the 2 x 2 pieces at once (non-integral rule): the four centres lie on psi's sample
-// level j, so each value is a z pass then an x pass over the 6 x 6 samples of that level around it.
-// The two centres along an axis are half a cell apart, so their sample bases differ by 0 or 1 and
-// the four stencils fit in 7 x 7 samples.  Columns are visited in x order: each gets one z pass
-// per z centre (14 evaluations in all) into a 6-column window, and a piece's x pass runs when the
-// window holds its six columns (4 more), the same arithmetic as weno3d.
-FIA_HD double zero_velocity_weno4(const FaceParams &P, int j, const double xl[2], const double xh[2],
-                                  const double zl[2], const double zh[2]) {
+// WENO6 psi of the 2 x 2 pieces of the y faces i0 .. i1 - 1 at row = (j, k) of a plane (non-integral
+// rule, both axes cut in two): the four centres lie on psi's sample level j, so each value is a z pass
+// then an x pass over the 6 x 6 samples of that level around it, the same arithmetic as weno3d.  The
+// two centres along an axis are half a cell apart, so their sample bases differ by 0 or 1, and the
+// fractions are those of every face: columns are visited in x order, each gets one z pass per z centre
+// into a 6-column window, shared by the faces around it, and a piece's x pass runs when the window
+// holds its six columns: six evaluations a face (18 for a face on its own).  The first x centre's
+// pieces are complete one column early when the second's base is one further (dx).
+FIA_HD void zero_velocity_weno(const FaceParams &P, unsigned row, int i0, int i1) {
+    const int my1 = P.g.m[1] + 1, mz = P.g.m[2];
+    const int j = (int)(row / (unsigned)mz), k = (int)(row - (unsigned)j * (unsigned)mz);
     const double opx = 0.5 - 0.5 * P.g.e[0], opz = 0.5 - 0.5 * P.g.e[2];
+    double off, xl[2], xh[2], zl[2], zh[2];
     int bx[2], bz[2];
     float tx[2], tz[2];
+    const bool cx = split_offset(P.split, 0, off);
+    unit_interval_pieces(i0 - 0.5 * P.g.e[0], cx, off, xl, xh);
+    const bool cz = split_offset(P.split, 1, off);
+    unit_interval_pieces(k - 0.5 * P.g.e[2], cz, off, zl, zh);
+#pragma unroll
     for (int a = 0; a < 2; ++a) {
         split_coord(0.5 * (xl[a] + xh[a]) - opx, bx[a], tx[a]);
         split_coord(0.5 * (zl[a] + zh[a]) - opz, bz[a], tz[a]);
     }
     const int dx = bx[1] - bx[0], dz = bz[1] - bz[0];   // 0 or 1
-    const Loader<double> PS{P.psi, P.g.m[0], P.g.m[1] + 1, P.g.m[2]};
+    const double x0 = xh[0] - xl[0], x1 = xh[1] - xl[1], z0 = zh[0] - zl[0], z1 = zh[1] - zl[1];
     const WenoCoef wz0(tz[0], P.kappa_psi), wz1(tz[1], P.kappa_psi);
-    double w0[6] = {0, 0, 0, 0, 0, 0}, w1[6] = {0, 0, 0, 0, 0, 0};   // z passes of the last 6 columns
-    double flux = 0.0;
-#pragma unroll 1
-    for (int c = 0; c < 7; ++c) {
-        double f[7];
+    const WenoCoef wx0(tx[0], P.kappa_psi), wx1(tx[1], P.kappa_psi);
+    unsigned at[7];
 #pragma unroll
-        for (int r = 0; r < 7; ++r) f[r] = PS(bx[0] - 2 + c, j, bz[0] - 2 + r);
-        double g[6];
+    for (int r = 0; r < 7; ++r) at[r] = (unsigned)(j * mz + clampi(bz[0] - 2 + r, 0, mz - 1));
+    double w0[6] = {0, 0, 0, 0, 0, 0}, w1[6] = {0, 0, 0, 0, 0, 0};   // z passes of the last 6 columns
+    double first = 0.0;   // the first x centre's pieces of the face in progress
+    const size_t plane = (size_t)my1 * mz;
+    const int lead = 5 + dx;   // column c completes face i0 + c - lead
+#pragma unroll 1
+    for (int c = 0; c < i1 - i0 + lead; ++c) {
+        const double *__restrict__ psi = P.psi + (size_t)clampi(bx[0] - 2 + c, 0, P.g.m[0] - 1) * plane;
+        double f[7], g[6];
+#pragma unroll
+        for (int r = 0; r < 7; ++r) f[r] = psi[at[r]];
 #pragma unroll
         for (int r = 0; r < 6; ++r) g[r] = dz ? f[r + 1] : f[r];
-        const double v0 = weno6<double>(f, wz0), v1 = weno6<double>(g, wz1);
 #pragma unroll
         for (int r = 0; r < 5; ++r) { w0[r] = w0[r + 1]; w1[r] = w1[r + 1]; }
-        w0[5] = v0; w1[5] = v1;
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            if (c != 5 + (a == 1 ? dx : 0)) continue;
-            const WenoCoef wx(tx[a], P.kappa_psi);
-            flux += ((xh[a] - xl[a]) * (zh[0] - zl[0])) * weno6<double>(w0, wx);
-            flux += ((xh[a] - xl[a]) * (zh[1] - zl[1])) * weno6<double>(w1, wx);
-        }
+        w0[5] = weno6<double>(f, wz0);
+        w1[5] = weno6<double>(g, wz1);
+        if (c < 5) continue;
+        const double mine = (x0 * z0) * weno6<double>(w0, wx0) + (x0 * z1) * weno6<double>(w1, wx0);
+        if (dx == 0) first = mine;
+        if (c >= lead)
+            P.flux[1][(size_t)(i0 + c - lead) * plane + row] =
+                first + (x1 * z0) * weno6<double>(w0, wx1) + (x1 * z1) * weno6<double>(w1, wx1);
+        first = mine;
     }
-    return flux;
 }
 
 // The value of piece q = (x strip a, z band b) of a face whose strips and bands are given, by the
@@ -1163,28 +1177,31 @@ FIA_HD double zero_velocity_piece(const FaceParams &P, double y, const double xl
 template <bool FAST, bool LINEAR = false> FIA_HD void zero_velocity_face_body(const FaceParams &P, long id) {
     int i, j, k;
     decode_face(P.g, 1, id, i, j, k);
+    if constexpr (FAST) return zero_velocity_weno(P, (unsigned)(j * P.g.m[2] + k), i, i + 1);
     const double x0 = i - 0.5 * P.g.e[0], y = j - 0.5 * P.g.e[1], z0 = k - 0.5 * P.g.e[2];
     double ox, oz;
     const bool cx = split_offset(P.split, 0, ox), cz = split_offset(P.split, 1, oz);
     double xl[2], xh[2], zl[2], zh[2];
     const int nx = unit_interval_pieces(x0, cx, ox, xl, xh), nz = unit_interval_pieces(z0, cz, oz, zl, zh);
-    if constexpr (FAST) {
-        P.flux[1][id] = (nx == 2 && nz == 2) ? zero_velocity_weno4(P, j, xl, xh, zl, zh) : 0.0;
-        return;
-    } else {
-        double f = 0.0;
+    double f = 0.0;
 #pragma unroll 1
-        for (int q = 0; q < nx * nz; ++q) {
-            const int a = q / nz, b = q - a * nz;   // x strips outer, z bands inner
-            f += zero_velocity_piece<LINEAR>(P, y, xl, xh, zl, zh, a, b);
-        }
-        P.flux[1][id] = f;
+    for (int q = 0; q < nx * nz; ++q) {
+        const int a = q / nz, b = q - a * nz;   // x strips outer, z bands inner
+        f += zero_velocity_piece<LINEAR>(P, y, xl, xh, zl, zh, a, b);
     }
+    P.flux[1][id] = f;
 }
-template <bool FAST, bool LINEAR = false> __global__ void __launch_bounds__(kBlock) zero_velocity_face_kernel(FaceParams P) {
+template <bool LINEAR> __global__ void __launch_bounds__(kBlock) zero_velocity_face_kernel(FaceParams P) {
     const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= (long)P.g.faces(1)) return;
-    zero_velocity_face_body<FAST, LINEAR>(P, id);
+    zero_velocity_face_body<false, LINEAR>(P, id);
+}
+// One row of a chunk of x planes per thread (VALU bound; 256^3: 690 us with a thread per face, 161 so).
+__global__ void __launch_bounds__(kBlock) zero_velocity_weno_kernel(FaceParams P, int chunk) {
+    const unsigned row = blockIdx.x * blockDim.x + threadIdx.x;
+    if (row >= (unsigned)(P.g.m[1] + 1) * (unsigned)P.g.m[2]) return;
+    const int i0 = (int)blockIdx.y * chunk;
+    zero_velocity_weno(P, row, i0, min(P.g.m[0], i0 + chunk));
 }
 
 // Work counters: block sum in LDS, then one atomic per counter and block on one of kStatSlots
@@ -2203,12 +2220,21 @@ hipError_t launch_zero_velocity_faces(const FaceParams &p, hipStream_t s) {
     const dim3 grid(grid_for(p.g.faces(1), b));
     // (the closed form's shared stencils are the WENO6 rule's; "WENO6-optimized" takes the
     // general quadrature per piece)
-    if (p.interp == IM_WENO6 && !p.weno_opt && !p.integral && zero_velocity_cuts_both(p))
+    if (p.interp == IM_WENO6 && !p.weno_opt && !p.integral && zero_velocity_cuts_both(p)) {
+        // planes per thread: a chunk repeats five or six columns, so long ones where the chip stays
+        // full (256^3 with 32 and 64 planes: 161 and 185 us; 128^3 with 4 and 8: 40 and 36), four on
+        // 75x96x50 (13 us, 15 with 8 and 22 with one) and one where four leave CUs idle (32^3: 8 and 11)
+        const size_t rows = grid_for((size_t)(p.g.m[1] + 1) * p.g.m[2], b), all = rows * p.g.m[0] * b / kBlock;
+        const size_t chunk = std::min<size_t>(
+            std::max<size_t>({all / 1024, std::min<size_t>(4, all / 256), (size_t)1}), 32);
+        hipLaunchKernelGGL(zero_velocity_weno_kernel,
+                           dim3((unsigned)rows, (unsigned)(((size_t)p.g.m[0] + chunk - 1) / chunk)), dim3(b), 0, s, p,
+                           (int)chunk);
+    } else if (p.fuse_value) {   // linear or 1Dy_linear psi, not integral
         hipLaunchKernelGGL(zero_velocity_face_kernel<true>, grid, dim3(b), 0, s, p);
-    else if (p.fuse_value)   // linear or 1Dy_linear psi, not integral
-        hipLaunchKernelGGL((zero_velocity_face_kernel<false, true>), grid, dim3(b), 0, s, p);
-    else
+    } else {
         hipLaunchKernelGGL(zero_velocity_face_kernel<false>, grid, dim3(b), 0, s, p);
+    }
     return hipGetLastError();
 }
 
