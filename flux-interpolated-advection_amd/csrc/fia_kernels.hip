@@ -1012,9 +1012,11 @@ template <int FAM> FIA_HD void seg_piece_body(const FaceParams &P, long id, unsi
                   m > 0 ? (double)(z0 + m - 1) : -kNoBound, m < nzc ? (double)(z0 + m) : kNoBound, acc);
     store_piece(P, geom, acc.area2, acc.mxi, acc.meta, acc.ay2, P.face_start[gid] + local);
 }
-// x and z faces (one cut direction each) fit 128 VGPRs, four waves per SIMD, with one spilled value
-// in the piece-by-piece phase (1.03 -> 0.86 ms per launch at 256^3); the y faces (two cut
-// directions) need 160 and keep three waves (bound to 128 they spill 126 values)
+// VALU bound (FP64; 1,100 instructions a wave on x and z faces, 1,800 on y faces, half of them in the
+// stores' centres and divides and in the few faces cut piece by piece).  x and z faces (one cut
+// direction each) fit 128 VGPRs, four waves per SIMD: 0.75 and 0.74 ms per launch at 256^3.  The y faces
+// (two cut directions) take 140 and keep three waves, 1.31 ms: bound to 128 they spill 18 values and the
+// density step takes 18.6 ms instead of 17.6.
 struct SegShared {
     unsigned face[kBlock];   // the block's faces cut piece by piece (index in the family)
     unsigned end[kBlock];    // their slot counts, then the inclusive prefix of them
@@ -1933,7 +1935,7 @@ hipError_t launch_vertices(const VertexParams &p, hipStream_t s) {
 }
 
 // Grids under this many faces are bound by launches: the cutters of the three families run as one
-// launch, at the y faces' 157 registers, and the count kernel adds up the scan's tile sums with
+// launch, at the y faces' 140 registers, and the count kernel adds up the scan's tile sums with
 // atomics instead of a kernel that reads the counts (density step, merged and separate: 16^3 330 and
 // 430 us, 32^3 320 and 388, 64^3 626 and 702, 80^3 911 and 962, 96^3 1,347 and 1,342, 104^3 1,757 and
 // 1,740).
