@@ -472,6 +472,11 @@ FIA_HD bool face_twisted(const double col[4][2]) {
 // it the recursive cut decides which side gets the edge from the rounding of interpolated
 // colours; such faces take the recursive cutter, as twisted ones do.
 FIA_HD bool face_degenerate(const double col[4][2]) {
+    // most faces have no integer corner colour at all
+    bool any = false;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) any = any | (col[c][0] == floor(col[c][0])) | (col[c][1] == floor(col[c][1]));
+    if (!any) return false;
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
         const double lo = fmin(fmin(col[0][d], col[1][d]), fmin(col[2][d], col[3][d]));

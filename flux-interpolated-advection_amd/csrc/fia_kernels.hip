@@ -455,11 +455,14 @@ FIA_HD bool load_face(const FaceParams &P, int fam, int i, int j, int k, double 
     const bool moving = P.disp[0] != nullptr;
     float d[4][3];
     if (moving) {
+        // one 64-bit index for the four corners, the others at uniform distances from it (with the test
+        // in face_degenerate: counts 419 -> 376 us, y faces 1,308 -> 1,249 at 256^3)
+        const size_t v0 = idx3(i, j, k, ly, lz);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             int o[3];
             face_corner_offsets(fam, c, o);
-            const size_t vi = idx3(i + o[0], j + o[1], k + o[2], ly, lz);
+            const size_t vi = v0 + (o[0] ? (size_t)ly * lz : 0) + (o[1] ? (size_t)lz : 0) + o[2];
 #pragma unroll
             for (int a = 0; a < 3; ++a) d[c][a] = P.disp[a][vi];
         }
@@ -1012,10 +1015,10 @@ template <int FAM> FIA_HD void seg_piece_body(const FaceParams &P, long id, unsi
                   m > 0 ? (double)(z0 + m - 1) : -kNoBound, m < nzc ? (double)(z0 + m) : kNoBound, acc);
     store_piece(P, geom, acc.area2, acc.mxi, acc.meta, acc.ay2, P.face_start[gid] + local);
 }
-// VALU bound (FP64; 1,100 instructions a wave on x and z faces, 1,800 on y faces, half of them in the
+// VALU bound (FP64; about 1,050 instructions a wave on x and z faces, 1,700 on y faces, half in the
 // stores' centres and divides and in the few faces cut piece by piece).  x and z faces (one cut
-// direction each) fit 128 VGPRs, four waves per SIMD: 0.75 and 0.74 ms per launch at 256^3.  The y faces
-// (two cut directions) take 140 and keep three waves, 1.31 ms: bound to 128 they spill 18 values and the
+// direction each) fit 128 VGPRs, four waves per SIMD: 0.73 ms per launch each at 256^3.  The y faces
+// (two cut directions) take 140 and keep three waves, 1.25 ms: bound to 128 they spill 18 values and the
 // density step takes 18.6 ms instead of 17.6.
 struct SegShared {
     unsigned face[kBlock];   // the block's faces cut piece by piece (index in the family)
