@@ -64,10 +64,11 @@ FIA_HD void atomic_cas_i32(int *p, int cmp, int v) {
 // ---------------------------------------------------------------------------------------------
 // psi (reference src/calc_psi_3D.cpp:10-308 density, :311-537 velocity)
 // ---------------------------------------------------------------------------------------------
-// Increment of psi across cell jj of column (i, k): the integral of q over the cell in y.
-FIA_HD float psi_increment(const PsiParams &P, const Loader<float> &Q, int i, int jj, int k) {
+// Increment of psi across cell jj of column (i, k): the integral of q over the cell in y.  WENO: the
+// WENO6 integral rule may be asked for.
+template <bool WENO = true> FIA_HD float psi_increment(const PsiParams &P, const Loader<float> &Q, int i, int jj, int k) {
     if (!P.integral || P.mode == 0) return Q(i, jj, k);
-    if (P.mode == 1) {
+    if (!WENO || P.mode == 1) {
         // trilinear at (x_c, jj + 1/4, z_c) and (x_c, jj + 3/4, z_c): x, z on nodes
         const float a = 0.25f * Q(i, jj - 1, k) + 0.75f * Q(i, jj, k);   // sample jj - 1/4
         const float b = 0.75f * Q(i, jj, k) + 0.25f * Q(i, jj + 1, k);   // sample jj + 1/4
@@ -200,11 +201,13 @@ template <bool HELD> __global__ void __launch_bounds__(64 * kPsiSegs) psi_kernel
     psi_segment(my, w, j0, j1);
     __shared__ double tot[kPsiSegs][64];
     if constexpr (HELD) {
+        // (with the WENO6 rule's code in the loop it is too long to unroll and the increments go to
+        // scratch memory: 77 us at 256^3, 37 without it)
         float inc[kPsiHeld];
         double s = 0.0;
 #pragma unroll
         for (int r = 0; r < kPsiHeld; ++r) {
-            inc[r] = (own && j0 + r < j1) ? psi_increment(P, Q, i, j0 + r, k) : 0.0f;
+            inc[r] = (own && j0 + r < j1) ? psi_increment<false>(P, Q, i, j0 + r, k) : 0.0f;
             s += (double)inc[r];
         }
         tot[w][lane] = s;
