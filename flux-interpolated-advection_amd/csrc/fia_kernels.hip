@@ -13,6 +13,7 @@
 //   degenerate_kernel clipping pipeline for faces with a corner colour on an interior integer
 //   zero_velocity_face_kernel  the zero-velocity correction pass: the undeformed y faces' pieces
 //                     in closed form (at most 2 x 2 axis-aligned rectangles per face)
+//                     (zero_velocity_weno_kernel: the WENO6 rule, rows marched along x)
 //   weno_table_kernel, piece_brick_kernel  quadrature of every piece slot under the WENO6 integral
 //                     rule: the z stencils' interpolants in tables, read from LDS by bricks of faces
 //   piece_kernel      quadrature of every piece slot, any rule (small grids: piece_kernel<1>)
@@ -1018,10 +1019,10 @@ template <int FAM> FIA_HD void seg_piece_body(const FaceParams &P, long id, unsi
                   m > 0 ? (double)(z0 + m - 1) : -kNoBound, m < nzc ? (double)(z0 + m) : kNoBound, acc);
     store_piece(P, geom, acc.area2, acc.mxi, acc.meta, acc.ay2, P.face_start[gid] + local);
 }
-// VALU bound (FP64; about 1,050 instructions a wave on x and z faces, 1,700 on y faces, half in the
+// VALU bound (FP64; 850-990 instructions a wave on x and z faces, 1,440-1,670 on y faces, half in the
 // stores' centres and divides and in the few faces cut piece by piece).  x and z faces (one cut
-// direction each) fit 128 VGPRs, four waves per SIMD: 0.73 ms per launch each at 256^3.  The y faces
-// (two cut directions) take 140 and keep three waves, 1.25 ms: bound to 128 they spill 18 values and the
+// direction each) fit 128 VGPRs, four waves per SIMD: 0.70 and 0.71 ms per launch at 256^3.  The y faces
+// (two cut directions) take 140 and keep three waves, 1.22 ms: bound to 128 they spill 18 values and the
 // density step takes 18.6 ms instead of 17.6.
 struct SegShared {
     unsigned face[kBlock];   // the block's faces cut piece by piece (index in the family)
