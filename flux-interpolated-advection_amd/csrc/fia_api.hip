@@ -357,7 +357,9 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     for (int f = 0; f < 3; ++f) {
         if (g.faces(f) >= (size_t(1) << 30)) return fail(FIA_ERR_INVALID_ARG, "grid too large for the face index");
         HIP_TRY(fs.f[f].ensure(g.faces(f)));
-        if (!fs.c[f].p || fs.c[f].n < g.faces(f)) {   // new corrections and masks start at zero
+        // new corrections and masks start at zero, both of them if either is new: an earlier call may have
+        // had memory for the first alone
+        if (!fs.c[f].holds(g.faces(f)) || !fs.m[f].holds((fs.c[f].n + 31) / 32)) {
             HIP_TRY(fs.c[f].ensure(g.faces(f)));
             HIP_TRY(fs.m[f].ensure((fs.c[f].n + 31) / 32));
             HIP_TRY(hipMemsetAsync(fs.c[f].p, 0, fs.c[f].bytes(), c->stream));

@@ -17,16 +17,23 @@ struct WenoHalf;   // fia_math.hpp
 template <class T> struct DevBuf {
     T *p = nullptr;
     size_t n = 0;
+    bool holds(size_t want) const { return want <= n && p; }
+    // a failure is the caller's to handle, and not left for the check after the next launch
     hipError_t ensure(size_t want) {
-        if (want <= n && p) return hipSuccess;
+        if (holds(want)) return hipSuccess;
         if (p) { hipError_t e = hipFree(p); if (e != hipSuccess) return e; p = nullptr; n = 0; }
         hipError_t e = hipMalloc((void **)&p, std::max<size_t>(want, 1) * sizeof(T));
-        if (e == hipSuccess) n = want;
+        if (e == hipSuccess) {
+            n = want;
+        } else {
+            p = nullptr;
+            (void)hipGetLastError();
+        }
         return e;
     }
     // for sizes that follow the data: an eighth more than asked when it has to grow, so that a
     // slightly larger next call does not allocate (and so synchronise) again
-    hipError_t ensure_slack(size_t want) { return want <= n && p ? hipSuccess : ensure(want + want / 8); }
+    hipError_t ensure_slack(size_t want) { return holds(want) ? hipSuccess : ensure(want + want / 8); }
     void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
     size_t bytes() const { return n * sizeof(T); }
 };
