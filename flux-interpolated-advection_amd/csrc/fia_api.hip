@@ -4,6 +4,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -105,6 +106,8 @@ struct fia_ctx {
     double *host_scal = nullptr;                 // pinned: PCG scalars of two solves read back while iterating
     DevBuf<double> piece_c[3], piece_ay, piece_val;
     DevBuf<WenoHalf> weno_tab[2];          // z stencils of q and psi (WENO6 integral quadrature)
+    bool tables_used = false;              // a pass is taking them up: not to be given back
+    fia_ctx *prev = nullptr, *next = nullptr;   // the process's contexts (both under g_contexts_lock)
     DevBuf<unsigned> gen_n;                 // twisted faces: pieces per face and orientation
     DevBuf<unsigned long long> gen_start;   // their exclusive scan and total
     DevBuf<double> gen_c[3], gen_ay, gen_val;   // the twisted faces' piece records and values
@@ -201,7 +204,49 @@ struct fia_unet {
     DevBuf<double> rhs;
 };
 
+// The process's contexts, whose tables an allocation may take back.
+static std::mutex g_contexts_lock;
+static fia_ctx *g_contexts = nullptr;
+
+static void list_context(fia_ctx *c) {
+    const std::lock_guard<std::mutex> lock(g_contexts_lock);
+    c->next = g_contexts;
+    if (g_contexts) g_contexts->prev = c;
+    g_contexts = c;
+}
+static void unlist_context(fia_ctx *c) {
+    const std::lock_guard<std::mutex> lock(g_contexts_lock);
+    if (c->prev) c->prev->next = c->next;
+    else if (g_contexts == c) g_contexts = c->next;
+    if (c->next) c->next->prev = c->prev;
+}
+// Between them the context's tables are its own pass's: from their allocation until the launches
+// that read them are enqueued (hipFree waits for those).
+struct TableUse {
+    fia_ctx *c;
+    explicit TableUse(fia_ctx *ctx) : c(ctx) { set(true); }
+    ~TableUse() { set(false); }
+    void set(bool used) {
+        const std::lock_guard<std::mutex> lock(g_contexts_lock);
+        c->tables_used = used;
+    }
+};
+
 namespace fia {
+bool give_back_scratch() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    const std::lock_guard<std::mutex> lock(g_contexts_lock);
+    bool any = false;
+    for (fia_ctx *c = g_contexts; c; c = c->next) {
+        if (c->device != dev || c->tables_used) continue;
+        for (auto &t : c->weno_tab) {
+            any = any || t.p;
+            t.release();
+        }
+    }
+    return any;
+}
 int ctx_device(const fia_ctx *c) { return c->device; }
 hipStream_t ctx_stream(const fia_ctx *c) { return c->stream; }
 int ctx_precond(const fia_ctx *c) { return c->precond; }
@@ -215,7 +260,11 @@ size_t ctx_bytes(const fia_ctx *c) {
     size_t b = c->psi.bytes() + c->twisted.bytes() + c->degen.bytes() + c->counters.bytes() + c->scal.bytes() + c->bits.bytes() +
                c->solid.bytes() + c->genI.bytes();
     b += c->fsa.bytes() + c->fsb.bytes() + c->face_n.bytes() + c->face_start.bytes() + c->scan_tmp.bytes() +
-         c->piece_ay.bytes() + c->piece_val.bytes() + c->weno_tab[0].bytes() + c->weno_tab[1].bytes();
+         c->piece_ay.bytes() + c->piece_val.bytes();
+    {
+        const std::lock_guard<std::mutex> lock(g_contexts_lock);
+        b += c->weno_tab[0].bytes() + c->weno_tab[1].bytes();
+    }
     for (int a = 0; a < 3; ++a) b += c->piece_c[a].bytes() + c->gen_c[a].bytes();
     b += c->gen_n.bytes() + c->gen_start.bytes() + c->gen_ay.bytes() + c->gen_val.bytes();
     for (int a = 0; a < 3; ++a) b += c->disp[a].bytes() + c->work[a].bytes() + c->gen[a].bytes();
@@ -352,6 +401,43 @@ void bind_general(fia_ctx *c, FaceParams &p) {
     p.gen_val = c->gen_val.p;
 }
 
+// The twisted faces' fixed records (kGenStride per face and orientation), and whether the device has
+// memory for them: without, the pieces are counted first, as those of a long list are.
+fia_status fixed_records(fia_ctx *c, int n_twisted, bool &held) {
+    const size_t pairs = 2 * (size_t)n_twisted, most = pairs * kGenStride;
+    hipError_t e = c->gen_n.ensure_slack(pairs);
+    for (int a = 0; a < 3 && e == hipSuccess; ++a) e = c->gen_c[a].ensure_slack(most);
+    if (e == hipSuccess) e = c->gen_ay.ensure_slack(most);
+    if (e == hipSuccess) e = c->gen_val.ensure_slack(most);
+    held = e == hipSuccess;
+    if (e != hipErrorOutOfMemory) {
+        HIP_TRY(e);
+        return FIA_OK;
+    }
+    c->gen_n.release(); c->gen_ay.release(); c->gen_val.release();
+    for (int a = 0; a < 3; ++a) c->gen_c[a].release();
+    return FIA_OK;
+}
+
+// The z stencil tables of pass p, for the grids that take them and where the device has memory for
+// them (32 bytes an entry, 65 a cell): without, piece_kernel evaluates the stencils from their samples.
+fia_status weno_tables(fia_ctx *c, FaceParams &p) {
+    size_t psi_halves = 0;
+    const size_t q_halves = weno_table_halves(p, psi_halves);
+    if (q_halves == 0) return FIA_OK;
+    hipError_t e = c->weno_tab[0].ensure_spare(q_halves);
+    if (e == hipSuccess) e = c->weno_tab[1].ensure_spare(psi_halves);
+    if (e == hipErrorOutOfMemory) {
+        for (auto &t : c->weno_tab) t.release();
+        return FIA_OK;
+    }
+    HIP_TRY(e);
+    HIP_TRY(launch_weno_tables(p, c->weno_tab[0].p, c->weno_tab[1].p, c->stream));
+    p.q_tab = c->weno_tab[0].p;
+    p.psi_tab = c->weno_tab[1].p;
+    return FIA_OK;
+}
+
 fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, FluxSet &fs, const PassSpec &s,
                     int fam_mask, double h) {
     for (int f = 0; f < 3; ++f) {
@@ -443,13 +529,12 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     p.piece_val = c->piece_val.p;
     // twisted faces first: their pieces into kGenStride records per face and orientation, and whether
     // that held them, read back while the kernels below run
-    bool strided = n_twisted > 0 && !p.general_all && (size_t)n_twisted <= kGenListMost;
+    bool strided = false;
+    fia_status st;
+    if (n_twisted > 0 && !p.general_all && (size_t)n_twisted <= kGenListMost &&
+        (st = fixed_records(c, n_twisted, strided)) != FIA_OK)
+        return st;
     if (strided) {
-        const size_t pairs = 2 * (size_t)n_twisted, most = pairs * kGenStride;
-        HIP_TRY(c->gen_n.ensure_slack(pairs));
-        for (int a = 0; a < 3; ++a) HIP_TRY(c->gen_c[a].ensure_slack(most));
-        HIP_TRY(c->gen_ay.ensure_slack(most));
-        HIP_TRY(c->gen_val.ensure_slack(most));
         bind_general(c, p);
         p.gen_stride = kGenStride;
         p.gen_over = c->host_flags + 2;
@@ -464,16 +549,11 @@ fia_status do_faces(fia_ctx *c, const CompGrid &g, const float *q, bool moving, 
     const bool weno_quad = piece_quadrature_mode(p) != 0;
     int sq = -1;
     if (weno_quad) HIP_TRY(span_begin(c, SK_QUAD, sq));
-    size_t psi_halves = 0;
-    const size_t q_halves = weno_table_halves(p, psi_halves);
-    if (q_halves > 0) {
-        HIP_TRY(c->weno_tab[0].ensure(q_halves));
-        HIP_TRY(c->weno_tab[1].ensure(psi_halves));
-        HIP_TRY(launch_weno_tables(p, c->weno_tab[0].p, c->weno_tab[1].p, c->stream));
-        p.q_tab = c->weno_tab[0].p;
-        p.psi_tab = c->weno_tab[1].p;
+    if (!p.fuse_value) {   // fused: the cutters stored the values
+        const TableUse use(c);
+        if ((st = weno_tables(c, p)) != FIA_OK) return st;
+        HIP_TRY(launch_pieces(p, nslots, c->stream));
     }
-    if (!p.fuse_value) HIP_TRY(launch_pieces(p, nslots, c->stream));   // fused: the cutters stored the values
     if (weno_quad) HIP_TRY(span_end(c, sq));
     HIP_TRY(launch_face_sum(p, c->stream));
     if (n_twisted > 0) {
@@ -1104,6 +1184,7 @@ static fia_status ctx_create(int device, hipStream_t stream, fia_ctx **out) {
         (void)hipEventDestroy(c->lists_read);
         drop_stream(); delete c; return FIA_ERR_DEVICE;
     }
+    list_context(c);
     *out = c;
     return FIA_OK;
 }
@@ -1119,6 +1200,7 @@ void *fia_ctx_stream(fia_ctx *c) { return c ? (void *)c->stream : nullptr; }
 
 fia_status fia_ctx_destroy(fia_ctx *c) {
     if (!c) return FIA_OK;
+    unlist_context(c);
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     c->psi.release(); c->twisted.release(); c->degen.release(); c->counters.release(); c->scal.release(); c->bits.release();

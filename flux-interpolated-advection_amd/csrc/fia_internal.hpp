@@ -13,13 +13,33 @@ namespace fia {
 
 struct WenoHalf;   // fia_math.hpp
 
+// Takes back device scratch that the process's contexts hold but can do without: the z stencil
+// tables, of the contexts on the current device whose tables no pass is using.  False if there was none.
+bool give_back_scratch();
+
 // Device buffer that grows on demand (contents are not kept when it grows).
+constexpr size_t kSlackBytes = (size_t)16 << 20;
 template <class T> struct DevBuf {
     T *p = nullptr;
     size_t n = 0;
     bool holds(size_t want) const { return want <= n && p; }
-    // a failure is the caller's to handle, and not left for the check after the next launch
     hipError_t ensure(size_t want) {
+        if (holds(want)) return hipSuccess;
+        hipError_t e = ensure_spare(want);
+        if (e == hipErrorOutOfMemory && give_back_scratch()) e = ensure_spare(want);
+        return e;
+    }
+    // for sizes that follow the data: more than asked when it has to grow (an eighth, at most
+    // kSlackBytes), so that a slightly larger next call does not allocate (and so synchronise) again;
+    // exactly the size asked for where the device has no memory for more
+    hipError_t ensure_slack(size_t want) {
+        if (holds(want)) return hipSuccess;
+        const hipError_t e = ensure_spare(want + std::min(want / 8, kSlackBytes / sizeof(T)));
+        return e == hipErrorOutOfMemory ? ensure(want) : e;
+    }
+    // for scratch that the caller can do without: nothing is taken back for it.  A failure is the
+    // caller's to handle, and not left for the check after the next launch.
+    hipError_t ensure_spare(size_t want) {
         if (holds(want)) return hipSuccess;
         if (p) { hipError_t e = hipFree(p); if (e != hipSuccess) return e; p = nullptr; n = 0; }
         hipError_t e = hipMalloc((void **)&p, std::max<size_t>(want, 1) * sizeof(T));
@@ -31,9 +51,6 @@ template <class T> struct DevBuf {
         }
         return e;
     }
-    // for sizes that follow the data: an eighth more than asked when it has to grow, so that a
-    // slightly larger next call does not allocate (and so synchronise) again
-    hipError_t ensure_slack(size_t want) { return holds(want) ? hipSuccess : ensure(want + want / 8); }
     void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
     size_t bytes() const { return n * sizeof(T); }
 };
