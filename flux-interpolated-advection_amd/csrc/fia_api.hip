@@ -772,13 +772,12 @@ static fia_status pressure_system(fia_ctx *c, const fia_grid3d *g, const GridVie
     return assemble_system(c, g, gv, solid ? c->solid.p : nullptr, c->pcg_b.p, c->pcg_flags.p, pg);
 }
 
-// Whether a Jacobi solve with the device to itself runs the fused sweep.  By default it does: one
-// launch and one pass over the partial sums per iteration instead of two (fused and two-sweep
-// iterations: 32^3 12.9 and 15.2 us, 64^3 12.7 and 16.2, 128^3 26.0 and 36.6, 160^3 42.9 and 59.7,
-// 256^3 137 and 203); a shape tuned for one of the two-sweep update forms keeps it under 4M cells.
-static bool fused_choice(const fia_tuning &t, size_t cells) {
+// Whether a Jacobi solve with the device to itself runs the fused sweep: by default where it is the
+// faster form; a shape tuned for one of the two-sweep update forms keeps it under 4M cells.
+static bool fused_choice(const fia_tuning &t, const PcgGrid &pg) {
     if (t.pcg_fused >= 0) return t.pcg_fused == 1;
-    return t.pcg_recompute < 0 || cells >= ((size_t)1 << 22);
+    return t.pcg_recompute < 0 ? pcg_fused_pays(pg.nx, pg.ny, pg.nz)
+                               : (size_t)pg.nx * pg.ny * pg.nz >= ((size_t)1 << 22);
 }
 
 // Buffers B (allocated here for the grid of pg) bound into a CG state over the system (b, flags).
@@ -790,7 +789,7 @@ static fia_status bind_solve(fia_ctx::PcgBufs &B, const PcgGrid &pg, const doubl
                              PcgState &ps, bool mg, const fia_tuning &tu, bool batched, bool shared) {
     const size_t n = (size_t)pg.nx * pg.ny * pg.nz;
     ps.nblocks = pcg_blocks(n);
-    ps.fused = !mg && !batched && !shared && fused_choice(tu, n);
+    ps.fused = !mg && !batched && !shared && fused_choice(tu, pg);
     pcg_direction_tiling(pg.nx, pg.ny, pg.nz, ps, tu.pcg_chunk_x, tu.pcg_recompute, shared);
     HIP_TRY(B.x.ensure(n)); HIP_TRY(B.r.ensure(n)); HIP_TRY(B.p0.ensure(n)); HIP_TRY(B.p1.ensure(n));
     HIP_TRY(B.part.ensure(pcg_partial_words(ps))); HIP_TRY(B.scal.ensure(kPcgScalars));
@@ -1426,10 +1425,9 @@ fia_status fia_ctx_autotune(fia_ctx *c, const fia_grid3d *g, const uint8_t *soli
     if ((st = time_cg(best, best_cg)) != FIA_OK) return st;
     // a candidate's launches: chunk length, and the q policy of the two-sweep iteration or the
     // fused sweep (Jacobi only)
-    const size_t ncells = (size_t)pg.nx * pg.ny * pg.nz;
     auto launch_key = [&](const fia_tuning &t) {
         PcgState ps;
-        ps.fused = !use_mg && fused_choice(t, ncells);
+        ps.fused = !use_mg && fused_choice(t, pg);
         pcg_direction_tiling(pg.nx, pg.ny, pg.nz, ps, t.pcg_chunk_x, t.pcg_recompute);
         return std::make_pair(ps.dir_chunk_x, ps.fused ? 2 : (int)ps.recompute_q);
     };

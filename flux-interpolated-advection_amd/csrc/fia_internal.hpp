@@ -295,6 +295,8 @@ struct PcgState {
 };
 int pcg_blocks(size_t n);
 int pcg_resident_blocks(bool fused);
+// whether the fused sweep is the faster Jacobi iteration of a solve that has the device to itself
+bool pcg_fused_pays(int nx, int ny, int nz);
 // chunk_x > 0: the x planes one tile sweeps (else one round of the device's resident blocks of
 // st.fused's form, or about 2048 cells per block for a solve sharing the device: shared);
 // recompute 0 / 1: the update streams q / recomputes it (else chosen by grid size and chunk)

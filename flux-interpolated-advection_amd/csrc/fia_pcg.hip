@@ -25,7 +25,8 @@
 // long x chunks (large grids); on small grids, whose chunks are a few planes, the halo planes
 // cost more than q and the streaming form is faster.  Under Jacobi, for a solve that has the
 // device to itself, one kernel per iteration replaces the two (pcg_fused_kernel, below: 35 bytes per cell
-// and iteration), and a geometric multigrid V-cycle can replace the Jacobi preconditioner.
+// and iteration) except on thin boxes (pcg_fused_pays), and a geometric multigrid V-cycle can replace
+// the Jacobi preconditioner.
 //
 // Reductions without fences: every block writes its partial sums with plain stores, and every
 // block of the NEXT kernel sums all partials itself, in block order, before its own work (the
@@ -1590,24 +1591,51 @@ int pcg_resident_blocks(bool fused) {
 // A fused sweep whose vectors stay in the last-level cache (45 bytes a cell) is bound by its blocks'
 // chain of planes, not by memory, and the round need not be full: with 1, 2 or 3 blocks on every CU
 // a sweep of c planes per block took about 10.2 + 2.25 c, 13.4 + 2.85 c and 13.3 + 4.3 c us (grids of
-// 64^3 to 160^3).  The least of the three: 128^3 runs chunks of 4 planes, 512 blocks, in 26.0 us an
+// 64^3 to 160^3; thin boxes the same: 300x300x3 at c = 12 46.0, 1000x100x10 at 14 52.5, 256x256x16 at
+// 8 36.0).  The least of the three: 128^3 runs chunks of 4 planes, 512 blocks, in 26.0 us an
 // iteration against 28.2 for the full round's 3 planes and 29.0 for 256 blocks of 8.  Larger grids
 // are bound by memory and fill the round (256^3).
 constexpr size_t kCachedCells = (size_t)1 << 22;
-static long fused_chunks(int nx, long tiles, int resident) {
+struct FusedPlan {
+    long chunks;   // per tile column
+    double us;     // an iteration by the fit above
+};
+static FusedPlan fused_plan(int nx, long tiles, int resident) {
     constexpr double fixed[3] = {10.2, 13.4, 13.3}, plane[3] = {2.25, 2.85, 4.3};
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        return std::max<long>(1, std::min<long>(nx, resident / tiles));
-    long best = 1;
-    double least = 1e300;
+        return {std::max<long>(1, std::min<long>(nx, resident / tiles)), 0.0};
+    FusedPlan best{1, 1e300};
     for (int k = 1; k <= 3 && k * cus <= resident; ++k) {
         const long chunks = std::max<long>(1, std::min<long>(nx, (long)k * cus / tiles));
         const double t = fixed[k - 1] + plane[k - 1] * (double)((nx + chunks - 1) / chunks);
-        if (t < least) { least = t; best = chunks; }
+        if (t < best.us) best = {chunks, t};
     }
     return best;
+}
+
+// chunks per tile column that fill one round of resident blocks (rounded down: a few blocks over
+// the round would run alone in a second one)
+static long round_chunks(int nx, long tiles, int resident) {
+    return std::max<long>(1, std::min<long>(nx, resident / tiles));
+}
+
+// Whether the fused sweep is the faster Jacobi iteration.  From kCachedCells on both forms are bound
+// by memory and it moves less.  Below, its plane costs the same however few of a tile's 64 x 16
+// columns the grid has, while the two sweeps' cost follows the cells: with a full round of c planes per
+// block and n million cells they took about 12 + 2.2 c + 7.9 n us (64 boxes of 8^3 to 4 M cells,
+// 8^3 and some of one or two planes aside within 10%).  Fused and two sweeps: 128^3 26.5 and 35.5 us,
+// 64^3 13.3 and 15.2, 1024x64x32 36.5 and 41.5, 200x100x50 23.0 and 23.7; 300x300x3 46.0 and 33.5,
+// 600x600x6 125 and 96, 4000x4x4 28.2 and 21.4, 256x256x16 36.0 and 33.2, 97x194x22 22.4 and 20.2.
+bool pcg_fused_pays(int nx, int ny, int nz) {
+    const size_t n = (size_t)nx * ny * nz;
+    const int fused = pcg_resident_blocks(true), two = pcg_resident_blocks(false);
+    if (n >= kCachedCells || fused <= 0 || two <= 0) return true;
+    const long tiles = (long)((ny + kTileY - 1) / kTileY) * ((nz + kTileZ - 1) / kTileZ);
+    const long chunks = round_chunks(nx, tiles, two);
+    const double two_us = 12.0 + 2.2 * (double)((nx + chunks - 1) / chunks) + 7.9e-6 * (double)n;
+    return fused_plan(nx, tiles, fused).us <= two_us;
 }
 
 // Tiling of the tile sweeps: kTileZ x kTileY column tiles, x cut into chunks so that the launch
@@ -1621,11 +1649,9 @@ void pcg_direction_tiling(int nx, int ny, int nz, PcgState &st, int chunk_x, int
     const long tiles = (long)st.dir_tiles_y * st.dir_tiles_z;
     // a solve that shares its launches with others (batched scenes) has no round of its own to fill
     const int resident = shared ? 0 : pcg_resident_blocks(st.fused);
-    // chunks per tile column: as many as fit in one round of resident blocks (rounded down: a few
-    // blocks over the round would run alone in a second one)
     const bool cached = resident > 0 && st.fused && (size_t)nx * ny * nz < kCachedCells;
-    const long want = cached ? fused_chunks(nx, tiles, resident)
-                    : resident > 0 ? std::max<long>(1, std::min<long>(nx, resident / tiles))
+    const long want = cached ? fused_plan(nx, tiles, resident).chunks
+                    : resident > 0 ? round_chunks(nx, tiles, resident)
                                    : std::max<long>(1, std::min<long>(nx, ((long)target_blocks((size_t)nx * ny * nz) +
                                                                            tiles - 1) / tiles));
     st.dir_chunk_x = chunk_x > 0 ? std::min(chunk_x, nx) : (int)((nx + want - 1) / want);

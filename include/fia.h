@@ -269,9 +269,9 @@ typedef struct fia_tuning {
     int pcg_chunk_x;     /* x planes one 64 x 16 CG tile sweeps (0: one block per resident slot) */
     int pcg_recompute;   /* the CG update recomputes q = L p (1) or streams it (0); -1: by size  */
     int pcg_fused;       /* Jacobi: one sweep per CG iteration (1) or the direction and update
-                            sweeps (0); -1: fused, unless pcg_recompute names a two-sweep form
-                            and the grid is under 4M cells.  Multigrid and batched solves use
-                            two sweeps. */
+                            sweeps (0); -1: fused, but under 4M cells on thin boxes, where two
+                            sweeps are faster, or with a pcg_recompute that names a two-sweep
+                            form.  Multigrid and batched solves use two sweeps. */
 } fia_tuning;
 /* The shapes used on grids of nx x ny x nz cells (their staggered velocity components and
  * pressure systems included); nx = ny = nz = 0 sets them for shapes without an entry of their
