@@ -1169,21 +1169,27 @@ FIA_HD void zero_velocity_weno(const FaceParams &P, unsigned row, int i0, int i1
     }
 }
 
-// The value of piece q = (x strip a, z band b) of a face whose strips and bands are given, by the
-// general quadrature or (LINEAR) the non-integral rule of linear and 1Dy_linear psi alone.
-template <bool LINEAR>
+// What a zero-velocity kernel is compiled for: one interpolation's rules, or the non-integral rule of
+// linear and 1Dy_linear psi (kZeroValue); kZeroAny, every rule in one, serves the host only.  On the
+// device it waited at the registers of the rules that it does not run: 256^3, every rule's kernel and a
+// rule's own, linear integral 1,083 and 204 us, WENO6 integral 1,000 and 312, WENO6 with one axis cut
+// 507 and 190.
+constexpr int kZeroAny = -1, kZeroValue = -2;
+
+// The value of piece q = (x strip a, z band b) of a face whose strips and bands are given.
+template <int RULE>
 FIA_HD double zero_velocity_piece(const FaceParams &P, double y, const double xl[2], const double xh[2],
                                   const double zl[2], const double zh[2], int a, int b) {
     const double c3[3] = {0.5 * (xl[a] + xh[a]), y, 0.5 * (zl[b] + zh[b])};
     const double ay = (xh[a] - xl[a]) * (zh[b] - zl[b]);
     int npts = 0;
-    if constexpr (LINEAR) return piece_value_linear(P, c3, ay);
-    else return piece_flux(P, c3, ay, npts);
+    if constexpr (RULE == kZeroValue) return piece_value_linear(P, c3, ay);
+    else return piece_flux<RULE>(P, c3, ay, npts);
 }
 
 // FAST: WENO6 non-integral rule with both axes cut in two (the host decides from the split and the
-// grid's staggering); otherwise the general quadrature per piece.
-template <bool FAST, bool LINEAR = false> FIA_HD void zero_velocity_face_body(const FaceParams &P, long id) {
+// grid's staggering); otherwise RULE's quadrature per piece.
+template <bool FAST, int RULE = kZeroAny> FIA_HD void zero_velocity_face_body(const FaceParams &P, long id) {
     int i, j, k;
     decode_face(P.g, 1, id, i, j, k);
     if constexpr (FAST) return zero_velocity_weno(P, (unsigned)(j * P.g.m[2] + k), i, i + 1);
@@ -1196,14 +1202,14 @@ template <bool FAST, bool LINEAR = false> FIA_HD void zero_velocity_face_body(co
 #pragma unroll 1
     for (int q = 0; q < nx * nz; ++q) {
         const int a = q / nz, b = q - a * nz;   // x strips outer, z bands inner
-        f += zero_velocity_piece<LINEAR>(P, y, xl, xh, zl, zh, a, b);
+        f += zero_velocity_piece<RULE>(P, y, xl, xh, zl, zh, a, b);
     }
     P.flux[1][id] = f;
 }
-template <bool LINEAR> __global__ void __launch_bounds__(kBlock) zero_velocity_face_kernel(FaceParams P) {
+template <int RULE> __global__ void __launch_bounds__(kBlock) zero_velocity_face_kernel(FaceParams P) {
     const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= (long)P.g.faces(1)) return;
-    zero_velocity_face_body<false, LINEAR>(P, id);
+    zero_velocity_face_body<false, RULE>(P, id);
 }
 // One row of a chunk of x planes per thread (VALU bound; 256^3: 690 us with a thread per face, 161 so).
 __global__ void __launch_bounds__(kBlock) zero_velocity_weno_kernel(FaceParams P, int chunk) {
@@ -2240,9 +2246,15 @@ hipError_t launch_zero_velocity_faces(const FaceParams &p, hipStream_t s) {
                            dim3((unsigned)rows, (unsigned)(((size_t)p.g.m[0] + chunk - 1) / chunk)), dim3(b), 0, s, p,
                            (int)chunk);
     } else if (p.fuse_value) {   // linear or 1Dy_linear psi, not integral
-        hipLaunchKernelGGL(zero_velocity_face_kernel<true>, grid, dim3(b), 0, s, p);
+        hipLaunchKernelGGL(zero_velocity_face_kernel<kZeroValue>, grid, dim3(b), 0, s, p);
     } else {
-        hipLaunchKernelGGL(zero_velocity_face_kernel<false>, grid, dim3(b), 0, s, p);
+        switch (p.interp == IM_WENO6 && p.weno_opt ? (int)IM_WENO6_OPT : p.interp) {
+        case IM_LINEAR: hipLaunchKernelGGL(zero_velocity_face_kernel<IM_LINEAR>, grid, dim3(b), 0, s, p); break;
+        case IM_WENO6: hipLaunchKernelGGL(zero_velocity_face_kernel<IM_WENO6>, grid, dim3(b), 0, s, p); break;
+        case IM_1DY_LINEAR: hipLaunchKernelGGL(zero_velocity_face_kernel<IM_1DY_LINEAR>, grid, dim3(b), 0, s, p); break;
+        case IM_1DY_WENO6: hipLaunchKernelGGL(zero_velocity_face_kernel<IM_1DY_WENO6>, grid, dim3(b), 0, s, p); break;
+        default: hipLaunchKernelGGL(zero_velocity_face_kernel<IM_WENO6_OPT>, grid, dim3(b), 0, s, p); break;
+        }
     }
     return hipGetLastError();
 }
