@@ -1511,13 +1511,11 @@ FIA_HD void degenerate_pieces(const FaceParams &P, int t, int first, int step) {
     }
 }
 FIA_HD void degenerate_body(const FaceParams &P, int t) { degenerate_pieces(P, t, 0, 1); }
-// kFaceLanes lanes share a face's pieces (most have two to six; the list is short, so the kernel is
-// one face's latency long)
-constexpr int kFaceLanes = 8;
-__global__ void __launch_bounds__(64) degenerate_kernel(FaceParams P) {
-    const int count = *P.degen_count;
-    for (int t = (blockIdx.x * blockDim.x + threadIdx.x) / kFaceLanes; t < count; t += gridDim.x * blockDim.x / kFaceLanes)
-        degenerate_pieces(P, t, (int)threadIdx.x % kFaceLanes, kFaceLanes);
+// 2^share lanes share a face's pieces.
+__global__ void __launch_bounds__(64) degenerate_kernel(FaceParams P, int share) {
+    const int count = *P.degen_count, lanes = 1 << share, first = (int)threadIdx.x & (lanes - 1);
+    for (int t = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> share); t < count; t += (int)(gridDim.x * blockDim.x >> share))
+        degenerate_pieces(P, t, first, lanes);
 }
 // With fuse_value (no quadrature launch): the values of the degenerate faces' pieces from the
 // records degenerate_kernel stored.
@@ -2259,9 +2257,10 @@ hipError_t launch_zero_velocity_faces(const FaceParams &p, hipStream_t s) {
     return hipGetLastError();
 }
 
-// grid-stride kernels over a face list of `count` faces: one 64-lane block per 64 faces, at most
-// 1024 blocks (one wave per SIMD at these kernels' register counts)
-static unsigned list_blocks(int count) { return (unsigned)std::min(1024, (count + 63) / 64); }
+// grid-stride kernels over a face list: one 64-lane block per 64 of `count` lanes, at most kListBlocks
+// (one wave per SIMD at these kernels' register counts)
+constexpr int kListBlocks = 1024;
+static unsigned list_blocks(int count) { return (unsigned)std::min(kListBlocks, count / 64 + (count % 64 != 0)); }
 
 hipError_t launch_seg_faces(const FaceParams &p, hipStream_t s) {
     const int b = block_or_default(p.face_block);
@@ -2275,10 +2274,19 @@ hipError_t launch_seg_faces(const FaceParams &p, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Lanes a degenerate face's pieces are shared over: eight while that leaves each lane one face (most
+// have two to six pieces, and a short list is one face's latency long), fewer on longer lists, whose
+// lanes without a piece only take up the machine (8, 4, 2 and 1 lanes: 2,141 faces 22, 28, 36 and 52 us,
+// 14,787 35, 27, 35 and 49, 33,288 82, 62, 48 and 61, 131,863 170, 110, 97 and 94).
+static int face_share(int count) {
+    int share = 3;
+    while (share > 0 && ((long)count << share) > (long)kListBlocks * 64) --share;
+    return share;
+}
 hipError_t launch_faces_degenerate(const FaceParams &p, int count, hipStream_t s) {
     if (count <= 0) return hipSuccess;
-    hipLaunchKernelGGL(degenerate_kernel, dim3(list_blocks((int)std::min<long>((long)count * kFaceLanes, INT32_MAX - 63))),
-                       dim3(64), 0, s, p);
+    const int share = face_share(count);
+    hipLaunchKernelGGL(degenerate_kernel, dim3(list_blocks(count << share)), dim3(64), 0, s, p, share);
     if (p.fuse_value) hipLaunchKernelGGL(degenerate_value_kernel, dim3(list_blocks(count)), dim3(64), 0, s, p);
     return hipGetLastError();
 }
