@@ -2228,18 +2228,25 @@ static bool zero_velocity_cuts_both(const FaceParams &p) {
     return cx && cz && fx != floor(fx) && fz != floor(fz);
 }
 
+// x planes per thread of zero_velocity_weno_kernel, for rows of a plane in blocks of b: a chunk repeats
+// six columns, so long ones where the chip stays full (256^3 with 32 and 64 planes: 161 and 185 us;
+// 128^3 with 4 and 8: 40 and 36), four on 75x96x50 (13 us, 15 with 8 and 22 with one) and one where four
+// leave CUs idle (32^3: 8 and 11).  The chunks are the launch's gridDim.y, at most kMostGridY of them.
+constexpr size_t kMostGridY = 65535;
+static size_t zero_velocity_chunk(const CompGrid &g, int b) {
+    const size_t planes = (size_t)g.m[0], rows = grid_for((size_t)(g.m[1] + 1) * g.m[2], b);
+    const size_t all = rows * planes * b / kBlock;
+    const size_t chunk = std::min<size_t>(std::max<size_t>({all / 1024, std::min<size_t>(4, all / 256), (size_t)1}), 32);
+    return std::max(chunk, (planes + kMostGridY - 1) / kMostGridY);
+}
+
 hipError_t launch_zero_velocity_faces(const FaceParams &p, hipStream_t s) {
     const int b = block_or_default(p.face_block);
     const dim3 grid(grid_for(p.g.faces(1), b));
     // (the closed form's shared stencils are the WENO6 rule's; "WENO6-optimized" takes the
     // general quadrature per piece)
     if (p.interp == IM_WENO6 && !p.weno_opt && !p.integral && zero_velocity_cuts_both(p)) {
-        // planes per thread: a chunk repeats five or six columns, so long ones where the chip stays
-        // full (256^3 with 32 and 64 planes: 161 and 185 us; 128^3 with 4 and 8: 40 and 36), four on
-        // 75x96x50 (13 us, 15 with 8 and 22 with one) and one where four leave CUs idle (32^3: 8 and 11)
-        const size_t rows = grid_for((size_t)(p.g.m[1] + 1) * p.g.m[2], b), all = rows * p.g.m[0] * b / kBlock;
-        const size_t chunk = std::min<size_t>(
-            std::max<size_t>({all / 1024, std::min<size_t>(4, all / 256), (size_t)1}), 32);
+        const size_t chunk = zero_velocity_chunk(p.g, b), rows = grid_for((size_t)(p.g.m[1] + 1) * p.g.m[2], b);
         hipLaunchKernelGGL(zero_velocity_weno_kernel,
                            dim3((unsigned)rows, (unsigned)(((size_t)p.g.m[0] + chunk - 1) / chunk)), dim3(b), 0, s, p,
                            (int)chunk);
