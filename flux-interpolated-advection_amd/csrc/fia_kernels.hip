@@ -353,86 +353,111 @@ template <int METHOD> __global__ void __launch_bounds__(kBlock) vertex_kernel(Ve
 // pass.  One component per blockIdx.y; 256^3, three components: 1,027 -> 250 us (cell
 // lattice), 1,594 -> 244 (face components).
 constexpr int kVtxTile = 16;
+// Thread tid of the block of tile blk (x chunk, y tile, z tile) and component comp: its column of
+// lattice vertices (j, k), planes i0 .. i1 - 1, and where their passes read.
+struct VertexMarch {
+    int comp, i0, i1, j, k, m[3], base[3];
+    bool half[3], zy, second;   // z passes then y passes; the thread also takes one of the last five rows
+    // offsets in a plane of the six samples of this thread's z pass (row j0 + y - 2 if the y pass
+    // follows, row j otherwise) or, with z on a sample, of its y pass (or of its one sample); step: from
+    // there to the tile's last five rows of z passes
+    unsigned off[6], step;
+    int planes, first;
+    FIA_HD VertexMarch(const VertexParams &P, int comp_, int blk, int tiles_y, int tiles_z, int chunk, int tid) {
+        comp = comp_;
+        const int z = tid % kVtxTile, y = tid / kVtxTile;
+        const int bz = blk % tiles_z, by = (blk / tiles_z) % tiles_y, bx = blk / (tiles_z * tiles_y);
+        const int j0 = by * kVtxTile;
+        i0 = bx * chunk; i1 = min_of(P.g.m[0] + 1, i0 + chunk); j = j0 + y; k = bz * kVtxTile + z;
+        // sample coordinate of lattice index l along axis a: l + base_a, plus a half if half_a
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const int e = P.g.e[a], o = a != comp;
+            m[a] = P.g.n[a] + (a == comp);
+            half[a] = (e + o) & 1;
+            base[a] = -((e + o + 1) >> 1);
+        }
+        zy = half[2] && half[1];
+        const int jr = (zy ? j0 + y - 2 : j) + base[1], kz = k + base[2];
+        const unsigned mz = (unsigned)m[2], row = (unsigned)clampi(jr, 0, m[1] - 1) * mz;
+#pragma unroll
+        for (int r = 0; r < 6; ++r)
+            off[r] = half[2] ? row + (unsigned)clampi(kz - 2 + r, 0, m[2] - 1)
+                             : (unsigned)clampi(half[1] ? jr - 2 + r : jr, 0, m[1] - 1) * mz +
+                                   (unsigned)clampi(kz, 0, m[2] - 1);
+        second = zy && y < 5;
+        step = (unsigned)clampi(jr + kVtxTile, 0, m[1] - 1) * mz - row;
+        planes = i1 - i0 + (half[0] ? 5 : 0);
+        first = i0 + base[0] - (half[0] ? 2 : 0);
+    }
+    FIA_HD const float *plane(const VertexParams &P, int p) const {
+        const float *F = comp == 0 ? P.u : (comp == 1 ? P.v : P.w);
+        return F + (size_t)clampi(first + p, 0, m[0] - 1) * m[1] * m[2];
+    }
+    // the pass over this thread's six samples of a plane, `shift` further on
+    FIA_HD float pass(const float *__restrict__ plane, unsigned shift, const WenoCoef &wc) const {
+        float f[6];
+#pragma unroll
+        for (int r = 0; r < 6; ++r) f[r] = plane[off[r] + shift];
+        return weno6<float>(f, wc);
+    }
+    // the y pass over the tile's rows of z passes
+    FIA_HD static float rows_pass(const float *rows, int tid, const WenoCoef &wc) {
+        float f[6];
+#pragma unroll
+        for (int r = 0; r < 6; ++r) f[r] = rows[tid + r * kVtxTile];
+        return weno6<float>(f, wc);
+    }
+    // the x pass over the thread's last six values, of plane p; false while there are fewer
+    FIA_HD bool x_pass(float (&yv)[6], int p, float &v, const WenoCoef &wc) const {
+        if (!half[0]) return true;
+#pragma unroll
+        for (int r = 0; r < 5; ++r) yv[r] = yv[r + 1];
+        yv[5] = v;
+        if (p < 5) return false;
+        v = weno6<float>(yv, wc);
+        return true;
+    }
+    FIA_HD void store(const VertexParams &P, int p, float v) const {
+        const int ly = P.g.m[1] + 1, lz = P.g.m[2] + 1, i = i0 + p - (half[0] ? 5 : 0);
+        if (j >= ly || k >= lz) return;
+        float *__restrict__ out = P.disp[0];
+        if (comp == 1) out = P.disp[1];
+        if (comp == 2) out = P.disp[2];
+        const int lat[3] = {i, j, k};
+        float d = -P.dt_over_h * v;
+        double pos = 0.0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if (a == P.g.comp && (lat[a] <= 1 || lat[a] >= P.g.n[a])) d = 0.0f;
+            if (a == comp) pos = lat[a] - 0.5 * P.g.e[a];
+        }
+        out[idx3(i, j, k, ly, lz)] = clamp_displacement(P.g, comp, pos, d);
+    }
+};
 __global__ void __launch_bounds__(kVtxTile * kVtxTile) vertex_weno_kernel(VertexParams P, int tiles_y, int tiles_z,
                                                                           int chunk) {
     __shared__ float zs[2][(kVtxTile + 5) * kVtxTile];
-    const int comp = blockIdx.y, tid = threadIdx.x, z = tid % kVtxTile, y = tid / kVtxTile;
-    const int bz = blockIdx.x % tiles_z, by = (blockIdx.x / tiles_z) % tiles_y, bx = blockIdx.x / (tiles_z * tiles_y);
-    const int lx = P.g.m[0] + 1, ly = P.g.m[1] + 1, lz = P.g.m[2] + 1;
-    const int i0 = bx * chunk, i1 = min(lx, i0 + chunk), j0 = by * kVtxTile, j = j0 + y, k = bz * kVtxTile + z;
-    const float *__restrict__ F = comp == 0 ? P.u : (comp == 1 ? P.v : P.w);
-    float *__restrict__ out = P.disp[0];
-    if (comp == 1) out = P.disp[1];
-    if (comp == 2) out = P.disp[2];
-    // sample coordinate of lattice index l along axis a: l + base_a, plus a half if half_a
-    int m[3], base[3];
-    bool half[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const int e = P.g.e[a], o = a != comp;
-        m[a] = P.g.n[a] + (a == comp);
-        half[a] = (e + o) & 1;
-        base[a] = -((e + o + 1) >> 1);
-    }
+    const int tid = threadIdx.x;
+    const VertexMarch t(P, blockIdx.y, blockIdx.x, tiles_y, tiles_z, chunk, tid);
     const WenoCoef wc(0.5f, 1.0f);
-    // offsets in a plane of the six samples of this thread's z pass (row j0 + y - 2 if the y pass
-    // follows, row j otherwise) or, with z on a sample, of its y pass (or of its one sample)
-    const bool zy = half[2] && half[1];
-    const int jr = (zy ? j0 + y - 2 : j) + base[1], kz = k + base[2];
-    const unsigned mz = (unsigned)m[2], row = (unsigned)clampi(jr, 0, m[1] - 1) * mz;
-    unsigned off[6];
-#pragma unroll
-    for (int r = 0; r < 6; ++r)
-        off[r] = half[2] ? row + (unsigned)clampi(kz - 2 + r, 0, m[2] - 1)
-                         : (unsigned)clampi(half[1] ? jr - 2 + r : jr, 0, m[1] - 1) * mz +
-                               (unsigned)clampi(kz, 0, m[2] - 1);
-    // the tile's last five rows of z passes
-    const bool second = zy && y < 5;
-    const unsigned step = (unsigned)clampi(jr + kVtxTile, 0, m[1] - 1) * mz - row;
-    const int planes = i1 - i0 + (half[0] ? 5 : 0), first = i0 + base[0] - (half[0] ? 2 : 0);
     float yv[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (int p = 0; p < planes; ++p) {
-        const float *__restrict__ plane = F + (size_t)clampi(first + p, 0, m[0] - 1) * m[1] * m[2];
-        float f[6], v;
-        if (half[2] || half[1]) {
-#pragma unroll
-            for (int r = 0; r < 6; ++r) f[r] = plane[off[r]];
-            v = weno6<float>(f, wc);
-            if (zy) {
+    for (int p = 0; p < t.planes; ++p) {
+        const float *__restrict__ plane = t.plane(P, p);
+        float v;
+        if (t.half[2] || t.half[1]) {
+            v = t.pass(plane, 0u, wc);
+            if (t.zy) {
                 float *rows = zs[p & 1];
                 rows[tid] = v;
-                if (second) {
-#pragma unroll
-                    for (int r = 0; r < 6; ++r) f[r] = plane[off[r] + step];
-                    rows[tid + kVtxTile * kVtxTile] = weno6<float>(f, wc);
-                }
+                if (t.second) rows[tid + kVtxTile * kVtxTile] = t.pass(plane, t.step, wc);
                 __syncthreads();
-#pragma unroll
-                for (int r = 0; r < 6; ++r) f[r] = rows[tid + r * kVtxTile];
-                v = weno6<float>(f, wc);
+                v = VertexMarch::rows_pass(rows, tid, wc);
             }
         } else {
-            v = plane[off[0]];
+            v = plane[t.off[0]];
         }
-        if (half[0]) {
-#pragma unroll
-            for (int r = 0; r < 5; ++r) yv[r] = yv[r + 1];
-            yv[5] = v;
-            if (p < 5) continue;
-            v = weno6<float>(yv, wc);
-        }
-        const int i = i0 + p - (half[0] ? 5 : 0);
-        if (j < ly && k < lz) {
-            const int lat[3] = {i, j, k};
-            float d = -P.dt_over_h * v;
-            double pos = 0.0;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                if (a == P.g.comp && (lat[a] <= 1 || lat[a] >= P.g.n[a])) d = 0.0f;
-                if (a == comp) pos = lat[a] - 0.5 * P.g.e[a];
-            }
-            out[idx3(i, j, k, ly, lz)] = clamp_displacement(P.g, comp, pos, d);
-        }
+        if (t.x_pass(yv, p, v, wc)) t.store(P, p, v);
     }
 }
 
@@ -1299,57 +1324,124 @@ struct Bricks {
     }
     size_t count() const { return (size_t)n[0] * n[1] * n[2]; }
 };
-template <bool OPT>
-__global__ void __launch_bounds__(kBrickThreads) piece_brick_kernel(FaceParams P, Bricks br) {
-    __shared__ WenoHalf win[kWinX * kWinY * 2 * kWinZ];
-    __shared__ unsigned long long row_start[kBrickRows];
-    __shared__ unsigned row_end[kBrickRows];   // lengths, then the inclusive prefix of them
-    __shared__ int box[6];                     // least bx, J, bz and greatest
-    // workgroups go to the 8 XCDs in turn: each XCD takes one contiguous eighth of the bricks
-    const int per = (int)(gridDim.x / 8), count = br.n[0] * br.n[1] * br.n[2];
-    const int brick = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if (brick >= count) return;
-    const int tid = threadIdx.x, lane = tid & 63;
-    // the brick's cells [lo, hi) on each axis; the last brick also takes the faces past the last cell
-    const int bi[3] = {brick / (br.n[2] * br.n[1]), brick / br.n[2] % br.n[1], brick % br.n[2]};
-    constexpr int size[3] = {kBrickX, kBrickY, kBrickZ};
+// The brick's cells [lo, hi) on each axis; the last brick of an axis also takes the faces past its
+// last cell.
+struct BrickCells {
     int lo[3], hi[3];
+    bool end[3];
+    FIA_HD BrickCells(const CompGrid &g, const Bricks &br, int brick) {
+        const int bi[3] = {brick / (br.n[2] * br.n[1]), brick / br.n[2] % br.n[1], brick % br.n[2]};
+        constexpr int size[3] = {kBrickX, kBrickY, kBrickZ};
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        lo[a] = bi[a] * size[a];
-        hi[a] = min(lo[a] + size[a], P.g.m[a]);
-    }
-    int rows = 0;
-#pragma unroll
-    for (int fam = 0; fam < 3; ++fam) {
-        int end[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) end[a] = hi[a] + (fam == a && bi[a] == br.n[a] - 1 ? 1 : 0);
-        const int ny = end[1] - lo[1], n = (end[0] - lo[0]) * ny, t = tid - rows;
-        if (t >= 0 && t < n) {
-            const int i = lo[0] + t / ny, j = lo[1] + t % ny;
-            const size_t first = P.fam_base[fam] + ((size_t)i * P.g.fy[fam].d + j) * P.g.fz[fam].d + lo[2];
-            const size_t last = first + (size_t)(end[2] - lo[2]) - 1;
-            const unsigned long long s0 = P.face_start[first];
-            row_start[tid] = s0;
-            row_end[tid] = (unsigned)(P.face_start[last] + P.face_n[last] - s0);
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = bi[a] * size[a];
+            hi[a] = min_of(lo[a] + size[a], g.m[a]);
+            end[a] = bi[a] == br.n[a] - 1;
         }
-        rows += n;
     }
-    if (tid < 6) box[tid] = tid < 3 ? INT32_MAX : INT32_MIN;
-    // the moved vertices' bases (x, z: floor(p - (0.5 - e/2)); y: the level floor(p + e/2))
-    int least[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, most[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
-    const int vy = hi[1] - lo[1] + 1, vz = hi[2] - lo[2] + 1;
-    for (int t = tid; t < (hi[0] - lo[0] + 1) * vy * vz; t += kBrickThreads) {
+    // the rows of the brick's faces, (x, y) of each family in turn; row t's slots into start and len
+    FIA_HD int rows(const FaceParams &P, int t, unsigned long long &start, unsigned &len) const {
+        int rows = 0;
+#pragma unroll
+        for (int fam = 0; fam < 3; ++fam) {
+            int to[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) to[a] = hi[a] + (fam == a && end[a] ? 1 : 0);
+            const int ny = to[1] - lo[1], n = (to[0] - lo[0]) * ny, u = t - rows;
+            if (u >= 0 && u < n) {
+                const int i = lo[0] + u / ny, j = lo[1] + u % ny;
+                const size_t first = P.fam_base[fam] + ((size_t)i * P.g.fy[fam].d + j) * P.g.fz[fam].d + lo[2];
+                const size_t last = first + (size_t)(to[2] - lo[2]) - 1;
+                const unsigned long long s0 = P.face_start[first];
+                start = s0;
+                len = (unsigned)(P.face_start[last] + P.face_n[last] - s0);
+            }
+            rows += n;
+        }
+        return rows;
+    }
+    // moved vertex t's sample bases (x, z: floor(p - (0.5 - e/2)); y: the level floor(p + e/2))
+    FIA_HD int vertices() const { return (hi[0] - lo[0] + 1) * (hi[1] - lo[1] + 1) * (hi[2] - lo[2] + 1); }
+    FIA_HD void bases(const FaceParams &P, int t, int (&c)[3]) const {
+        const int vy = hi[1] - lo[1] + 1, vz = hi[2] - lo[2] + 1;
         const int k = t % vz, j = t / vz % vy, i = t / (vz * vy);
         const int lat[3] = {lo[0] + i, lo[1] + j, lo[2] + k};
         const size_t v = idx3(lat[0], lat[1], lat[2], P.g.m[1] + 1, P.g.m[2] + 1);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const float p = (float)lat[a] + (P.disp[a] ? P.disp[a][v] : 0.0f) - (a == 1 ? 0.0f : 0.5f);
-            const int c = floor_index((double)p);
-            least[a] = min(least[a], c);
-            most[a] = max(most[a], c);
+            c[a] = floor_index((double)p);
+        }
+    }
+};
+// The staged box of q's table, from the least and greatest bases (x, J, z): columns bx - 2 .. bx + 3,
+// rows J - 3 .. J + 3 and the z entries of the bases, or the middle of them.
+struct BrickBox {
+    int wx, wy, wz, nx, ny, nz;
+    FIA_HD BrickBox(const int (&range)[6], int mz) {
+        wx = middle(range[0] - 2, range[3] + 3, kWinX, nx);
+        wy = middle(range[1] - 3, range[4] + 3, kWinY, ny);
+        wz = middle(weno_entry_index(range[2], mz), weno_entry_index(range[5], mz), kWinZ, nz);
+    }
+    FIA_HD static int middle(int from, int to, int cap, int &n) {
+        n = min_of(to - from + 1, cap);
+        return from + (to - from + 1 - n) / 2;
+    }
+    // half entry t of the box, in kWinZ steps per (column, row, half): where it goes and comes from
+    FIA_HD int halves() const { return nx * ny * 2 * kWinZ; }
+    FIA_HD bool half_entry(const CompGrid &g, int t, int &to, size_t &from) const {
+        const int e = t % kWinZ, hr = t / kWinZ, half = hr & 1, row = hr >> 1;
+        const int x = row / ny, y = row - x * ny;
+        if (e >= nz) return false;
+        const size_t src = ((size_t)clampi(wx + x, 0, g.m[0] - 1) * g.m[1] + clampi(wy + y, 0, g.m[1] - 1)) * 2 + half;
+        to = ((x * kWinY + y) * 2 + half) * kWinZ + e;
+        from = src * (size_t)(g.m[2] + kWenoPad) + wz + e;
+        return true;
+    }
+    // the first of a piece's entries in the box (entry (ix, iy) is (ix kWinY + iy) 2 kWinZ further on),
+    // or -1 where not all of them are
+    FIA_HD int corner(const PiecePoint &t, int mz) const {
+        const int dx = t.bx - 2 - wx, dy = t.J - 3 - wy, dz = weno_entry_index(t.bz, mz) - wz;
+        const bool in = dx >= 0 && dx + 5 < nx && dy >= 0 && dy + 6 < ny && dz >= 0 && dz < nz;
+        return in ? (dx * kWinY + dy) * 2 * kWinZ + dz : -1;
+    }
+};
+// a piece's flux with q's entries read from the box at `at` (BrickBox::corner)
+template <bool OPT>
+FIA_HD double piece_flux_box(const FaceParams &P, const PiecePoint &t, double ay, const WenoHalf *at) {
+    return piece_flux_at<OPT>(P, t, ay, [&](int ix, int iy) {
+        const WenoHalf *e = at + (ix * kWinY + iy) * 2 * kWinZ;
+        return WenoEntry{e[0], e[kWinZ]};
+    });
+}
+template <bool OPT>
+__global__ void __launch_bounds__(kBrickThreads) piece_brick_kernel(FaceParams P, Bricks br) {
+    __shared__ WenoHalf win[kWinX * kWinY * 2 * kWinZ];
+    __shared__ unsigned long long row_start[kBrickRows];
+    __shared__ unsigned row_end[kBrickRows];   // lengths, then the inclusive prefix of them
+    __shared__ int range[6];                   // least bx, J, bz and greatest
+    // workgroups go to the 8 XCDs in turn: each XCD takes one contiguous eighth of the bricks
+    const int per = (int)(gridDim.x / 8), count = br.n[0] * br.n[1] * br.n[2];
+    const int brick = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (brick >= count) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const BrickCells cells(P.g, br, brick);
+    unsigned long long start = 0;
+    unsigned len = 0;
+    const int rows = cells.rows(P, tid, start, len);
+    if (tid < rows) {
+        row_start[tid] = start;
+        row_end[tid] = len;
+    }
+    if (tid < 6) range[tid] = tid < 3 ? INT32_MAX : INT32_MIN;
+    int least[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, most[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
+    for (int t = tid; t < cells.vertices(); t += kBrickThreads) {
+        int c[3];
+        cells.bases(P, t, c);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            least[a] = min(least[a], c[a]);
+            most[a] = max(most[a], c[a]);
         }
     }
 #pragma unroll
@@ -1363,8 +1455,8 @@ __global__ void __launch_bounds__(kBrickThreads) piece_brick_kernel(FaceParams P
     if (lane == 0) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            atomicMin(&box[a], least[a]);
-            atomicMax(&box[3 + a], most[a]);
+            atomicMin(&range[a], least[a]);
+            atomicMax(&range[3 + a], most[a]);
         }
     }
     if (tid < 64) {   // one wave scans the rows' lengths
@@ -1383,21 +1475,12 @@ __global__ void __launch_bounds__(kBrickThreads) piece_brick_kernel(FaceParams P
         }
     }
     __syncthreads();
-    const int mx = P.g.m[0], my = P.g.m[1], mz = P.g.m[2], len = mz + kWenoPad;
-    // the box: columns bx - 2 .. bx + 3, rows J - 3 .. J + 3, z entries of the bases
-    const auto middle = [](int from, int to, int cap, int &n) {
-        n = min(to - from + 1, cap);
-        return from + (to - from + 1 - n) / 2;
-    };
-    int nx, ny, nz;
-    const int wx = middle(box[0] - 2, box[3] + 3, kWinX, nx), wy = middle(box[1] - 3, box[4] + 3, kWinY, ny);
-    const int wz = middle(weno_entry_index(box[2], mz), weno_entry_index(box[5], mz), kWinZ, nz);
-    for (int t = tid; t < nx * ny * 2 * kWinZ; t += kBrickThreads) {
-        const int e = t % kWinZ, hr = t / kWinZ, half = hr & 1, row = hr >> 1;
-        const int x = row / ny, y = row - x * ny;
-        if (e >= nz) continue;
-        const size_t src = ((size_t)clampi(wx + x, 0, mx - 1) * my + clampi(wy + y, 0, my - 1)) * 2 + half;
-        win[((x * kWinY + y) * 2 + half) * kWinZ + e] = P.q_tab[src * len + wz + e];
+    const int mz = P.g.m[2];
+    const BrickBox box(range, mz);
+    for (int t = tid; t < box.halves(); t += kBrickThreads) {
+        int to;
+        size_t from;
+        if (box.half_entry(P.g, t, to, from)) win[to] = P.q_tab[from];
     }
     __syncthreads();
     const unsigned total = row_end[rows - 1];
@@ -1419,16 +1502,8 @@ __global__ void __launch_bounds__(kBrickThreads) piece_brick_kernel(FaceParams P
         if (ay != 0.0) {
             const double c3[3] = {P.piece_c[0][q], P.piece_c[1][q], P.piece_c[2][q]};
             const PiecePoint t = piece_point<OPT>(P, c3);
-            const int dx = t.bx - 2 - wx, dy = t.J - 3 - wy, dz = weno_entry_index(t.bz, mz) - wz;
-            if (dx >= 0 && dx + 5 < nx && dy >= 0 && dy + 6 < ny && dz >= 0 && dz < nz) {
-                const WenoHalf *at = win + (dx * kWinY + dy) * 2 * kWinZ + dz;
-                val = piece_flux_at<OPT>(P, t, ay, [&](int ix, int iy) {
-                    const WenoHalf *e = at + (ix * kWinY + iy) * 2 * kWinZ;
-                    return WenoEntry{e[0], e[kWinZ]};
-                });
-            } else {
-                val = piece_flux_memory<OPT>(P, t, ay);
-            }
+            const int at = box.corner(t, mz);
+            val = at >= 0 ? piece_flux_box<OPT>(P, t, ay, win + at) : piece_flux_memory<OPT>(P, t, ay);
             npieces += 1; npts += piece_points(t.f); nevals += piece_evals(t.f);
         }
         P.piece_val[q] = val;
@@ -1924,18 +1999,25 @@ hipError_t launch_psi(const PsiParams &p, hipStream_t s) {
 // and 8,192 blocks: 272, 250 and 243 us, 128^3 with 4,096 and 8,192: 48 and 52; at least 2, 4 and 8
 // planes on 75x96x50: 18, 17 and 21 us).
 constexpr unsigned kVtxBlocks = 4096;
+struct VertexTiles {
+    int ty, tz;
+    size_t chunk, blocks;   // per component
+    explicit VertexTiles(const CompGrid &g) {
+        const size_t lx = (size_t)g.m[0] + 1;
+        ty = (g.m[1] + kVtxTile) / kVtxTile;
+        tz = (g.m[2] + kVtxTile) / kVtxTile;
+        const size_t tiles = (size_t)ty * tz;
+        chunk = std::min<size_t>(std::max<size_t>(lx * tiles * 3 / kVtxBlocks, 4), 64);
+        blocks = tiles * ((lx + chunk - 1) / chunk);
+    }
+};
 
 hipError_t launch_vertices(const VertexParams &p, hipStream_t s) {
-    const int lx = p.g.m[0] + 1, ly = p.g.m[1] + 1, lz = p.g.m[2] + 1;
     // in-plane byte offsets of the WENO6 kernel are 32 bits
-    if (p.interp == IM_WENO6 && (size_t)ly * lz < ((size_t)1 << 29)) {
-        const int ty = (ly + kVtxTile - 1) / kVtxTile, tz = (lz + kVtxTile - 1) / kVtxTile;
-        const size_t tiles = (size_t)ty * tz;
-        size_t chunk = (size_t)lx * tiles * 3 / kVtxBlocks;
-        chunk = std::min<size_t>(std::max<size_t>(chunk, 4), 64);
-        const size_t blocks = tiles * (((size_t)lx + chunk - 1) / chunk);
-        hipLaunchKernelGGL(vertex_weno_kernel, dim3((unsigned)blocks, 3), dim3(kVtxTile * kVtxTile), 0, s, p, ty, tz,
-                           (int)chunk);
+    if (p.interp == IM_WENO6 && (size_t)(p.g.m[1] + 1) * (p.g.m[2] + 1) < ((size_t)1 << 29)) {
+        const VertexTiles t(p.g);
+        hipLaunchKernelGGL(vertex_weno_kernel, dim3((unsigned)t.blocks, 3), dim3(kVtxTile * kVtxTile), 0, s, p, t.ty, t.tz,
+                           (int)t.chunk);
         return hipGetLastError();
     }
     const dim3 grid(grid_for(p.g.lattice(), kBlock));

@@ -26,6 +26,7 @@
 namespace fia {
 
 FIA_HD int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
+FIA_HD int min_of(int a, int b) { return a < b ? a : b; }
 FIA_HD size_t idx3(int i, int j, int k, int my, int mz) { return ((size_t)i * my + j) * mz + k; }
 
 FIA_HD float fast_rcp(float x) {

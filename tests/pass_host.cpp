@@ -1,6 +1,8 @@
 // Host replay of the library's flux passes: the __host__ __device__ kernel bodies of
 // flux-interpolated-advection_amd/csrc/fia_kernels.hip (the same source the GPU build compiles),
-// driven over host arrays in the order fia_api.hip launches them, on host threads.
+// driven over host arrays in the order fia_api.hip launches them, on host threads.  One form for every
+// size: vertices and undeformed faces one by one, the quadrature from the stencils' samples, twisted
+// faces counted first; tests/forms_host.cpp replays the forms that the launchers choose.
 //
 // The replay context mirrors fia_ctx's device scratch: buffers only grow, their contents are not
 // kept when they grow, and nothing is cleared between calls.  New memory is filled with 0xFF bytes
