@@ -319,7 +319,11 @@ struct MgLevel {
     float *dense;     // the coarsest level: its sweeps as a matrix, column e at dense + e cells
 };
 constexpr int kMgCoarsestCells = 256;   // most cells of the coarsest level
-constexpr int kMgTailCells = 5120;      // most cells of the tail's smoothed levels together
+// Most cells of the tail's smoothed levels together: two to a thread of its block.  Larger levels take
+// one CU longer than their own launches (cut-offs of 256, 1,024, 2,048 and 5,120 cells, the last what
+// LDS holds; us an iteration: 32^3 55.7 52.4 52.3 55.3, 50x77x64 63.6 59.8 59.7 63.5, 96^3 93.8 93.7 91.6
+// 91.7, 128^3 117.2 112.7 112.8 115.9, 256^3 455 451 449 452; 24^3 with 1,536 53.4, with 2,048 51.0).
+constexpr int kMgTailCells = 2048;
 struct MgHier {
     int levels = 0;
     MgLevel lv[kMgMaxLevels];

@@ -1223,9 +1223,8 @@ __global__ void __launch_bounds__(kPB) mg_up_kernel(PcgState st, MgLevel F, cons
     mg_up_body(st, F, corr, cny, cnz, blockIdx.x);
 }
 // The V-cycle's tail: its levels from `first` on (mg_tail_level: the smoothed ones hold at most
-// kMgTailCells cells together) in one block, in LDS.  As launches of their own each was 4 us of
-// latency (the coarsest 17), five of them on a 256^3 grid (34 us); one block takes 17 us for all of them.  Each cell's
-// arithmetic is that of the level kernels.
+// kMgTailCells cells together) in one block, in LDS.  Bound by latency: as launches of their own each
+// level is 4 us (the coarsest, swept, was 17).  Each cell's arithmetic is that of the level kernels.
 constexpr int kTailThreads = 1024;
 // cell index -> (i, j, k) in a level of at most kMgTailCells cells, by multiplications (c nz < 2^32)
 struct TailCells {
