@@ -1139,12 +1139,12 @@ FIA_HD int unit_interval_pieces(double a, bool cut, double off, double lo[2], do
 
 // WENO6 psi of the 2 x 2 pieces of the y faces i0 .. i1 - 1 at row = (j, k) of a plane (non-integral
 // rule, both axes cut in two): the four centres lie on psi's sample level j, so each value is a z pass
-// then an x pass over the 6 x 6 samples of that level around it, the same arithmetic as weno3d.  The
-// two centres along an axis are half a cell apart, so their sample bases differ by 0 or 1, and the
-// fractions are those of every face: columns are visited in x order, each gets one z pass per z centre
-// into a 6-column window, shared by the faces around it, and a piece's x pass runs when the window
-// holds its six columns: six evaluations a face (18 for a face on its own).  The first x centre's
-// pieces are complete one column early when the second's base is one further (dx).
+// then an x pass over the 6 x 6 samples of that level around it, the same arithmetic as weno3d.  An
+// axis that is cut is cut at the half, so the two centres along it lie a quarter before and after a
+// sample: the second's base is one further than the first's, and the fractions are those of every face.
+// Columns are visited in x order, each gets one z pass per z centre into a 6-column window, shared by the
+// faces around it, and a piece's x pass runs when the window holds its six columns, the first x
+// centre's pieces one column early: six evaluations a face (18 for a face on its own).
 FIA_HD void zero_velocity_weno(const FaceParams &P, unsigned row, int i0, int i1) {
     const int my1 = P.g.m[1] + 1, mz = P.g.m[2];
     const int j = (int)(row / (unsigned)mz), k = (int)(row - (unsigned)j * (unsigned)mz);
@@ -1161,7 +1161,6 @@ FIA_HD void zero_velocity_weno(const FaceParams &P, unsigned row, int i0, int i1
         split_coord(0.5 * (xl[a] + xh[a]) - opx, bx[a], tx[a]);
         split_coord(0.5 * (zl[a] + zh[a]) - opz, bz[a], tz[a]);
     }
-    const int dx = bx[1] - bx[0], dz = bz[1] - bz[0];   // 0 or 1
     const double x0 = xh[0] - xl[0], x1 = xh[1] - xl[1], z0 = zh[0] - zl[0], z1 = zh[1] - zl[1];
     const WenoCoef wz0(tz[0], P.kappa_psi), wz1(tz[1], P.kappa_psi);
     const WenoCoef wx0(tx[0], P.kappa_psi), wx1(tx[1], P.kappa_psi);
@@ -1171,26 +1170,22 @@ FIA_HD void zero_velocity_weno(const FaceParams &P, unsigned row, int i0, int i1
     double w0[6] = {0, 0, 0, 0, 0, 0}, w1[6] = {0, 0, 0, 0, 0, 0};   // z passes of the last 6 columns
     double first = 0.0;   // the first x centre's pieces of the face in progress
     const size_t plane = (size_t)my1 * mz;
-    const int lead = 5 + dx;   // column c completes face i0 + c - lead
+    constexpr int kLead = 6;   // column c completes face i0 + c - kLead
 #pragma unroll 1
-    for (int c = 0; c < i1 - i0 + lead; ++c) {
+    for (int c = 0; c < i1 - i0 + kLead; ++c) {
         const double *__restrict__ psi = P.psi + (size_t)clampi(bx[0] - 2 + c, 0, P.g.m[0] - 1) * plane;
-        double f[7], g[6];
+        double f[7];
 #pragma unroll
         for (int r = 0; r < 7; ++r) f[r] = psi[at[r]];
 #pragma unroll
-        for (int r = 0; r < 6; ++r) g[r] = dz ? f[r + 1] : f[r];
-#pragma unroll
         for (int r = 0; r < 5; ++r) { w0[r] = w0[r + 1]; w1[r] = w1[r + 1]; }
         w0[5] = weno6<double>(f, wz0);
-        w1[5] = weno6<double>(g, wz1);
-        if (c < 5) continue;
-        const double mine = (x0 * z0) * weno6<double>(w0, wx0) + (x0 * z1) * weno6<double>(w1, wx0);
-        if (dx == 0) first = mine;
-        if (c >= lead)
-            P.flux[1][(size_t)(i0 + c - lead) * plane + row] =
+        w1[5] = weno6<double>(f + 1, wz1);
+        if (c < kLead - 1) continue;
+        if (c >= kLead)
+            P.flux[1][(size_t)(i0 + c - kLead) * plane + row] =
                 first + (x1 * z0) * weno6<double>(w0, wx1) + (x1 * z1) * weno6<double>(w1, wx1);
-        first = mine;
+        first = (x0 * z0) * weno6<double>(w0, wx0) + (x0 * z1) * weno6<double>(w1, wx0);
     }
 }
 

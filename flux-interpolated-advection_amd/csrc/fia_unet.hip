@@ -64,17 +64,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 
 __device__ __forceinline__ long vox(int x, int y, int z, int ny, int nz) { return ((long)x * ny + y) * nz + z; }
 
-// channels [c, c + 4) of a convolution's input at an in-range voxel
-__device__ __forceinline__ bf16x4 load4(const ConvArgs &a, int x, int y, int z, int c) {
-    const uint16_t *p;
-    if (c < a.cA)
-        p = a.upA ? a.srcA + vox(x >> 1, y >> 1, z >> 1, a.ny >> 1, a.nz >> 1) * a.cA + c
-                  : a.srcA + vox(x, y, z, a.ny, a.nz) * a.cA + c;
-    else
-        p = a.srcB + vox(x, y, z, a.ny, a.nz) * a.cB + (c - a.cA);
-    return *reinterpret_cast<const bf16x4 *>(p);
-}
-
 constexpr int kCB = 256;   // threads per convolution block (4 waves x 64 voxels)
 
 // Block tile of the convolution: 4 (x) x M (y) x 16 (z) voxels; wave w owns x-plane w of the tile,
@@ -208,13 +197,15 @@ __global__ void __launch_bounds__(kCB) conv3_kernel(ConvArgs a) {
     }
 }
 
-// One block computes every output channel of its tile while that gives each CU a block; below that
+// One block computes every output channel of its tile while that gives kFill blocks; below that
 // each takes 16 channels, and below that one y-row as well: a level of 8^3 voxels is 4 blocks of
 // 64 channels (60 us, nearly all latency) or 64 of 16 (18 us).  Every output sums the same
-// products in the same order in all forms.
+// products in the same order in all forms.  kFill is a block for each of the 256 CUs (a forward pass with
+// 128, 256, 512 and 1,024: 32^3 208 192 193 191 us, 48^3 294 275 287 287, 64^3 378 345 333 333, 96^3 597
+// 581 597 636, 128^3 1,203 1,153 1,150 1,151).
+constexpr long kFill = 256;
 template <int MODE>
 static hipError_t conv3_nb(const ConvArgs &a, hipStream_t s) {
-    constexpr long kFill = 256;
     const auto tiles = [&](int m) {
         return (long)((a.nx + kTX - 1) / kTX) * ((a.ny + m - 1) / m) * ((a.nz + kTZ - 1) / kTZ);
     };
