@@ -2108,9 +2108,12 @@ int piece_quadrature_mode(const FaceParams &p) {
 constexpr size_t kBrickLeast = 128;
 size_t weno_table_halves(const FaceParams &p, size_t &psi_halves) {
     psi_halves = 0;
-    if (piece_quadrature_mode(p) != 1 || Bricks(p.g).count() < kBrickLeast) return 0;
+    const size_t bricks = Bricks(p.g).count();
+    if (piece_quadrature_mode(p) != 1 || bricks < kBrickLeast) return 0;
     const size_t len = (size_t)p.g.m[2] + kWenoPad;
     const size_t q = (size_t)p.g.m[0] * p.g.m[1] * len, psi = (size_t)p.g.m[0] * (p.g.m[1] + 1) * len;
+    // (boxes of one cell's thickness have more bricks or entries than a launch has threads)
+    if (std::max((bricks + 8) * kBrickThreads, psi + kBlock) >> 32) return 0;
     psi_halves = 2 * psi;
     return 2 * q;
 }
@@ -2131,10 +2134,25 @@ hipError_t launch_weno_tables(const FaceParams &p, WenoHalf *q_tab, WenoHalf *ps
     return hipGetLastError();
 }
 
+// p with the piece arrays from slot `first` on
+static FaceParams slots_from(FaceParams p, unsigned long long first) {
+    for (int a = 0; a < 3; ++a) p.piece_c[a] += first;
+    p.piece_ay += first;
+    p.piece_val += first;
+    return p;
+}
+// piece_kernel over every slot.  A launch counts its threads in 32 bits, and grids from about 800^3 on
+// have more slots than that: launches of at most kLaunchSlots.
+constexpr unsigned long long kLaunchSlots = 1ull << 31;
+template <int QM, bool OPT> static void launch_slots(const FaceParams &p, unsigned long long nslots, hipStream_t s) {
+    const int b = block_or_default(p.piece_block);
+    for (unsigned long long first = 0; first < nslots; first += kLaunchSlots) {
+        const unsigned long long n = std::min(kLaunchSlots, nslots - first);
+        hipLaunchKernelGGL((piece_kernel<QM, OPT>), dim3(grid_for(n, b)), dim3(b), 0, s, slots_from(p, first), n);
+    }
+}
 hipError_t launch_pieces(const FaceParams &p, unsigned long long nslots, hipStream_t s) {
     if (nslots == 0) return hipSuccess;
-    const int b = block_or_default(p.piece_block);
-    const dim3 grid(grid_for(nslots, b));
     const int qm = piece_quadrature_mode(p);
     if (p.q_tab) {
         const Bricks br(p.g);
@@ -2142,17 +2160,17 @@ hipError_t launch_pieces(const FaceParams &p, unsigned long long nslots, hipStre
         if (p.weno_opt) hipLaunchKernelGGL(piece_brick_kernel<true>, bricks, dim3(kBrickThreads), 0, s, p, br);
         else hipLaunchKernelGGL(piece_brick_kernel<false>, bricks, dim3(kBrickThreads), 0, s, p, br);
     } else if (p.weno_opt) {
-        if (qm == 1) hipLaunchKernelGGL((piece_kernel<1, true>), grid, dim3(b), 0, s, p, nslots);
-        else if (qm == 2) hipLaunchKernelGGL((piece_kernel<2, true>), grid, dim3(b), 0, s, p, nslots);
-        else hipLaunchKernelGGL((piece_kernel<0, true>), grid, dim3(b), 0, s, p, nslots);
+        if (qm == 1) launch_slots<1, true>(p, nslots, s);
+        else if (qm == 2) launch_slots<2, true>(p, nslots, s);
+        else launch_slots<0, true>(p, nslots, s);
     } else if (qm == 1) {
-        hipLaunchKernelGGL((piece_kernel<1, false>), grid, dim3(b), 0, s, p, nslots);
+        launch_slots<1, false>(p, nslots, s);
     } else if (qm == 2) {
-        hipLaunchKernelGGL((piece_kernel<2, false>), grid, dim3(b), 0, s, p, nslots);
+        launch_slots<2, false>(p, nslots, s);
     } else if (p.interp == IM_LINEAR) {
-        hipLaunchKernelGGL((piece_kernel<kPieceLinear, false>), grid, dim3(b), 0, s, p, nslots);
+        launch_slots<kPieceLinear, false>(p, nslots, s);
     } else {
-        hipLaunchKernelGGL((piece_kernel<0, false>), grid, dim3(b), 0, s, p, nslots);
+        launch_slots<0, false>(p, nslots, s);
     }
     return hipGetLastError();
 }

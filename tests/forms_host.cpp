@@ -5,7 +5,7 @@
 //   - the zero-velocity march in chunks of x planes, and the other zero-velocity kernels' rules;
 //   - degenerate faces shared over lanes;
 //   - the z stencil tables, and the table quadrature by bricks: rows of slots, box, staging, and the
-//     pieces that read the box or the table;
+//     pieces that read the box or the table; the quadrature of slots in parts (launch_slots);
 //   - twisted faces' pieces in fixed records, and counted where those do not hold them.
 // Not replayed: the scan kernels and the count kernels' sums (a plain scan here), the psi kernels' held
 // columns (psi_body), and what one block's threads exchange through LDS or lane shuffles beyond the
@@ -293,15 +293,20 @@ int faces_forms(FormsCtx &c, const CompGrid &g, const float *q, const double *ps
         if (tables) {
             if (!(p.weno_opt ? bricks_forms<true>(c, p, nslots, st) : bricks_forms<false>(c, p, nslots, st))) return -1;
         } else {
-            parallel_for((long)nslots, [&](long k) {
-                int a = 0, b = 0, e = 0;
-                const unsigned long long slot = (unsigned long long)k;
-                if (qm == 1 && p.weno_opt) piece_body<1, true>(p, slot, a, b, e);
-                else if (qm == 1) piece_body<1>(p, slot, a, b, e);
-                else if (qm == 2 && p.weno_opt) piece_body<2, true>(p, slot, a, b, e);
-                else if (qm == 2) piece_body<2>(p, slot, a, b, e);
-                else if (p.interp == IM_LINEAR) piece_body<kPieceLinear>(p, slot, a, b, e);
-                else piece_body<0>(p, slot, a, b, e);
+            // launch_slots, in parts of a thousand slots
+            constexpr unsigned long long kPart = 1009;
+            parallel_for((long)((nslots + kPart - 1) / kPart), [&](long k) {
+                const unsigned long long first = (unsigned long long)k * kPart, n = std::min(kPart, nslots - first);
+                const FaceParams part = slots_from(p, first);
+                for (unsigned long long slot = 0; slot < n; ++slot) {
+                    int a = 0, b = 0, e = 0;
+                    if (qm == 1 && p.weno_opt) piece_body<1, true>(part, slot, a, b, e);
+                    else if (qm == 1) piece_body<1>(part, slot, a, b, e);
+                    else if (qm == 2 && p.weno_opt) piece_body<2, true>(part, slot, a, b, e);
+                    else if (qm == 2) piece_body<2>(part, slot, a, b, e);
+                    else if (p.interp == IM_LINEAR) piece_body<kPieceLinear>(part, slot, a, b, e);
+                    else piece_body<0>(part, slot, a, b, e);
+                }
             });
         }
     }
@@ -396,6 +401,18 @@ int plain_interp(int interp, Options &o) {
 }  // namespace
 
 extern "C" {
+
+// whether the launcher gives the WENO6 integral pass of an nx x ny x nz cell grid the z stencil tables
+int forms_takes_tables(int nx, int ny, int nz) {
+    FaceParams p;
+    memset(&p, 0, sizeof(p));
+    p.g.init(-1, nx, ny, nz);
+    p.interp = IM_WENO6;
+    p.integral = 1;
+    p.gauss = gauss_table(1);
+    size_t psi_halves = 0;
+    return weno_table_halves(p, psi_halves) > 0;
+}
 
 int forms_cols(void) { return kFormCols; }
 void *forms_create(void) { return new FormsCtx(); }

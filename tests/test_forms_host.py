@@ -122,6 +122,15 @@ def test_zero_velocity_march_fits_a_launch(forms):
             assert 1 <= chunk and -(-nx // chunk) <= 65535
 
 
+def test_tables_fit_a_launch(forms):
+    # a launch counts its threads in 32 bits: 768 a brick of 4 x 8 x 16 cells, and one per table entry
+    takes = forms.L.forms_takes_tables
+    assert takes(256, 256, 256) and takes(36, 40, 40) and takes(900, 900, 900) and takes(18000, 1, 18000)
+    assert not takes(24, 24, 24)            # fewer than 128 bricks
+    assert not takes(19500, 1, 19500)       # 4875 x 1 x 1219 bricks
+    assert not takes(31000, 31000, 1)       # 961 million rows of six entries
+
+
 @pytest.mark.parametrize("comp", [-1, 0, 1, 2])
 @pytest.mark.parametrize("shape", [(9, 15, 15), (8, 16, 14), (4, 14, 16), (1, 2, 3), (23, 33, 18), (70, 3, 40)])
 def test_vertex_tiles_give_each_vertex_its_value(forms, shape, comp):
