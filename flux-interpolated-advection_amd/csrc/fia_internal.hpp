@@ -55,7 +55,6 @@ template <class T> struct DevBuf {
     size_t bytes() const { return n * sizeof(T); }
 };
 
-
 constexpr int kMaxGauss = 49;
 // work counters are kept as kStatSlots triples (pieces, density points, 1D WENO6 evaluations),
 // summed on read

@@ -18,10 +18,11 @@
 //                     rule: the z stencils' interpolants in tables, read from LDS by bricks of faces
 //   piece_kernel      quadrature of every piece slot, any rule (small grids: piece_kernel<1>)
 //   face_sum_kernel   face flux = ordered sum of its slots
-//   general_*         the exact recursive cutter for the few twisted faces: pieces counted and
-//                     stored per face, integrated one thread per piece, summed per face; their
-//                     corrections are marked in a bit mask per family (corr_reset_kernel clears
-//                     them before the flux set's next pass)
+//   general_*         the exact recursive cutter for the few twisted faces: one wave per face and
+//                     orientation, pieces stored in records of a fixed number per face (where those
+//                     would not fit: counted and scanned first), integrated one thread per piece,
+//                     summed per face; their corrections are marked in a bit mask per family
+//                     (corr_reset_kernel clears them before the flux set's next pass)
 //   gather_kernel     per cell: sum of its six signed face fluxes (deterministic, no atomics)
 // Each interior face is computed once; its flux enters the two neighbouring cells with opposite
 // signs, so nothing is lost or created inside the domain.
@@ -244,8 +245,8 @@ FIA_HD bool psi_weno_held(const PsiParams &P) {
     return P.integral && P.mode == 2 && (P.g.m[1] + kPsiSegs - 1) / kPsiSegs <= kPsiHeld &&
            P.gauss.n <= kPsiWenoGauss;
 }
-// bound to 128 VGPRs (three values spilled): two 8-wave blocks per CU instead of one (0.127 ->
-// 0.106 ms per launch on the 256^3 velocity grids)
+// bound to 128 VGPRs (six values spilled): two 8-wave blocks per CU instead of one (0.127 ->
+// 0.106 ms per launch on the 256^3 velocity grids as first bound; 0.086-0.102 now)
 __global__ void __launch_bounds__(64 * kPsiSegs) __attribute__((amdgpu_waves_per_eu(4))) psi_weno_held_kernel(PsiParams P) {
     const int my = P.g.m[1], mz = P.g.m[2];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1280,8 +1281,8 @@ FIA_HD void piece_body(const FaceParams &P, unsigned long long q, int &npieces, 
     }
     P.piece_val[q] = val;
 }
-// QM = 1 serves the grids that take no tables (weno_table_halves), held to three waves per SIMD (no
-// spill).  OPT: the "WENO6-optimized" interpolation (left to the compiler).
+// QM = 1 serves the grids that take no tables (weno_table_halves) or have no room for them, held to
+// three waves per SIMD (168 VGPRs, one value spilled).  OPT: the "WENO6-optimized" interpolation (left to the compiler).
 template <int QM, bool OPT>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(QM == 1 && !OPT ? 3 : 1)))
 piece_kernel(FaceParams P, unsigned long long nslots) {
@@ -1302,11 +1303,13 @@ piece_kernel(FaceParams P, unsigned long long nslots) {
 //      where the flow deforms the brick by more than the box's spare rows, its middle;
 //   3. the pieces, 64 at a time per wave; one whose rows are not all in the box (also a sliver's
 //      far centroid) reads the table in memory.
-// Bound by VALU issue (83% of the cycles at 256^3, CFL 4): 1,566 VALU a wave of pieces, of which the
+// Bound by VALU issue (80% of the cycles at 256^3, CFL 4): 1,570 VALU a wave of pieces, of which the
 // 42 z stencils take 10 and a reciprocal each, where evaluating the stencils from their samples took
-// 3,960; 15.8 -> 8.1 ms per launch (density step 26.1 -> 19.6 ms, with 0.25 ms for the two tables).
-// 768 threads: three waves per SIMD at 168 VGPRs; 512 leave latency (density step 21.1 ms), 1,024
-// spill (20.9).
+// 3,960; 15.9 -> 7.8 ms per launch as traced, and 0.30 ms for the two tables.  It moves 12.7 GB, at a
+// fifth of the copy rate.
+// 768 threads: three waves per SIMD at 168 VGPRs, five values spilled (29 under OPT: 8.6 ms by events
+// against 7.9).  512 leave latency and 1,024 spill more: density steps of 21.1 and 20.9 ms where 768
+// took 19.6.
 constexpr int kBrickX = 4, kBrickY = 8, kBrickZ = 16, kBrickThreads = 768;
 constexpr int kWinX = 12, kWinY = 18, kWinZ = 22;   // 149 KB of the CU's 160
 constexpr int kBrickRows = 3 * (kBrickX + 1) * (kBrickY + 1);

@@ -167,7 +167,7 @@ template <class V> FIA_HD void load_row6(const V *__restrict__ base, unsigned of
 //   delta = t g_2 + t (t - 1) Q(s) / (1 + d_1 s + d_2 s^2),   Q a cubic:
 // the sum of C_r b_r (candidate r) over the sum of C_r b_r, b_r = 1 / e_r^2, both divided by the
 // latter's value at s = 0.  WenoEntry holds the nine numbers (the 1 left out): evaluating it takes
-// 12 instructions where weno6_delta takes 57.  It is worth building where a stencil is evaluated
+// 12 instructions where weno6 takes about 50.  It is worth building where a stencil is evaluated
 // at many fractions: the pieces of a flux pass evaluate each z stencil some 300 times.
 // weno6_entry works in FP64 and rounds the result, so an entry is as close to the exact
 // interpolant as weno6_delta's FP32 weights are.
